@@ -59,6 +59,13 @@ int fail(int code, const std::string &msg) {
 
 int nbatch(int S, int sb) { return (S + sb - 1) / sb; }
 
+int forward_batch(const trace_handle *h) {
+  int sb = h->fwd_sb;
+  if (h->fwd_staged && sb == kStSlices) return sb;  // 64-bit addresses throughout
+  while (sb > 1 && wide_image(h->geo.N, sb)) sb /= 2;
+  return sb;
+}
+
 const char *last_error() { return g_err.c_str(); }
 void clear_error() { g_err.clear(); }
 
@@ -217,13 +224,14 @@ int backproject_ordered(trace_handle *h, int mode, const float *w, float *z, int
 int ensure_work(trace_handle *h, bool images, bool batched_copy) {
   const size_t nn = (size_t)h->geo.NN();
   const size_t S = (size_t)h->geo.S;
-  if (h->xb && h->xb_sb != h->fwd_sb) {
+  const int sb = forward_batch(h);
+  if (h->xb && h->xb_sb != sb) {
     dev_free(h->xb);
     h->xb = nullptr;
   }
   if (!h->xb && batched_copy) {
-    HIP_TRY(dev_alloc(&h->xb, (size_t)nbatch((int)S, h->fwd_sb) * h->fwd_sb * nn));
-    h->xb_sb = h->fwd_sb;
+    HIP_TRY(dev_alloc(&h->xb, (size_t)nbatch((int)S, sb) * sb * nn));
+    h->xb_sb = sb;
   }
   if (!h->w) HIP_TRY(dev_alloc(&h->w, (size_t)h->geo.P * S * h->geo.C + kWeightPad));
   if (!h->maxw) HIP_TRY(dev_alloc(&h->maxw, S));
@@ -308,6 +316,11 @@ bool fwd_shape_supported(int sb, int lanes) {
   return false;
 }
 
+// Lanes per ray at slice batch sb: the handle's, if compiled for it.
+int forward_lanes(const trace_handle *h, int sb) {
+  return fwd_shape_supported(sb, h->fwd_lanes) ? h->fwd_lanes : 1;
+}
+
 bool tile_shape_supported(int tw, int th, int sb) {
 #define TRACE_SHAPE_MATCH(TW_, TH_, SB_) \
   if (tw == TW_ && th == TH_ && sb == SB_) return true;
@@ -329,9 +342,10 @@ int forward(trace_handle *h, int mode, const float *sino, float *out) {
                                                      h->xb, sino, out, h->maxw, h->stream));
     return TRACE_OK;
   }
-  TIMED(TRACE_PHASE_FORWARD, launch_forward(h->geo, h->rays, h->fwd_sb, h->fwd_bundle,
-                                            h->fwd_lanes, mode, h->exact, h->xb, sino, out,
-                                            h->maxw, h->stream));
+  const int sb = forward_batch(h);
+  TIMED(TRACE_PHASE_FORWARD, launch_forward(h->geo, h->rays, sb, h->fwd_bundle,
+                                            forward_lanes(h, sb), mode, h->exact, h->xb, sino,
+                                            out, h->maxw, h->stream));
   return TRACE_OK;
 }
 
@@ -621,7 +635,7 @@ int trace_reconstruct(trace_handle_t *h, trace_alg_t alg, int iters,
   const bool reg = (alg == TRACE_PML || alg == TRACE_APMLR);
   if (int rc = ensure_work(h, reg)) return rc;
   hipStream_t st = h->stream;
-  const int sb = h->fwd_sb;
+  const int sb = forward_batch(h);
   const int nslots = nbatch(S, sb) * sb;
   const int fmode = (alg == TRACE_SIRT) ? kFwdOutSIRT : kFwdOutEM;
 
@@ -721,7 +735,7 @@ int trace_forward(trace_handle_t *h, const float *x, float *y) {
   if (int rc = ensure_rays(h)) return rc;
   if (int rc = ensure_work(h, false)) return rc;
   const Geometry &g = h->geo;
-  const int sb = h->fwd_sb;
+  const int sb = forward_batch(h);
   TIMED(TRACE_PHASE_SETUP,
         launch_pack(x, g.S, 0, 0.f, g.NN(), nbatch(g.S, sb) * sb, sb, h->xb, h->stream));
   return forward(h, kFwdOutY, nullptr, y);
@@ -732,7 +746,7 @@ int trace_forward_noalloc(trace_handle_t *h, const float *x, float *y) {
   if (!h) return fail(TRACE_E_INVALID, "handle is null");
   if (!x || !y) return fail(TRACE_E_INVALID, "null buffer");
   const Geometry &g = h->geo;
-  const int sb = h->fwd_sb;
+  const int sb = forward_batch(h);
   const size_t rays_b = ((size_t)g.rays_per_slice() * sizeof(RayInfo) + 255) & ~size_t(255);
   const size_t xb_b = (size_t)nbatch(g.S, sb) * sb * (size_t)g.NN() * sizeof(float);
   if (rays_b + xb_b > kScratchBytes)
@@ -747,8 +761,8 @@ int trace_forward_noalloc(trace_handle_t *h, const float *x, float *y) {
   // every scratch byte read below is written first on the same stream
   HIP_TRY(launch_ray_info(g, rays, h->stream, false));
   HIP_TRY(launch_pack(x, g.S, 0, 0.f, g.NN(), nbatch(g.S, sb) * sb, sb, xb, h->stream));
-  HIP_TRY(launch_forward(g, rays, sb, h->fwd_bundle, h->fwd_lanes, kFwdOutY, h->exact, xb,
-                         nullptr, y, nullptr, h->stream));
+  HIP_TRY(launch_forward(g, rays, sb, h->fwd_bundle, forward_lanes(h, sb), kFwdOutY, h->exact,
+                         xb, nullptr, y, nullptr, h->stream));
   return TRACE_OK;
 }
 

@@ -153,6 +153,10 @@ namespace trace_hip {
 // Number of batches of sb slices covering S slices.
 int nbatch(int S, int sb);
 
+// Slices per batch of the forward projector: the launch shape's, cut where
+// the whole-ray form could not address the batch (wide_image).
+int forward_batch(const trace_handle *h);
+
 // Ray table and segment statistics (count, longest segment); one
 // synchronous read-back per handle.
 int ensure_rays(trace_handle *h);

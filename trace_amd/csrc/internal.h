@@ -35,6 +35,13 @@ constexpr int kWeightPad = 32;
 // Pixel blocks (of 256 pixels) per work item of the batched image update.
 constexpr int kBatchUpdateBlocks = 16;
 
+// A slice batch of an N x N image of 2^32 bytes or more: past the reach of
+// the buffer resource and 32-bit offsets the forward projector gathers with.
+// One slice has a form for it; deeper batches are cut until they fit.
+__host__ __device__ inline bool wide_image(int N, int sb) {
+  return (uint64_t)N * (uint64_t)N * (uint64_t)sb * 4 >= (uint64_t(1) << 32);
+}
+
 enum Alg { kSIRT = 0, kMLEM = 1, kPML = 2, kAPMLR = 3 };
 enum FwdModeHost { kFwdOutY = 0, kFwdOutSIRT = 1, kFwdOutEM = 2 };
 enum BpModeHost { kBpOutSino = 0, kBpOutOnes = 1, kBpOutCount = 2 };

@@ -112,7 +112,57 @@ __device__ __forceinline__ void store_slices(float *__restrict__ p, const float 
 // each gathers and sums SB/LPR of the batch's slices, so a gather touches
 // LPR-fold fewer distinct cache lines per wavefront instruction (the
 // address unit, not the VALU, limits the one-lane form).
-template <int SB, int MODE, bool kExact, int LPR = 1>
+//
+// A lane walks K segments, issuing their gathers as it goes, and adds the
+// previous K meanwhile, in the walk's order: one segment's gather at a time
+// left a small launch (fewer wavefronts than the GPU holds) waiting for
+// memory at every step (one slice: 256^2 at 180 angles 102 -> 60 us a launch,
+// 2048^2 at 1500 angles, where full occupancy hides most of it, 8.7 -> 8.1 ms;
+// there the L1's line rate is the next bound, one line a clock).
+//
+// Gathers go through a buffer resource over the slice batch: an index past
+// the image (the reference's truncation sends a segment there) is outside
+// the resource's range and reads 0, and a sum that starts at +0 keeps its
+// bits when +0 is added, so no step tests its index.  kWide is the form for
+// images of 2^32 bytes and more, which a resource cannot cover.
+template <int SBL, bool kWide>
+struct ImageGather {
+  const float *base;
+  __amdgpu_buffer_rsrc_t rsrc;
+  unsigned NN;
+  int N, stride;  // stride: floats per pixel
+  __device__ __forceinline__ ImageGather(const float *p, int N_, int stride_, int skip)
+      : base(p + skip), NN((unsigned)N_ * (unsigned)N_), N(N_), stride(stride_) {
+    if constexpr (!kWide)
+      rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(p), 0,
+                                               (int)(NN * (unsigned)(stride_ * 4)), 0x00027000);
+  }
+  __device__ __forceinline__ void load(int ix, int iy, int skip_bytes, float (&o)[SBL]) const {
+    if constexpr (kWide) {
+      const unsigned idx = (unsigned)(ix + iy * N);
+#pragma unroll
+      for (int k = 0; k < SBL; ++k) o[k] = idx < NN ? base[(int64_t)idx * stride + k] : 0.f;
+    } else {
+      // ix, iy lie in [0, N]: the midpoints of points inside the square
+      const unsigned off = (__umul24(iy, N) + (unsigned)ix) * (unsigned)(stride * 4) + skip_bytes;
+      if constexpr (SBL == 1) {
+        o[0] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rsrc, off, 0, 0));
+      } else if constexpr (SBL == 2) {
+        const auto q = __builtin_amdgcn_raw_buffer_load_b64(rsrc, off, 0, 0);
+        o[0] = __uint_as_float(q[0]); o[1] = __uint_as_float(q[1]);
+      } else {
+#pragma unroll
+        for (int k = 0; k < SBL; k += 4) {
+          const auto q = __builtin_amdgcn_raw_buffer_load_b128(rsrc, off + 4 * k, 0, 0);
+#pragma unroll
+          for (int i = 0; i < 4; ++i) o[k + i] = __uint_as_float(q[i]);
+        }
+      }
+    }
+  }
+};
+
+template <int SB, int MODE, bool kExact, int LPR = 1, bool kWide = false>
 __device__ __forceinline__ void forward_bundle(const GridInfo &g, const AngleInfo *__restrict__ ang,
                                                const RayInfo *__restrict__ rays, int P, int S,
                                                int ba_log2, const float *__restrict__ xb,
@@ -124,6 +174,8 @@ __device__ __forceinline__ void forward_bundle(const GridInfo &g, const AngleInf
   static_assert(SB % LPR == 0, "slice batch must split evenly over the lanes of a ray");
   constexpr int SBL = SB / LPR;  // slices per lane
   constexpr int LPR_LOG2 = LPR == 1 ? 0 : (LPR == 2 ? 1 : 2);
+  // segments per set (half of those in flight per lane)
+  constexpr int K = SBL <= 2 ? 4 : (SBL <= 8 ? 2 : 1);
   const int C = g.C;
   const int lane = threadIdx.x & 63;
   const int sub = lane & (LPR - 1);    // slice group of this lane
@@ -133,8 +185,9 @@ __device__ __forceinline__ void forward_bundle(const GridInfo &g, const AngleInf
   const int p = (int)(bundle / nbc) * (1 << ba_log2) + (rl >> bc_log2);
   const int c = (int)(bundle % nbc) * (1 << bc_log2) + (rl & ((1 << bc_log2) - 1));
   const bool valid = (p < P) && (c < C);
-  const unsigned NN = (unsigned)g.N * (unsigned)g.N;
-  const float *xbb = xb + (int64_t)b * NN * SB + sub * SBL;
+  const int64_t NN = (int64_t)g.N * g.N;
+  const ImageGather<SBL, kWide> img(xb + b * NN * SB, g.N, SB, sub * SBL);
+  const int skip = sub * SBL * 4;
   float acc[SBL];
 #pragma unroll
   for (int k = 0; k < SBL; ++k) acc[k] = 0.f;
@@ -143,26 +196,62 @@ __device__ __forceinline__ void forward_bundle(const GridInfo &g, const AngleInf
   const int64_t t = (int64_t)p * C + c;
   if (valid) {
     const RayInfo r = rays[t];
-    traverse_full<kExact>(g, r, ang[p].quadrant, [&](int ix, int iy, float l, float l2) {
-      const unsigned idx = (unsigned)(ix + iy * g.N);
-      const bool in = idx < NN;
-      if constexpr (SBL == 1) {
-        // branch-free: a segment outside the image (skipped) loads pixel 0
-        // and adds +0, which leaves the sum's bits unchanged (a sum that
-        // starts at +0 is never -0 in round-to-nearest)
-        float v[1];
-        load_slices<1>(xbb + (int64_t)(in ? idx : 0u) * SB, v);
-        const float t = v[0] * l;
-        acc[0] += in ? t : 0.f;
-      } else if (in) {
-        float v[SBL];
-        load_slices<SBL>(xbb + (int64_t)idx * SB, v);
+    hit = (r.alo & kRayHits) != 0;
+    Walker w;
+    w.init(r, g.N, ang[p].quadrant);
+    w.seek(0, 0);
+    int rem = w.alen + w.blen - 1;  // segments left
+    if (rem >= 1) {
+      float px, py;
+      w.next(px, py);
+      // two sets of K segments, one walked while the other is added
+      float v[2 * K][SBL], l[2 * K], l2[2 * K];
 #pragma unroll
-        for (int k = 0; k < SBL; ++k) acc[k] += v[k] * l;
+      for (int u = K; u < 2 * K; ++u) {
+        l[u] = l2[u] = 0.f;
+#pragma unroll
+        for (int k = 0; k < SBL; ++k) v[u][k] = 0.f;
       }
-      hit |= in;
-      if (MODE == kFwdSIRT) a2 += l2;
-    });
+      auto step = [&](int u) {
+        float qx, qy;
+        w.next(qx, qy);
+        int ix, iy;
+        segment<kExact>(px, py, qx, qy, g.mg, ix, iy, l[u], l2[u]);
+        px = qx;
+        py = qy;
+        img.load(ix, iy, skip, v[u]);
+      };
+      auto add = [&](int u) {
+#pragma unroll
+        for (int k = 0; k < SBL; ++k) acc[k] += v[u][k] * l[u];
+        if (MODE == kFwdSIRT) a2 += l2[u];
+      };
+      // the scheduling barriers keep each set's sums after the other set's
+      // gathers: moved up, they would wait for loads just issued
+      for (; rem >= 2 * K; rem -= 2 * K) {
+#pragma unroll
+        for (int u = 0; u < K; ++u) step(u);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int u = K; u < 2 * K; ++u) add(u);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int u = K; u < 2 * K; ++u) step(u);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int u = 0; u < K; ++u) add(u);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+#pragma unroll
+      for (int u = K; u < 2 * K; ++u) add(u);
+      // what is left, its gathers again all issued before the first is used
+#pragma unroll
+      for (int u = 0; u < 2 * K - 1; ++u)
+        if (u < rem) step(u);
+#pragma unroll
+      for (int u = 0; u < 2 * K - 1; ++u)
+        if (u < rem) add(u);
+    }
   }
 #pragma unroll
   for (int k = 0; k < SBL; ++k) {
@@ -192,13 +281,13 @@ __device__ __forceinline__ void forward_bundle(const GridInfo &g, const AngleInf
   }
 }
 
-template <int SB, int MODE, bool kExact, int LPR>
+template <int SB, int MODE, bool kExact, int LPR, bool kWide = false>
 __global__ void __launch_bounds__(kRayBlock)
 k_forward(GridInfo g, const AngleInfo *__restrict__ ang, const RayInfo *__restrict__ rays,
           int P, int S, int ba_log2, const float *__restrict__ xb,
           const float *__restrict__ sino, float *__restrict__ out,
           unsigned *__restrict__ maxw) {
-  forward_bundle<SB, MODE, kExact, LPR>(
+  forward_bundle<SB, MODE, kExact, LPR, kWide>(
       g, ang, rays, P, S, ba_log2, xb, sino, out, maxw,
       xcd_chunked(blockIdx.x, gridDim.x) * (kRayBlock / 64) + (threadIdx.x >> 6), blockIdx.y);
 }
@@ -1021,12 +1110,19 @@ k_forward_batch(const BatchSliceDev *__restrict__ d, BatchQueues q, int it, int 
     const BatchSliceDev &sd = d[__builtin_amdgcn_readfirstlane(q.order[0][k])];
     if (it >= sd.iters) continue;
     const int64_t bundle = (int64_t)(item - start[k]) * (kRayBlock / 64) + (threadIdx.x >> 6);
-    if (sd.alg == 0)
-      forward_bundle<1, kFwdSIRT, kExact>(sd.g, sd.ang, sd.rays, sd.P, 1, ba_log2, sd.x,
-                                          sd.sino, sd.w, sd.maxw, bundle, 0);
-    else
-      forward_bundle<1, kFwdEM, kExact>(sd.g, sd.ang, sd.rays, sd.P, 1, ba_log2, sd.x, sd.sino,
-                                        sd.w, sd.maxw, bundle, 0);
+    auto run = [&](auto mode, auto wide) {
+      forward_bundle<1, decltype(mode)::value, kExact, 1, decltype(wide)::value>(
+          sd.g, sd.ang, sd.rays, sd.P, 1, ba_log2, sd.x, sd.sino, sd.w, sd.maxw, bundle, 0);
+    };
+    using std::integral_constant;
+    if (wide_image(sd.g.N, 1)) {
+      if (sd.alg == 0) run(integral_constant<int, kFwdSIRT>(), std::true_type());
+      else run(integral_constant<int, kFwdEM>(), std::true_type());
+    } else if (sd.alg == 0) {
+      run(integral_constant<int, kFwdSIRT>(), std::false_type());
+    } else {
+      run(integral_constant<int, kFwdEM>(), std::false_type());
+    }
   }
 }
 
@@ -1209,7 +1305,7 @@ inline unsigned blocks_for(int64_t n, int b) { return (unsigned)((n + b - 1) / b
 
 // ------------------------------------------------ launch-shape dispatch --
 
-template <int SB, bool E, int LPR>
+template <int SB, bool E, int LPR, bool kWide>
 hipError_t fwd_mode(int mode, const Geometry &g, const RayInfo *rays, int ba_log2,
                     const float *xb, const float *sino, float *out, unsigned *maxw,
                     hipStream_t st) {
@@ -1218,14 +1314,14 @@ hipError_t fwd_mode(int mode, const Geometry &g, const RayInfo *rays, int ba_log
   const int64_t bundles = (int64_t)((g.P + ba - 1) / ba) * ((g.C + bc - 1) / bc);
   dim3 grid(blocks_for(bundles, kRayBlock / 64), (g.S + SB - 1) / SB), block(kRayBlock);
   if (mode == kFwdY)
-    hipLaunchKernelGGL((k_forward<SB, kFwdY, E, LPR>), grid, block, 0, st, g.grid, g.d_ang,
-                       rays, g.P, g.S, ba_log2, xb, sino, out, maxw);
+    hipLaunchKernelGGL((k_forward<SB, kFwdY, E, LPR, kWide>), grid, block, 0, st, g.grid,
+                       g.d_ang, rays, g.P, g.S, ba_log2, xb, sino, out, maxw);
   else if (mode == kFwdSIRT)
-    hipLaunchKernelGGL((k_forward<SB, kFwdSIRT, E, LPR>), grid, block, 0, st, g.grid, g.d_ang,
-                       rays, g.P, g.S, ba_log2, xb, sino, out, maxw);
+    hipLaunchKernelGGL((k_forward<SB, kFwdSIRT, E, LPR, kWide>), grid, block, 0, st, g.grid,
+                       g.d_ang, rays, g.P, g.S, ba_log2, xb, sino, out, maxw);
   else
-    hipLaunchKernelGGL((k_forward<SB, kFwdEM, E, LPR>), grid, block, 0, st, g.grid, g.d_ang,
-                       rays, g.P, g.S, ba_log2, xb, sino, out, maxw);
+    hipLaunchKernelGGL((k_forward<SB, kFwdEM, E, LPR, kWide>), grid, block, 0, st, g.grid,
+                       g.d_ang, rays, g.P, g.S, ba_log2, xb, sino, out, maxw);
   return hipGetLastError();
 }
 
@@ -1233,8 +1329,15 @@ template <int SB, int LPR>
 hipError_t fwd_exact(bool exact, int mode, const Geometry &g, const RayInfo *rays, int ba_log2,
                      const float *xb, const float *sino, float *out, unsigned *maxw,
                      hipStream_t st) {
-  return exact ? fwd_mode<SB, true, LPR>(mode, g, rays, ba_log2, xb, sino, out, maxw, st)
-               : fwd_mode<SB, false, LPR>(mode, g, rays, ba_log2, xb, sino, out, maxw, st);
+  if (wide_image(g.N, SB)) {
+    if constexpr (SB == 1 && LPR == 1)
+      return exact ? fwd_mode<1, true, 1, true>(mode, g, rays, ba_log2, xb, sino, out, maxw, st)
+                   : fwd_mode<1, false, 1, true>(mode, g, rays, ba_log2, xb, sino, out, maxw, st);
+    return hipErrorInvalidValue;
+  }
+  return exact
+             ? fwd_mode<SB, true, LPR, false>(mode, g, rays, ba_log2, xb, sino, out, maxw, st)
+             : fwd_mode<SB, false, LPR, false>(mode, g, rays, ba_log2, xb, sino, out, maxw, st);
 }
 
 constexpr size_t kLdsBytes = 160 * 1024;
