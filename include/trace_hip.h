@@ -104,8 +104,8 @@ typedef struct trace_handle trace_handle_t;
                                   columns x lanes per ray); default 16 at
                                   four lanes per ray, else 8 */
 #define TRACE_OPT_FWD_LANES 5 /* lanes per ray of the forward projector
-                                 (1, 2, 4; default by stack depth: 4 at 32 or
-                                 more slices, 2 at 8-31, else 1): the lanes
+                                 (1, 2, 4; default by stack depth: 4 above
+                                 16 slices, 2 at 5-16, else 1): the lanes
                                  of a ray split its slice batch; compiled for
                                  batches 8, 16 and 32 (2 lanes) and 16, 32
                                  (4 lanes) */
@@ -128,12 +128,15 @@ typedef struct trace_handle trace_handle_t;
                                     segments per ray and pixel; checked once
                                     per geometry), else per pixel; 0 always
                                     per pixel */
-#define TRACE_OPT_FWD_STAGED 8 /* form of the forward projector at 32-slice
-                                  batches (same bits either way): 1 (default)
-                                  bundles of 16 angles x 64 columns sweep the
+#define TRACE_OPT_FWD_STAGED 8 /* form of the forward projector at batches of
+                                  4, 8, 16 and 32 slices (same bits either
+                                  way): 1: bundles of up to 16 angles of
+                                  similar direction x 64 columns sweep the
                                   image in slabs staged in LDS; 0: every ray
                                   reads its pixels from HBM (the form used at
-                                  other slice batches) */
+                                  other slice batches).  Until it is set, the
+                                  faster of the two for the geometry; reads
+                                  as 1 then */
 
 /* Kernel phases reported by trace_phase_times. */
 #define TRACE_PHASE_FORWARD 0 /* forward projection and per-ray weights */

@@ -109,9 +109,11 @@ struct trace_handle {
   int fwd_sb = 16;        // slices per forward lane (xb layout)
   int fwd_bundle = 8;     // adjacent angles per forward wavefront
   int fwd_lanes = 1;      // lanes per ray of the forward projector
-  int fwd_staged = 1;     // TRACE_OPT_FWD_STAGED
+  int fwd_staged = -1;    // TRACE_OPT_FWD_STAGED: 0 or 1 as set, -1 chosen by staged_faster
+  trace_hip::StagedLayout layout;  // angle groups at slice batch layout_sb
+  int layout_sb = 0;
+  bool layout_faster = false;
   trace_hip::StagedPlan staged;  // slab plan of the staged forward projector
-  bool staged_ready = false;
   trace_hip::TileShape tile{16, 16, 16};
   trace_hip::RayInfo *rays = nullptr;     // [P][C]
   bool rays_ready = false;
@@ -155,7 +157,9 @@ int nbatch(int S, int sb);
 
 // Slices per batch of the forward projector: the launch shape's, cut where
 // the whole-ray form could not address the batch (wide_image).
-int forward_batch(const trace_handle *h);
+int forward_batch(trace_handle *h);
+// Whether the forward projector runs its slab-staged form.
+bool forward_staged(trace_handle *h);
 
 // Ray table and segment statistics (count, longest segment); one
 // synchronous read-back per handle.

@@ -1,30 +1,44 @@
-// staged.hip -- forward projector with the image staged in LDS, for
-// 32-slice batches (one 128-byte line of xb per pixel).
+// staged.hip -- forward projector with the image staged in LDS, for slice
+// batches (a pixel's slices contiguous in xb).
 //
 // The whole-ray form (kernels.hip) reads every segment's pixel line from
 // L2; rays share lines only when they happen to meet in time, so each line
 // comes from memory hundreds of times per launch.  Here one workgroup holds
-// a bundle of kStG adjacent angles x kStW adjacent columns (one wavefront
-// per angle, one lane per ray) and walks all of its rays together through
-// the image in thin slabs across the walk direction:
+// a bundle of up to kStG angles x kStW adjacent columns (one wavefront per
+// angle, one lane per ray) and walks all of its rays together through the
+// image in thin slabs across the walk direction:
 //
-//   * shallow rays (|slope| <= 1) sweep slabs of kStH pixel columns left to
+//   * shallow rays (|slope| <= 1) sweep slabs of H pixel columns left to
 //     right (the walk is sorted by x, so the pixel column never decreases);
-//   * steep rays sweep slabs of kStH pixel rows, upwards or downwards with
-//     the sign of the slope.
+//   * steep rays sweep slabs of H pixel rows, upwards or downwards with the
+//     sign of the slope.
 //
-// For each slab the workgroup stages the pixels its rays cross (a window of
-// at most kStEmax pixels across the slab, planned once per geometry from the
-// bundle's outermost rays) in LDS, double-buffered, while the lanes consume
-// the previous slab.  Each lane still walks its own ray from start to end in
-// the reference's order and adds x[idx]*len per slice exactly as the
-// whole-ray form does (sirt.cc:4-19), so y is bit-identical; a segment whose
-// pixel is not in the staged window (outside the plan's margin, a row wrap
-// at ix == N, a window clipped to kStEmax) reads its line from HBM instead.
-// The staging plan therefore affects only speed, never the sums.
+// A bundle's angles come from the projections sorted by direction, never
+// across a change of sweep: a ray swept against its direction would read
+// everything from HBM (one such bundle, at 90 degrees, took 34 ms by itself
+// where the other bundles of a 1024^2, 720-angle launch take 4), and
+// projections need not be given in the order of their angles.
+//
+// For each slab the workgroup stages the pixels its rays cross (a window
+// planned once per geometry from the bundle's outermost rays) in LDS,
+// double-buffered, while the lanes consume the previous slab.  Each lane
+// still walks its own ray from start to end in the reference's order and
+// adds x[idx]*len per slice exactly as the whole-ray form does
+// (sirt.cc:4-19), so y is bit-identical; a segment whose pixel is not in the
+// staged window (outside the plan's margin, a row wrap at ix == N, a window
+// clipped to the buffer) reads its line from HBM instead.  The staging plan
+// therefore affects only speed, never the sums.
+//
+// Bound by vector issue (0.9 of the rate) with the LDS reads close behind: 45
+// instructions of walk and window test a segment, a multiply and an add per
+// slice.  64 slices of 2048^2 at 1500 angles take 49 ms; 64 with the bundles
+// in projection order and the walk before it lost its integer lines, 108 in
+// the whole-ray form.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
+#include <numeric>
 
 #include "staged.h"
 
@@ -34,64 +48,57 @@ namespace trace_hip {
 
 namespace {
 
-constexpr int kSB = kStSlices;
 // Four floats as a native vector: staged values live in registers across
 // the slab loop (an array of the float4 class does not reliably).
 typedef float f4 __attribute__((ext_vector_type(4)));
-constexpr int kBlock = kStG * 64;              // one wavefront per angle
-// A pixel's 128-byte line takes 144 bytes of LDS (nine float4 slots): the
-// lines of neighbouring pixels then start 4 banks apart, so the lanes of a
-// wavefront reading one group of neighbouring pixels hit different banks,
-// and the eight groups of a line sit at fixed offsets from its start.
-constexpr int kPix4 = 9;
-constexpr int kBuf4 = kStH * kStEmax * kPix4;  // float4 slots per slab buffer
-constexpr int kStage4 = (kStH * kStEmax * 8 + kBlock - 1) / kBlock;  // float4 staged per thread
-constexpr size_t kStLds = 2 * (size_t)kBuf4 * sizeof(f4);
+constexpr int kBlock = kStG * 64;  // one wavefront per angle
 static_assert(kStW == 64, "one lane per column of the bundle");
-static_assert(kStH == 4, "the staging order below takes the slab position from 2 bits");
-static_assert(kStLds <= 160 * 1024, "two slab buffers must fit the 160 KB of LDS");
 
-// Slab coordinates of pixel (row, col): u along the sweep, v across it.
-__device__ __forceinline__ void slab_uv(int axis, int N, int row, int col, int &u, int &v) {
-  u = axis == kStAxisX ? col : (axis == kStAxisYUp ? row : N - 1 - row);
-  v = axis == kStAxisX ? row : col;
-}
+// LDS layout and staging order of one slice batch and slab thickness.
+template <int SB, int H>
+struct Slab {
+  static constexpr int kGroups = SB / 4;  // float4 groups of a pixel's slices
+  // A pixel's slices take one float4 slot more than they fill (an odd count):
+  // the lines of neighbouring pixels then start 4 banks apart, so the lanes
+  // of a wavefront reading one group of neighbouring pixels hit different
+  // banks, and the groups of a line sit at fixed offsets from its start.
+  static constexpr int kPix4 = kGroups == 1 ? 1 : kGroups + 1;
+  static constexpr int kE = staged_pixels(SB) / H;  // pixels across a slab
+  static constexpr int kRow4 = kE * kPix4;          // slots of one pixel line along the slab
+  static constexpr int kBuf4 = H * kRow4;           // slots per buffer
+  static constexpr size_t kLds = 2 * (size_t)kBuf4 * sizeof(f4);
+  // Thread t stages group t % kGroups of the pixels (du, dv0 + j * kStep)
+  static constexpr int kStep = kBlock / kGroups / H;
+  static constexpr int kStage = (kE + kStep - 1) / kStep;  // float4 staged per thread
+  static_assert(kBlock % (kGroups * H) == 0, "whole pixels per staging pass");
+  static_assert(kLds <= 160 * 1024, "two slab buffers must fit the 160 KB of LDS");
+};
 
-// Plan of one bundle: its sweep axis, and per slab the first pixel and the
-// extent of the window across the slab (extent 0: nothing to stage).  One
-// block per bundle; the window of slab k holds the pixels, with one pixel
-// of margin, that the lines of the bundle's outermost rays (first and last
-// column of every angle: at a fixed position along the sweep the rays of an
-// angle are parallel lines ordered by column) cross within the slab.
+// Plan of one bundle: per slab the first pixel and the extent of the window
+// across the slab (extent 0: nothing to stage).  One block per bundle; the
+// window of slab k holds the pixels, with one pixel of margin, that the
+// lines of the bundle's outermost rays (first and last column of every
+// angle: at a fixed position along the sweep the rays of an angle are
+// parallel lines ordered by column) cross within the slab.
 __global__ void __launch_bounds__(256)
-k_staged_plan(GridInfo g, const RayInfo *__restrict__ rays, int P, int nslab, int ngc,
-              int *__restrict__ axis_out, int2 *__restrict__ range) {
+k_staged_plan(GridInfo g, const RayInfo *__restrict__ rays, const int *__restrict__ order,
+              const int4 *__restrict__ group, int H, int emax, int nslab, int ngc,
+              int2 *__restrict__ range) {
   const int wg = blockIdx.x;
-  const int ag = wg / ngc, cb = wg % ngc;
-  const int p0 = ag * kStG, c0 = cb * kStW;
-  const int pn = min(kStG, P - p0), cn = min(kStW, g.C - c0);
-  const int N = g.N;
-  const RayInfo &mid = rays[(int64_t)(p0 + pn / 2) * g.C + c0 + cn / 2];
-  const int axis = __builtin_fabsf(mid.slope) <= 1.0f
-                       ? kStAxisX
-                       : (mid.slope > 0.0f ? kStAxisYUp : kStAxisYDown);
-  if (threadIdx.x == 0) axis_out[wg] = axis;
+  const int4 ga = group[wg / ngc];
+  const int c0 = (wg % ngc) * kStW;
+  const int cn = min(kStW, g.C - c0);
+  const int N = g.N, axis = ga.z;
   const double mg = 0.5 * N;
   for (int k = threadIdx.x; k < nslab; k += blockDim.x) {
     // grid-coordinate interval of the slab along the sweep, half a pixel of
     // margin on either side
-    double ua, ub;
-    if (axis == kStAxisYDown) {
-      ua = (double)(N - k * kStH - kStH) - mg - 0.5;
-      ub = (double)(N - k * kStH) - mg + 0.5;
-    } else {
-      ua = (double)(k * kStH) - mg - 0.5;
-      ub = (double)(k * kStH + kStH) - mg + 0.5;
-    }
+    const int u0 = (axis == kStAxisYDown ? nslab - 1 - k : k) * H;
+    const double ua = (double)u0 - mg - 0.5, ub = (double)(u0 + H) - mg + 0.5;
     double lo = 1e30, hi = -1e30;
     bool any = false, wide = false;
-    for (int e = 0; e < 2 * pn; ++e) {
-      const int p = p0 + (e >> 1);
+    for (int e = 0; e < 2 * ga.y; ++e) {
+      const int p = order[ga.x + (e >> 1)];
       const int c = (e & 1) ? c0 + cn - 1 : c0;
       const RayInfo r = rays[(int64_t)p * g.C + c];
       double va, vb;
@@ -120,187 +127,176 @@ k_staged_plan(GridInfo g, const RayInfo *__restrict__ rays, int P, int nslab, in
       last = (int)fmin(fh, (double)(N - 1));
     }
     int extent = last >= first ? last - first + 1 : 0;
-    if (extent > kStEmax) {  // keep the middle of the window
-      first += (extent - kStEmax) / 2;
-      extent = kStEmax;
+    if (extent > emax) {  // keep the middle of the window
+      first += (extent - emax) / 2;
+      extent = emax;
     }
     range[(int64_t)wg * nslab + k] = make_int2(first, extent);
   }
 }
 
 // The walk of one lane, one segment ahead: the pending segment is computed
-// but not yet added (idx, len, len2; u, v its slab coordinates; key its
-// slab, -1 for a pixel outside the image, taken at once and adding nothing,
-// and kStDone once the walk is over).
-constexpr int kStDone = 1 << 30;
+// but not yet added.
+constexpr int kStDone = 1 << 30;  // u of a finished walk, past every slab
+template <int AXIS>
 struct StagedWalk {
   Walker w;
   float px, py;
-  int rem;
-  unsigned idx;
   float len, len2;
-  int key, u, v;
+  int u, v;  // pixel along and across the sweep (a row for u downwards)
+
+  template <bool kExact>
+  __device__ __forceinline__ void advance(const GridInfo &g) {
+    float qx, qy;
+    uint64_t none;
+    w.next(qx, qy, none);
+    int ix, iy;
+    segment<kExact>(px, py, qx, qy, g.mg, ix, iy, len, len2);
+    px = qx;
+    py = qy;
+    u = AXIS == kStAxisX ? ix : iy;
+    v = AXIS == kStAxisX ? iy : ix;
+    u = __builtin_amdgcn_inverse_ballot_w64(none) ? (AXIS == kStAxisYDown ? -kStDone : kStDone) : u;
+  }
 };
 
-template <bool kExact, int AXIS>
-__device__ __forceinline__ void staged_advance(StagedWalk &r, const GridInfo &g, unsigned NN) {
-  if (r.rem <= 0) {
-    r.key = kStDone;
-    return;
-  }
-  const int N = g.N;
-  float qx, qy;
-  r.w.next(qx, qy);
-  int ix, iy;
-  segment<kExact>(r.px, r.py, qx, qy, g.mg, ix, iy, r.len, r.len2);
-  r.px = qx;
-  r.py = qy;
-  --r.rem;
-  r.idx = (unsigned)(ix + iy * N);
-  const bool in = r.idx < NN;
-  int row = iy, col = ix;
-  if ((unsigned)ix >= (unsigned)N) {  // a wrap onto the next row
-    row = (int)(r.idx / (unsigned)N);
-    col = (int)(r.idx - (unsigned)row * (unsigned)N);
-  }
-  slab_uv(AXIS, N, row, col, r.u, r.v);
-  r.key = in ? (int)((unsigned)r.u / kStH) : -1;
-}
-
-// Global offset (in floats) of staged float4 f of slab k, or -1 if it holds
-// no pixel.  Float4 f is group f & 7 of pixel f >> 3; pixels in the order
-// (v, u) with u fastest.
-__device__ __forceinline__ int64_t stage_src(int f, int k, int lo, int E, int N, int axis) {
-  const int qg = f >> 3, du = qg & (kStH - 1), dv = qg >> 2;
-  const int u = k * kStH + du;
-  if (f >= kStH * E * 8 || u >= N) return -1;
-  const int v = lo + dv;
-  const int row = axis == kStAxisX ? v : (axis == kStAxisYUp ? u : N - 1 - u);
-  const int col = axis == kStAxisX ? u : v;
-  return ((int64_t)row * N + col) * kSB + 4 * (f & 7);
-}
-
-// LDS slot (in float4) of staged float4 f: pixel (du, dv) at q = du * E + dv.
-__device__ __forceinline__ int stage_dst(int f, int E) {
-  const int qg = f >> 3, du = qg & (kStH - 1), dv = qg >> 2;
-  return (du * E + dv) * kPix4 + (f & 7);
-}
-
-template <int MODE, bool kExact, int AXIS>
+template <int SB, int H, int MODE, bool kExact, int AXIS>
 __device__ __forceinline__ void forward_staged(
-    f4 *slab, int wg, int b, const GridInfo &g, const AngleInfo *__restrict__ ang,
-    const RayInfo *__restrict__ rays, int P, int S, int nslab, int ngc,
-    const int2 *__restrict__ range, const float *__restrict__ xb,
-    const float *__restrict__ sino, float *__restrict__ out, unsigned *__restrict__ maxw) {
-  constexpr int axis = AXIS;
-  const int ag = wg / ngc, cb = wg % ngc;
+    f4 *slab, const int4 &ga, const int *__restrict__ order, int cb, int b, const GridInfo &g,
+    const AngleInfo *__restrict__ ang, const RayInfo *__restrict__ rays, int S, int nslab,
+    const int2 *__restrict__ rng, const float *__restrict__ xb, const float *__restrict__ sino,
+    float *__restrict__ out, unsigned *__restrict__ maxw) {
+  using L = Slab<SB, H>;
   const int lane = threadIdx.x & 63;
-  const int p = ag * kStG + (threadIdx.x >> 6), c = cb * kStW + lane;
+  const int slot = threadIdx.x >> 6;
+  const int p = order[ga.x + min(slot, ga.y - 1)], c = cb * kStW + lane;
   const int C = g.C, N = g.N;
-  const bool valid = p < P && c < C;
+  const bool valid = slot < ga.y && c < C;
   const unsigned NN = (unsigned)N * (unsigned)N;
-  const float *xbb = xb + (int64_t)b * NN * kSB;
-  const int2 *rng = range + (int64_t)wg * nslab;
+  const float *xbb = xb + (int64_t)b * NN * SB;
 
-  float acc[kSB];
+  float acc[SB];
 #pragma unroll
-  for (int s = 0; s < kSB; ++s) acc[s] = 0.f;
+  for (int s = 0; s < SB; ++s) acc[s] = 0.f;
   float a2 = 0.f;
   bool hit = false;  // the ray has a segment in the image
 
-  StagedWalk r;
-  r.px = r.py = 0.f;
-  r.rem = 0;
-  r.idx = 0;
+  StagedWalk<AXIS> r;
+  r.u = AXIS == kStAxisYDown ? -kStDone : kStDone;
+  r.v = 0;
   r.len = r.len2 = 0.f;
-  r.key = kStDone;
-  r.u = r.v = 0;
   const int64_t t = (int64_t)p * C + c;
   if (valid) {
-    r.w.init(rays[t], N, ang[p].quadrant);
+    const RayInfo ri = rays[t];
+    hit = (ri.alo & kRayHits) != 0;
+    r.w.init(ri, N, ang[p].quadrant);
     r.w.seek(0, 0);
-    const int n = r.w.alen + r.w.blen;
-    if (n >= 2) {
+    if (r.w.alen + r.w.blen >= 2) {
       r.w.next(r.px, r.py);
-      r.rem = n - 1;
-      staged_advance<kExact, AXIS>(r, g, NN);
+      r.template advance<kExact>(g);
     }
   }
 
-  f4 stg[kStage4];
+  // this thread's share of a slab: offsets of its pixels in xb from the
+  // slab window's first one, and in a buffer
+  const int sg = threadIdx.x % L::kGroups, sq = threadIdx.x / L::kGroups;
+  const int du = sq % H, dv0 = sq / H;
+  const unsigned vstep = (unsigned)(L::kStep * SB * 4) * (AXIS == kStAxisX ? (unsigned)N : 1u);
+  const unsigned voff = ((unsigned)(AXIS == kStAxisX ? dv0 : du) * (unsigned)N +
+                         (unsigned)(AXIS == kStAxisX ? du : dv0)) * (unsigned)(SB * 4) + 16u * sg;
+  const int doff = du * L::kRow4 + dv0 * L::kPix4 + sg;
+  f4 stg[L::kStage];
+  auto slab_u = [&](int k) { return (AXIS == kStAxisYDown ? nslab - 1 - k : k) * H; };
+  auto window = [&](int k, int lo) {  // first pixel of the slab's window in xb
+    const int64_t u = slab_u(k);
+    return reinterpret_cast<const char *>(
+        xbb + (AXIS == kStAxisX ? (int64_t)lo * N + u : u * N + lo) * SB);
+  };
   int2 cur = rng[0];
+  {
+    const char *src = window(0, cur.x);
+    const int live = slab_u(0) + du < N ? cur.y : 0;
 #pragma unroll
-  for (int j = 0; j < kStage4; ++j) {
-    const int f = threadIdx.x + j * kBlock;
-    const int64_t o = stage_src(f, 0, cur.x, cur.y, N, axis);
-    if (o >= 0) slab[stage_dst(f, cur.y)] = *reinterpret_cast<const f4 *>(xbb + o);
+    for (int j = 0; j < L::kStage; ++j)
+      if (dv0 + j * L::kStep < live)
+        slab[doff + j * (L::kStep * L::kPix4)] =
+            *reinterpret_cast<const f4 *>(src + (voff + j * vstep));
   }
   __syncthreads();
   // Slab k: stage slab k + 1 into the other buffer while the lanes add their
   // segments up to slab k (and those of earlier slabs, from HBM: they were
-  // not staged).  The pass k == nslab, past the last slab (every segment in
-  // the image has a slab below nslab), adds what is left, from HBM (nothing
-  // for a ray inside the grid).
+  // not staged).  The pass k == nslab, past the last slab, adds what is left,
+  // from HBM (nothing for a ray inside the grid).
   for (int k = 0; k <= nslab; ++k) {
     const bool more = k + 1 < nslab;
     const int2 nxt = more ? rng[k + 1] : make_int2(0, 0);
-    int64_t so[kStage4];
+    const int live = more && slab_u(k + 1) + du < N ? nxt.y : 0;
+    if (more) {
+      const char *src = window(k + 1, nxt.x);
 #pragma unroll
-    for (int j = 0; j < kStage4; ++j) {
-      so[j] = more ? stage_src(threadIdx.x + j * kBlock, k + 1, nxt.x, nxt.y, N, axis) : -1;
-      if (so[j] >= 0) stg[j] = *reinterpret_cast<const f4 *>(xbb + so[j]);
+      for (int j = 0; j < L::kStage; ++j)
+        if (dv0 + j * L::kStep < live)
+          stg[j] = *reinterpret_cast<const f4 *>(src + (voff + j * vstep));
     }
-    const int kk = k;
-    const int lo = cur.x, E = k < nslab ? cur.y : 0;
-    const int base = (k & 1) * kBuf4;
-    while (r.key <= kk) {
-      if (r.key >= 0) {
-        const int dv = r.v - lo;
-        const bool staged = r.key == kk && (unsigned)dv < (unsigned)E;
-        const int q = (r.u - kk * kStH) * E + dv;
-        const int lq = base + q * kPix4;
-        if (staged) {
-          // two halves of the line, so that at most 16 loaded values are live
+    const bool last = k == nslab;
+    // pixels [u0, u1) along the sweep are staged; those the walk has passed
+    // or reached are taken (downwards: from u0 on; else: below u1)
+    const int u0 = last ? (AXIS == kStAxisYDown ? -1 : N) : slab_u(k);
+    const int u1 = last ? (AXIS == kStAxisYDown ? 0 : kStDone) : min(u0 + H, N);
+    const int lo = cur.x;
+    const unsigned E = last ? 0u : (unsigned)cur.y;
+    // byte offset of staged pixel (u, dv) is u * row + dv * pix + base
+    const int base = ((k & 1) * L::kBuf4 - u0 * L::kRow4) * 16;
+    while (AXIS == kStAxisYDown ? r.u >= u0 : r.u < u1) {
+      const unsigned dv = (unsigned)(r.v - lo);
+      const bool in_slab = AXIS == kStAxisYDown ? r.u < u1 : r.u >= u0;
+      if (in_slab && dv < E) {
+        const unsigned lq = __umul24((unsigned)r.u, L::kRow4 * 16) +
+                            (__umul24(dv, L::kPix4 * 16) + (unsigned)base);
+        const f4 *src = reinterpret_cast<const f4 *>(reinterpret_cast<const char *>(slab) + lq);
+        // a quarter to half of the line at a time, so that at most 16 loaded
+        // values are live
 #pragma unroll
-          for (int hlf = 0; hlf < 2; ++hlf) {
-            f4 f[4];
+        for (int h = 0; h < L::kGroups; h += 4) {
+          f4 f[4];
 #pragma unroll
-            for (int j = 0; j < 4; ++j) f[j] = slab[lq + 4 * hlf + j];
+          for (int j = 0; j < 4 && j < L::kGroups; ++j) f[j] = src[h + j];
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-              float *a = acc + 16 * hlf + 4 * j;
-              a[0] += f[j].x * r.len; a[1] += f[j].y * r.len;
-              a[2] += f[j].z * r.len; a[3] += f[j].w * r.len;
-            }
+          for (int j = 0; j < 4 && j < L::kGroups; ++j) {
+            float *a = acc + 4 * (h + j);
+            a[0] += f[j].x * r.len; a[1] += f[j].y * r.len;
+            a[2] += f[j].z * r.len; a[3] += f[j].w * r.len;
           }
-        } else {
+        }
+      } else {
+        const unsigned idx = AXIS == kStAxisX ? (unsigned)(r.u + r.v * N) : (unsigned)(r.v + r.u * N);
+        if (idx < NN) {
           // from HBM; the explicit wait keeps the merge point free of
           // waits, which would otherwise also wait for the staging loads
-          const f4 *gsrc = reinterpret_cast<const f4 *>(xbb + (int64_t)r.idx * kSB);
+          const f4 *gsrc = reinterpret_cast<const f4 *>(xbb + (int64_t)idx * SB);
 #pragma unroll
-          for (int hlf = 0; hlf < 2; ++hlf) {
+          for (int h = 0; h < L::kGroups; h += 4) {
             f4 f[4];
 #pragma unroll
-            for (int j = 0; j < 4; ++j) f[j] = gsrc[4 * hlf + j];
+            for (int j = 0; j < 4 && j < L::kGroups; ++j) f[j] = gsrc[h + j];
             wait_vector_loads();
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-              float *a = acc + 16 * hlf + 4 * j;
+            for (int j = 0; j < 4 && j < L::kGroups; ++j) {
+              float *a = acc + 4 * (h + j);
               a[0] += f[j].x * r.len; a[1] += f[j].y * r.len;
               a[2] += f[j].z * r.len; a[3] += f[j].w * r.len;
             }
           }
         }
       }
-      hit |= r.key >= 0;
       if (MODE == kFwdOutSIRT) a2 += r.len2;
-      staged_advance<kExact, AXIS>(r, g, NN);
+      r.template advance<kExact>(g);
     }
     if (more) {
-      const int nbase = ((k + 1) & 1) * kBuf4;
+      f4 *dst = slab + doff + ((k + 1) & 1) * L::kBuf4;
 #pragma unroll
-      for (int j = 0; j < kStage4; ++j)
-        if (so[j] >= 0) slab[nbase + stage_dst(threadIdx.x + j * kBlock, nxt.y)] = stg[j];
+      for (int j = 0; j < L::kStage; ++j)
+        if (dv0 + j * L::kStep < live) dst[j * (L::kStep * L::kPix4)] = stg[j];
     }
     // every staging load has been waited for by its store; saying so here
     // keeps the compiler from waiting again before the next slab's loads
@@ -310,8 +306,8 @@ __device__ __forceinline__ void forward_staged(
   }
 
 #pragma unroll
-  for (int k = 0; k < kSB; ++k) {
-    const int s = b * kSB + k;
+  for (int k = 0; k < SB; ++k) {
+    const int s = b * SB + k;
     const bool live = valid && (s < S);
     unsigned m = 0;
     if (live) {
@@ -334,71 +330,188 @@ __device__ __forceinline__ void forward_staged(
   }
 }
 
-template <int MODE, bool kExact>
+template <int SB, int H, int MODE, bool kExact>
 __global__ void __launch_bounds__(kBlock)
 k_forward_staged(GridInfo g, const AngleInfo *__restrict__ ang,
-                 const RayInfo *__restrict__ rays, int P, int S, int nslab, int ngc,
-                 const int *__restrict__ axis_of, const int2 *__restrict__ range,
-                 const float *__restrict__ xb, const float *__restrict__ sino,
-                 float *__restrict__ out, unsigned *__restrict__ maxw) {
-  extern __shared__ f4 slab[];  // [2][kBuf4]
+                 const RayInfo *__restrict__ rays, int S, int nslab, int ngc,
+                 const int *__restrict__ order, const int4 *__restrict__ group,
+                 const int2 *__restrict__ range, const float *__restrict__ xb,
+                 const float *__restrict__ sino, float *__restrict__ out,
+                 unsigned *__restrict__ maxw) {
+  extern __shared__ f4 slab[];  // [2][Slab::kBuf4]
   const int wg = (int)xcd_chunked(blockIdx.x, gridDim.x);
   const int b = blockIdx.y;
-  const int axis = axis_of[wg];  // uniform: one specialised body per sweep axis
-  if (axis == kStAxisX)
-    forward_staged<MODE, kExact, kStAxisX>(slab, wg, b, g, ang, rays, P, S, nslab, ngc, range,
-                                           xb, sino, out, maxw);
-  else if (axis == kStAxisYUp)
-    forward_staged<MODE, kExact, kStAxisYUp>(slab, wg, b, g, ang, rays, P, S, nslab, ngc,
-                                             range, xb, sino, out, maxw);
+  const int4 ga = group[wg / ngc];
+  const int cb = wg % ngc;
+  const int2 *rng = range + (int64_t)wg * nslab;
+  // uniform: one specialised body per sweep axis
+  if (ga.z == kStAxisX)
+    forward_staged<SB, H, MODE, kExact, kStAxisX>(slab, ga, order, cb, b, g, ang, rays, S, nslab,
+                                                  rng, xb, sino, out, maxw);
+  else if (ga.z == kStAxisYUp)
+    forward_staged<SB, H, MODE, kExact, kStAxisYUp>(slab, ga, order, cb, b, g, ang, rays, S,
+                                                    nslab, rng, xb, sino, out, maxw);
   else
-    forward_staged<MODE, kExact, kStAxisYDown>(slab, wg, b, g, ang, rays, P, S, nslab, ngc,
-                                               range, xb, sino, out, maxw);
+    forward_staged<SB, H, MODE, kExact, kStAxisYDown>(slab, ga, order, cb, b, g, ang, rays, S,
+                                                      nslab, rng, xb, sino, out, maxw);
 }
 
-template <int MODE, bool E>
+template <int SB, int H, int MODE, bool E>
 hipError_t staged_launch(const Geometry &g, const RayInfo *rays, const StagedPlan &pl,
                          const float *xb, const float *sino, float *out, unsigned *maxw,
                          hipStream_t st) {
-  auto kern = k_forward_staged<MODE, E>;
+  auto kern = k_forward_staged<SB, H, MODE, E>;
+  constexpr size_t lds = Slab<SB, H>::kLds;
   hipError_t e = hipFuncSetAttribute((const void *)kern,
-                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)kStLds);
+                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
   if (e != hipSuccess) return e;
-  const int64_t nwg = (int64_t)pl.ngc * ((g.P + kStG - 1) / kStG);
-  dim3 grid((unsigned)nwg, (g.S + kSB - 1) / kSB), block(kBlock);
-  hipLaunchKernelGGL(kern, grid, block, kStLds, st, g.grid, g.d_ang, rays, g.P, g.S, pl.nslab,
-                     pl.ngc, pl.axis, pl.range, xb, sino, out, maxw);
+  dim3 grid((unsigned)(pl.ngc * pl.ngroups), (g.S + SB - 1) / SB), block(kBlock);
+  hipLaunchKernelGGL(kern, grid, block, lds, st, g.grid, g.d_ang, rays, g.S, pl.nslab, pl.ngc,
+                     pl.order, pl.group, pl.range, xb, sino, out, maxw);
   return hipGetLastError();
+}
+
+template <int SB, int H>
+hipError_t staged_mode(const Geometry &g, const RayInfo *rays, const StagedPlan &pl, int mode,
+                       bool exact, const float *xb, const float *sino, float *out,
+                       unsigned *maxw, hipStream_t st) {
+  if (mode == kFwdOutY)
+    return exact ? staged_launch<SB, H, kFwdOutY, true>(g, rays, pl, xb, sino, out, maxw, st)
+                 : staged_launch<SB, H, kFwdOutY, false>(g, rays, pl, xb, sino, out, maxw, st);
+  if (mode == kFwdOutSIRT)
+    return exact ? staged_launch<SB, H, kFwdOutSIRT, true>(g, rays, pl, xb, sino, out, maxw, st)
+                 : staged_launch<SB, H, kFwdOutSIRT, false>(g, rays, pl, xb, sino, out, maxw, st);
+  return exact ? staged_launch<SB, H, kFwdOutEM, true>(g, rays, pl, xb, sino, out, maxw, st)
+               : staged_launch<SB, H, kFwdOutEM, false>(g, rays, pl, xb, sino, out, maxw, st);
 }
 
 }  // namespace
 
-void staged_plan_size(const Geometry &g, int &nwg, int &nslab, int &ngc) {
-  ngc = (g.C + kStW - 1) / kStW;
-  nwg = ngc * ((g.P + kStG - 1) / kStG);
-  nslab = (g.N + kStH - 1) / kStH;
+StagedLayout staged_layout(const Geometry &g, const AngleInfo *ang, int sb) {
+  // Directions from -45 degrees on: shallow, upwards and downwards rays in
+  // turn, then the same again pointing the other way (whose columns lie in
+  // reverse on the image), each by angle.
+  struct Dir {
+    double a, t, width;  // direction, its tangent against the sweep, pixels of a column block
+    int axis;
+    bool reverse;
+  };
+  std::vector<Dir> dir(g.P);
+  for (int p = 0; p < g.P; ++p) {
+    const double s = ang[p].sinq, c = ang[p].cosq;
+    Dir &d = dir[p];
+    d.axis = std::fabs(s) <= std::fabs(c) ? kStAxisX : (s * c > 0 ? kStAxisYUp : kStAxisYDown);
+    d.t = d.axis == kStAxisX ? s / c : c / s;
+    d.width = kStW / std::max(std::fabs(s), std::fabs(c));
+    d.reverse = (d.axis == kStAxisX ? c : s) < 0;
+    d.a = std::atan2(s, c) + (std::atan2(s, c) < -M_PI / 4 ? 2 * M_PI : 0.0);
+  }
+  StagedLayout best;
+  std::vector<int> order(g.P);
+  std::iota(order.begin(), order.end(), 0);
+  std::stable_sort(order.begin(), order.end(),
+                   [&](int i, int j) { return dir[i].a < dir[j].a; });
+  best.order = order;
+  double best_cost = 0;
+  // A group takes angles while its window stays within the buffer's at the
+  // image's edge; where the bundles fill the GPU at least twice over, within
+  // a quarter more (clipped there, where few rays are: a clipped slab waits
+  // for HBM, which other bundles then hide.  One 32-slice batch, limits 1.25
+  // and 1: 24.5 and 26.2 ms at 2048^2 / 1500 angles, 0.83 and 0.69 ms at
+  // 512^2 / 360).
+  const int64_t bundles =
+      (int64_t)((g.P + kStG - 1) / kStG) * ((g.C + kStW - 1) / kStW) * ((g.S + sb - 1) / sb);
+  const double over = bundles >= 512 ? 1.25 : 1.0;
+  for (int H : {4, 2, 1}) {
+    if (H == 1 && sb != 32) continue;
+    const double limit = over * staged_pixels(sb) / H;
+    std::vector<int4> group;
+    double cost = 0;
+    for (int i = 0; i < g.P;) {
+      const Dir &d0 = dir[order[i]];
+      int n = 1;
+      while (i + n < g.P && n < kStG) {
+        const Dir &d = dir[order[i + n]];
+        if (d.axis != d0.axis || d.reverse != d0.reverse) break;
+        const double e = std::max(d0.width, d.width) + 0.5 * g.N * std::fabs(d.t - d0.t) + 4.0;
+        if (e > limit) break;
+        ++n;
+      }
+      group.push_back(make_int4(i, n, d0.axis, 0));
+      cost += std::max(n, kStG / 2) * 1.4 * (45.0 + 2 * sb) + kStG * 60.0 / H;
+      i += n;
+    }
+    if (best.H == 0 || cost < best_cost) {
+      best.H = H;
+      best.group = group;
+      best_cost = cost;
+    }
+  }
+  // Each XCD runs a contiguous eighth of the workgroups (xcd_chunked).  A
+  // diagonal bundle takes up to 2.8 times as long as one along an axis, so
+  // the groups are dealt to the eighths in turn, longest first.
+  auto length = [&](const int4 &ga) {
+    const Dir &d = dir[order[ga.x + ga.y / 2]];
+    return d.width * ga.y;
+  };
+  std::stable_sort(best.group.begin(), best.group.end(),
+                   [&](const int4 &i, const int4 &j) { return length(i) > length(j); });
+  std::vector<int4> dealt;
+  for (size_t x = 0; x < 8; ++x)
+    for (size_t i = x; i < best.group.size(); i += 8) dealt.push_back(best.group[i]);
+  best.group = dealt;
+  return best;
+}
+
+// Estimated times of one projection by the two forms, from launches of one
+// batch on uniform angles (us; sb 4 / 8 / 16 / 32, staged against whole):
+//   2048^2, 1500 angles   9011 / 10127 / 17371 / 24494   12422 / 19763 / 33321 / 50221
+//   1024^2,  720          1370 /  1518 /  2426 /  3532    1694 /  2347 /  3935 /  5558
+//   1024^2,  180           702 /   721 /   921 /  1523     785 /   860 /  1354 /  2275
+//    640^2,  480           606 /   682 /   893 /  1231     439 /   639 /  1072 /  1402
+//    512^2,  360           364 /   409 /   512 /   687     266 /   345 /   575 /   688
+//    300^2,  181           204 /   228 /   288 /   342      80 /    88 /   123 /   160
+// A staged launch takes a sweep per bundle in flight (bundles fill the 256
+// CUs in rounds; one alone waits for its slabs), a whole-ray launch its
+// segments' gathers and the longest ray's latency.
+bool staged_faster(const Geometry &g, const StagedLayout &lay, int sb) {
+  const int i = sb == 4 ? 0 : (sb == 8 ? 1 : (sb == 16 ? 2 : 3));
+  static const double sweep[] = {0.51, 0.64, 0.75, 0.98};   // us per pixel of the sweep
+  static const double round[] = {0.33, 0.37, 0.63, 0.90};   // and per round of bundles
+  static const double gather[] = {1.9, 2.6, 5.5, 8.0};      // 1e-6 us per segment
+  const int nb = (g.S + sb - 1) / sb;
+  const double bundles = (double)lay.group.size() * ((g.C + kStW - 1) / kStW) * nb;
+  const double staged = g.N * (sweep[i] + round[i] * bundles / 256);
+  const double segments = 1.2 * g.N * std::min(g.N, g.C) * (double)g.P;
+  const double whole = nb * segments * gather[i] * 1e-6 + 0.1 * g.N;
+  return staged < whole;
 }
 
 hipError_t launch_staged_plan(const Geometry &g, const RayInfo *rays, StagedPlan &pl,
                               hipStream_t st) {
-  int nwg = 0;
-  staged_plan_size(g, nwg, pl.nslab, pl.ngc);
-  hipLaunchKernelGGL(k_staged_plan, dim3(nwg), dim3(256), 0, st, g.grid, rays, g.P, pl.nslab,
-                     pl.ngc, pl.axis, pl.range);
+  hipLaunchKernelGGL(k_staged_plan, dim3(pl.ngroups * pl.ngc), dim3(256), 0, st, g.grid, rays,
+                     pl.order, pl.group, pl.H, staged_pixels(pl.sb) / pl.H, pl.nslab, pl.ngc,
+                     pl.range);
   return hipGetLastError();
 }
 
 hipError_t launch_forward_staged(const Geometry &g, const RayInfo *rays, const StagedPlan &pl,
                                  int mode, bool exact, const float *xb, const float *sino,
                                  float *out, unsigned *maxw, hipStream_t st) {
-  if (mode == kFwdOutY)
-    return exact ? staged_launch<kFwdOutY, true>(g, rays, pl, xb, sino, out, maxw, st)
-                 : staged_launch<kFwdOutY, false>(g, rays, pl, xb, sino, out, maxw, st);
-  if (mode == kFwdOutSIRT)
-    return exact ? staged_launch<kFwdOutSIRT, true>(g, rays, pl, xb, sino, out, maxw, st)
-                 : staged_launch<kFwdOutSIRT, false>(g, rays, pl, xb, sino, out, maxw, st);
-  return exact ? staged_launch<kFwdOutEM, true>(g, rays, pl, xb, sino, out, maxw, st)
-               : staged_launch<kFwdOutEM, false>(g, rays, pl, xb, sino, out, maxw, st);
+#define TRACE_ST_CASE(SB_, H_)                                                             \
+  if (pl.sb == SB_ && pl.H == H_)                                                          \
+    return staged_mode<SB_, H_>(g, rays, pl, mode, exact, xb, sino, out, maxw, st);
+  TRACE_ST_CASE(32, 4)
+  TRACE_ST_CASE(32, 2)
+  TRACE_ST_CASE(32, 1)
+  TRACE_ST_CASE(16, 4)
+  TRACE_ST_CASE(16, 2)
+  TRACE_ST_CASE(8, 4)
+  TRACE_ST_CASE(8, 2)
+  TRACE_ST_CASE(4, 4)
+  TRACE_ST_CASE(4, 2)
+#undef TRACE_ST_CASE
+  return hipErrorInvalidValue;
 }
 
 }  // namespace trace_hip

@@ -249,13 +249,20 @@ struct Walker {
   // shorter square root one 2048^2 slice at 1500 angles projects forward in
   // 8.7 ms instead of 9.9 and back in 12.5 instead of 14.0.
   __device__ __forceinline__ void next(float &qx, float &qy) {
-    uint64_t save, lt;
+    uint64_t none;
+    next(qx, qy, none);
+  }
+  // The same, with the mask of the lanes whose lists held no element to emit
+  // (their q is meaningless).
+  __device__ __forceinline__ void next(float &qx, float &qy, uint64_t &none) {
+    uint64_t save;
     asm volatile(
         "v_cmp_neq_f32 vcc, %[ay], %[ay_end]\n\t"
-        "v_cmp_lt_f32 %[lt], %[ax], %[bx]\n\t"
-        "v_cmp_eq_f32 %[save], %[bx], %[bx_end]\n\t"
-        "s_or_b64 %[lt], %[lt], %[save]\n\t"
-        "s_and_b64 vcc, vcc, %[lt]\n\t"
+        "v_cmp_lt_f32 %[save], %[ax], %[bx]\n\t"
+        "v_cmp_eq_f32 %[none], %[bx], %[bx_end]\n\t"
+        "s_or_b64 %[save], %[save], %[none]\n\t"
+        "s_andn2_b64 %[none], %[none], vcc\n\t"
+        "s_and_b64 vcc, vcc, %[save]\n\t"
         "s_mov_b64 %[save], exec\n\t"
         "v_cndmask_b32 %[qx], %[bx], %[ax], vcc\n\t"
         "s_andn2_b64 exec, %[save], vcc\n\t"
@@ -271,7 +278,7 @@ struct Walker {
         "v_add_f32 %[ax], %[ax], %[srcx]\n\t"
         "s_mov_b64 exec, %[save]"
         : [qx] "=&v"(qx), [qy] "=&v"(qy), [ax] "+v"(ax), [ay] "+v"(ay), [bx] "+v"(bx),
-          [save] "=&s"(save), [lt] "=&s"(lt)
+          [save] "=&s"(save), [none] "=&s"(none)
         : [ay_end] "v"(ay_end), [bx_end] "v"(bx_end), [srcx] "v"(srcx), [srcy] "v"(srcy),
           [slope] "v"(slope), [islope] "v"(islope), [dA] "v"(dA)
         : "vcc", "scc");
