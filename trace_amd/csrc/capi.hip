@@ -485,14 +485,32 @@ int trace_create(trace_handle_t **out, const trace_geom_t *g, int device,
   // default launch shape by stack depth (the fastest measured at 2048^2,
   // 1500 angles; trace_amd.autotune refines it for a given geometry)
   const int S = g->num_slices;
-  if (S >= 32) {
+  const int n = g->num_grids;
+  // backprojector: the stack in one batch up to 32 slices.  A 32x32 tile's
+  // pairs serve more segments for their set-up than a 16x16 tile's, but it
+  // pays only where the tiles fill the 256 CUs once, nearly, or a few times;
+  // the deeper the batch (LDS and registers then hold fewer workgroups) the
+  // more.  One launch, 16x16 / 32x32 tiles (us):
+  //   4 slices    400^2, 300 angles 202 / 217    512^2, 360 308 / 258
+  //               560^2, 400        404 / 525   1100^2, 700 2196 / 1906
+  //   8 slices    512^2             350 / 288    600^2, 361 471 / 531
+  //              1100^2            2504 / 2142
+  //   16 slices   512^2             532 / 448    600^2      773 / 847
+  //              1100^2            3746 / 3837  2048^2, 1500 24999 / 25227
+  //   64 slices  2048^2, in batches of 32 82.9 ms, of 16 in 32x32 95.9 ms
+  const double fill = (double)((n + 31) / 32) * ((n + 31) / 32) / 256;
+  const bool once = fill >= 0.75 && fill <= 1.0;
+  if (S > 16) {
     h->tile = TileShape{16, 16, 32};
-  } else if (S >= 16) {
-    h->tile = TileShape{16, 16, 16};
-  } else if (S >= 8) {
-    h->tile = TileShape{16, 16, 8};
+  } else if (S > 8) {
+    const int side = once ? 32 : 16;
+    h->tile = TileShape{side, side, 16};
+  } else if (S > 4) {
+    const int side = once || fill >= 3.5 ? 32 : 16;
+    h->tile = TileShape{side, side, 8};
   } else {
-    h->tile = TileShape{32, 32, 4};
+    const int side = once || fill >= 1.5 ? 32 : 16;
+    h->tile = TileShape{side, side, S > 2 ? 4 : 2};
   }
   // forward: the stack in one batch up to 32 slices (a deeper batch walks
   // each ray once for all: 2048^2, 1500 angles, 4 / 8 / 16 / 32 slices in one
@@ -506,14 +524,13 @@ int trace_create(trace_handle_t **out, const trace_geom_t *g, int device,
   } else if (S >= 3) {
     h->fwd_sb = 4, h->fwd_lanes = 1;
   } else if (S == 2) {
-    h->fwd_sb = 2, h->fwd_lanes = 1, h->tile = TileShape{32, 32, 2};
+    h->fwd_sb = 2, h->fwd_lanes = 1;
   } else {
     // one slice: one atomic per segment, so larger tiles pay off as the
     // image grows (the autotuner's picks at 1500 angles: 16x16 up to 512
     // pixels, 32x32 at 1024 and 1536, 64x64 at 2048)
-    const int n = g->num_grids > 0 ? g->num_grids : g->num_cols;
-    const int side = n >= 1792 ? 64 : (n >= 768 ? 32 : 16);
-    h->fwd_sb = 1, h->fwd_lanes = 1, h->tile = TileShape{side, side, 1};
+    const int one = n >= 1792 ? 64 : (n >= 768 ? 32 : 16);
+    h->fwd_sb = 1, h->fwd_lanes = 1, h->tile = TileShape{one, one, 1};
   }
   // 16 angles x 1 column per wavefront at four lanes per ray (measured at
   // 2048^2 / 1500 angles: 110 vs 116 ms for 8 angles x 2 columns), 8 x 8/LPR

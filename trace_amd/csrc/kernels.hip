@@ -25,6 +25,7 @@
 // DISP replicas + tree merge, disp_engine_reduction.h:104-185).
 #include <hip/hip_runtime.h>
 
+#include <climits>
 #include <type_traits>
 
 #include "internal.h"
@@ -376,6 +377,8 @@ __device__ __forceinline__ int fixed_exponent(float maxw, float maxlen, bool &fi
   return 29 - ilogbf(m);
 }
 
+constexpr int kNotFixed = INT_MIN;  // exponent of a slice summed in float
+
 // Scale exponent of a weights slice (kBpSino): both bounds above.
 __device__ __forceinline__ int weight_exponent(float maxw, float denmax, float maxlen,
                                                bool &fixed) {
@@ -389,14 +392,21 @@ __device__ __forceinline__ int weight_exponent(float maxw, float denmax, float m
 constexpr float kRoundMagic = 12582912.0f;        // 1.5 * 2^23
 constexpr unsigned kRoundMagicBits = 0x4B400000u;  // its bits
 
-// Bits of 1.5 * 2^23 + rne(len * ws), for |len * ws| < 2^22.
-__device__ __forceinline__ unsigned fixed_bits(float len, float ws) {
-  return __float_as_uint(__builtin_fmaf(len, ws, kRoundMagic));
+// The rounding constant of a slice with scale exponent e, 1.5 * 2^(23 - e):
+// fl(len * w + it) is it + 2^-e rne(len * w * 2^e) exactly, so its bits minus
+// the constant's are the integer term, without scaling the weights first.
+// Its exponent must be a float's (e in [-100, 140]).
+__device__ __forceinline__ bool has_magic(int e) { return e >= -100 && e <= 140; }
+__device__ __forceinline__ float slice_magic(int e) { return ldexpf(1.5f, 23 - e); }
+
+// Bits of `magic` + rne(len * w) in the last place of a slice's magic.
+__device__ __forceinline__ unsigned fixed_bits(float len, float w, float magic) {
+  return __float_as_uint(__builtin_fmaf(len, w, magic));
 }
 
 // rne(len * ws) as an integer, for |len * ws| < 2^22.
 __device__ __forceinline__ int fixed_term(float len, float ws) {
-  return (int)(fixed_bits(len, ws) - kRoundMagicBits);
+  return (int)(fixed_bits(len, ws, kRoundMagic) - kRoundMagicBits);
 }
 
 // Accumulator word of a mode: the weights backprojector sums 32-bit fixed
@@ -409,10 +419,10 @@ using BpWord = typename std::conditional<MODE == kBpSino, unsigned, unsigned lon
 // word, planes [SB/2][TH][TW + 1] of 64-bit words, the even slice in the
 // low half, then one plane [TH][TW + 1] of 32-bit per-pixel term counts.
 // When every slice of the batch is fixed point, one ds_add_u64 adds both
-// terms as the raw fma results: with a, b the rounded terms and M the bits
-// of 1.5 * 2^23, the 64-bit value 2^32 (M + b) + (M + a) is exact (both
-// halves are positive and below 2^31), so after n terms the word holds
-// 2^32 (n M + sum b) + n M + sum a (mod 2^64).  Subtracting n M (2^32 + 1)
+// terms as the raw fma results: with a, b the rounded terms and M, L the bits
+// of the two slices' magics, the 64-bit value 2^32 (L + b) + (M + a) is exact
+// (both halves are positive and below 2^31), so after n terms the word holds
+// 2^32 (n L + sum b) + n M + sum a (mod 2^64).  Subtracting n (2^32 L + M)
 // leaves 2^32 sum(b) + sum(a): its low half is sum(a) (|sum(a)| < 2^31) and
 // the rest / 2^32 is sum(b).  A term then costs one fma per slice and the
 // two slices one ds_add_u64; the count costs one ds_add_u32 per segment.
@@ -439,11 +449,11 @@ struct BpPacked {
 // walks the flagged rays through the strip just left of the right edge,
 // rows ty0-1 .. ty1-1, and adds only their wrapped segments.  Each segment
 // is added by exactly one pass.
-template <int TW, int TH, int SB, int MODE, bool kExact, bool ALLFX, bool EDGE>
+template <int TW, int TH, int SB, int MODE, bool kExact, bool ALLFX, bool EDGE, int BLK>
 __device__ __forceinline__ void bp_tile_loop(const TileArgs &a, BpWord<MODE> *acc,
                                              const int *count, int tx0, int tx1, int ty0,
-                                             int ty1, int b, const int (&ex)[SB],
-                                             const bool (&fx)[SB]) {
+                                             int ty1, int b, const int *ex,
+                                             const float (&magic)[SB]) {
   static_assert(SB <= kWeightPad, "a slice batch of weights past the last row must be allocated");
   constexpr int PITCH = TilePitch<TW, TH>::kPitch;
   constexpr int PLANE = TilePitch<TW, TH>::kPlane;
@@ -456,7 +466,8 @@ __device__ __forceinline__ void bp_tile_loop(const TileArgs &a, BpWord<MODE> *ac
   const float y0 = grid_line(N, wy0), y1 = grid_line(N, wy1);
   // the strip's column range is at most one wider than a tile's
   constexpr int extra = EDGE ? 1 : 0;
-  // Lane t takes flat slots t, t + kTileBlock, ... of the tile's (angle,
+  const bool full = (b + 1) * SB <= a.S;  // no slot past the stack's last slice
+  // Lane t takes flat slots t, t + BLK, ... of the tile's (angle,
   // column) pairs.  One slice (kRank): slot f is rank r = f / P of angle
   // p = f % P, rank r being the r-th of the angle's column slots counted
   // from the middle of its range outward, so the lanes of a wavefront take
@@ -467,16 +478,19 @@ __device__ __forceinline__ void bp_tile_loop(const TileArgs &a, BpWord<MODE> *ac
   // same rank walk nearly the same pixels, and their LDS atomics contend
   // for one address; that costs little with one atomic per segment, and too
   // much with one per slice pair (measured: 15.4 vs 19.8 ms for one
-  // 2048^2 slice at 32x32 tiles; 532 vs 109 ms for 64 slices).
+  // 2048^2 slice at 32x32 tiles; 532 vs 109 ms for 64 slices).  One wavefront
+  // takes kRankG adjacent ranks, which halves and quarters the lanes that
+  // meet at one address.
   constexpr bool kRank = (SB == 1);
+  constexpr int kRankG = 4;
   constexpr int kRanks = isqrt_ceil(TW * TW + TH * TH) + 4 + extra;  // >= count[p] + extra
   // Slot iteration: (r, p, k) -> the lane's next (angle, column slot).
   auto advance = [&](int &r, int &p, int &k) {
     if (kRank) {
-      p += kTileBlock;
-      while (p >= a.P) { p -= a.P; ++r; }
+      p += BLK / kRankG;
+      while (p >= a.P) { p -= a.P; r += kRankG; }
     } else {
-      k += kTileBlock;
+      k += BLK;
       while (p < a.P && k >= count[p] + extra) { k -= count[p] + extra; ++p; }
     }
   };
@@ -541,8 +555,9 @@ __device__ __forceinline__ void bp_tile_loop(const TileArgs &a, BpWord<MODE> *ac
   };
   int r = 0, p = 0, k = threadIdx.x;
   if (kRank) {
-    r = threadIdx.x / a.P;
-    p = threadIdx.x % a.P;
+    const int g = threadIdx.x / kRankG;
+    r = g / a.P * kRankG + threadIdx.x % kRankG;
+    p = g % a.P;
   } else {
     while (p < a.P && k >= count[p] + extra) { k -= count[p] + extra; ++p; }
   }
@@ -564,36 +579,45 @@ __device__ __forceinline__ void bp_tile_loop(const TileArgs &a, BpWord<MODE> *ac
     Pair nxt;
     fetch(sn, angn, nxt);
     if (cur.ok) {
-      // weights pre-scaled by 2^e (exact: a power-of-two scaling commutes
-      // with rounding), so fl(len * ws) = fl(len * w) * 2^e per segment
+      // ALLFX takes the weights as they are and rounds by the slices' magics;
+      // otherwise they are pre-scaled by 2^e (exact: a power-of-two scaling
+      // commutes with rounding, so fl(len * ws) = fl(len * w) * 2^e)
       float wv[SB];
       bool any = true;
       if (MODE == kBpSino) {
-        any = false;
+        unsigned nz = 0;
 #pragma unroll
         for (int q = 0; q < SB; ++q) {
           // slots past the stack's last slice (read from the next row) add 0
-          const float wq = b * SB + q < a.S ? cur.w[q] : 0.f;
-          any |= (wq != 0.f);
-          wv[q] = (ALLFX || fx[q]) ? ldexpf(wq, ex[q]) : wq;
+          const float wq = full || b * SB + q < a.S ? cur.w[q] : 0.f;
+          nz |= __float_as_uint(wq);
+          wv[q] = (!ALLFX && ex[q] != kNotFixed) ? ldexpf(wq, ex[q]) : wq;
         }
+        any = (nz << 1) != 0;  // some weight is not +-0
       } else if (MODE == kBpOnes) {
         wv[0] = ldexpf(1.0f, ex[0]);
       }
       if (any && (!EDGE || (cur.ray.alo & kRayWraps))) {
         traverse_window<kExact, kRank>(a.g, cur.ray, cur.quadrant, wx0, wx1, wy0, wy1,
                                 [&](int ix, int iy, float l, float) {
-          // ix == N is pixel 0 of the next row (truncation); this pass takes
-          // the wrapped segments (EDGE) or the others (the bounds test below
-          // rejects the rest without a branch of its own)
-          const bool wrap = (ix == N);
-          const bool take = EDGE ? wrap : !wrap;
-          ix = wrap ? 0 : ix;
-          iy = wrap ? iy + 1 : iy;
-          const unsigned lx = take ? (unsigned)(ix - tx0) : 0xffffffffu;
-          const unsigned ly = (unsigned)(iy - ty0);
-          if (lx < (unsigned)(tx1 - tx0) && ly < (unsigned)(ty1 - ty0)) {
-            BpWord<MODE> *dst = acc + ly * PITCH + lx;
+          // ix == N is pixel 0 of the next row (truncation).  The edge pass
+          // takes those segments; the others reject them, as no tile has a
+          // pixel column N (a cell past the image in a tile cut by its edge
+          // is summed but not written out).
+          bool in;
+          unsigned lx, ly;
+          if constexpr (EDGE) {
+            lx = 0;
+            ly = (unsigned)(iy + 1 - ty0);
+            in = ix == N && ly < (unsigned)(ty1 - ty0);
+          } else {
+            lx = (unsigned)(ix - tx0);
+            ly = (unsigned)(iy - ty0);
+            in = lx < (unsigned)TW && ly < (unsigned)TH;
+          }
+          if (in) {
+            const unsigned cell = __umul24(ly, PITCH) + lx;
+            BpWord<MODE> *dst = acc + cell;
             if (MODE == kBpCount) {
               atomicAdd(dst, (BpWord<MODE>)1);
             } else if (MODE == kBpOnes) {
@@ -601,20 +625,21 @@ __device__ __forceinline__ void bp_tile_loop(const TileArgs &a, BpWord<MODE> *ac
               atomicAdd(dst, (BpWord<MODE>)(long long)(int)(l * wv[0]));
             } else if (BpPacked<MODE, SB>::value) {
               // 32-bit index of the pixel's 64-bit word in pair plane 0
-              unsigned *d2 = reinterpret_cast<unsigned *>(acc) + 2 * (ly * PITCH + lx);
+              unsigned *d2 = reinterpret_cast<unsigned *>(acc) + 2 * cell;
 #pragma unroll
               for (int k2 = 0; k2 < SB / 2; ++k2) {
                 unsigned *dk = d2 + 2 * k2 * PLANE;
                 if (ALLFX) {
                   const unsigned long long v =
-                      ((unsigned long long)fixed_bits(l, wv[2 * k2 + 1]) << 32) |
-                      fixed_bits(l, wv[2 * k2]);
+                      ((unsigned long long)fixed_bits(l, wv[2 * k2 + 1], magic[2 * k2 + 1])
+                       << 32) |
+                      fixed_bits(l, wv[2 * k2], magic[2 * k2]);
                   atomicAdd(reinterpret_cast<unsigned long long *>(dk), v);
                 } else {
 #pragma unroll
                   for (int h = 0; h < 2; ++h) {
                     const int q = 2 * k2 + h;
-                    if (fx[q])
+                    if (ex[q] != kNotFixed)
                       atomicAdd(dk + h, (unsigned)fixed_term(l, wv[q]));
                     else
                       atomicAdd(reinterpret_cast<float *>(dk + h), l * wv[q]);
@@ -623,11 +648,14 @@ __device__ __forceinline__ void bp_tile_loop(const TileArgs &a, BpWord<MODE> *ac
               }
               // terms per pixel, for the magic offsets of the ALLFX words
               if (ALLFX)
-                atomicAdd(reinterpret_cast<unsigned *>(acc) + SB * PLANE + ly * PITCH + lx, 1u);
+                atomicAdd(reinterpret_cast<unsigned *>(acc) + SB * PLANE + cell, 1u);
             } else {
 #pragma unroll
               for (int q = 0; q < SB; ++q) {
-                if (ALLFX || fx[q]) {
+                if (ALLFX) {
+                  atomicAdd(dst + q * PLANE, (BpWord<MODE>)(fixed_bits(l, wv[q], magic[q]) -
+                                                            __float_as_uint(magic[q])));
+                } else if (ex[q] != kNotFixed) {
                   atomicAdd(dst + q * PLANE, (BpWord<MODE>)fixed_term(l, wv[q]));
                 } else {
                   atomicAdd(reinterpret_cast<float *>(dst + q * PLANE), l * wv[q]);
@@ -662,7 +690,7 @@ constexpr int bp_acc_words() {
 // dynamic LDS (bp_acc_words() words of BpWord<MODE>, then int count[P]
 // when a.count_lds); the body starts and ends with a workgroup barrier, so a
 // persistent workgroup may run it for one tile after another.
-template <int TW, int TH, int SB, int MODE, bool kExact>
+template <int TW, int TH, int SB, int MODE, bool kExact, int BLK>
 __device__ __forceinline__ void bp_tile_body(const TileArgs &a, int tile, int b,
                                              unsigned long long *lds) {
   BpWord<MODE> *acc = reinterpret_cast<BpWord<MODE> *>(lds);
@@ -676,37 +704,49 @@ __device__ __forceinline__ void bp_tile_body(const TileArgs &a, int tile, int b,
   const int tx = tile % tiles_x, ty = tile / tiles_x;
   const int tx0 = tx * TW, ty0 = ty * TH;
   const int tx1 = min(tx0 + TW, N), ty1 = min(ty0 + TH, N);
-  __syncthreads();  // the previous tile's write-out has read acc
-  for (int i = threadIdx.x; i < WORDS; i += kTileBlock) acc[i] = 0;
+  __syncthreads();  // the previous tile's write-out has read acc and s_ex
+  for (int i = threadIdx.x; i < WORDS; i += BLK) acc[i] = 0;
   if (a.count_lds)
-    for (int i = threadIdx.x; i < a.P; i += kTileBlock) lcount[i] = a.count[i];
-  // per-slice scale exponents (uniform across the workgroup)
-  int ex[SB];
-  bool fx[SB];
-  bool all_fixed = true;
+    for (int i = threadIdx.x; i < a.P; i += BLK) lcount[i] = a.count[i];
+  // Per-slice scale exponents (kNotFixed: a float slice) in LDS, where the
+  // write-out and the mixed form read them; the all-fixed loop takes the
+  // slices' magics, uniform, straight into its fused multiply-adds (kept per
+  // slice with a flag each, they spilled 400 scalar registers at 32 slices).
+  __shared__ int s_ex[SB];
+  bool fixed = true;
+  if (threadIdx.x < SB) {
+    const int s = b * SB + (int)threadIdx.x;
+    int e;
+    if (MODE == kBpSino)
+      e = weight_exponent((s < a.S) ? __uint_as_float(a.maxw[s]) : 0.f, a.denmax, a.maxlen,
+                          fixed);
+    else
+      e = fixed_exponent(1.0f, a.maxlen, fixed);
+    s_ex[threadIdx.x] = fixed ? e : kNotFixed;
+    fixed = fixed && (MODE != kBpSino || has_magic(e));
+  }
+  const bool all_fixed = __syncthreads_and(fixed);
+  float magic[SB];
 #pragma unroll
   for (int q = 0; q < SB; ++q) {
-    const int s = b * SB + q;
-    if (MODE == kBpSino)
-      ex[q] = weight_exponent((s < a.S) ? __uint_as_float(a.maxw[s]) : 0.f, a.denmax, a.maxlen,
-                              fx[q]);
-    else
-      ex[q] = fixed_exponent(1.0f, a.maxlen, fx[q]);
-    all_fixed &= fx[q];
+    magic[q] = slice_magic(all_fixed ? s_ex[q] : 0);
+    // scalar registers hold up to 16 of them beside the rest
+    if constexpr (SB <= 16)
+      magic[q] = __uint_as_float((unsigned)__builtin_amdgcn_readfirstlane(
+          (int)__float_as_uint(magic[q])));
   }
-  __syncthreads();
   if (MODE == kBpCount || all_fixed) {
-    bp_tile_loop<TW, TH, SB, MODE, kExact, true, false>(a, acc, count, tx0, tx1, ty0, ty1, b, ex,
-                                                        fx);
+    bp_tile_loop<TW, TH, SB, MODE, kExact, true, false, BLK>(a, acc, count, tx0, tx1, ty0, ty1, b,
+                                                        s_ex, magic);
     if (tx0 == 0 && a.wraps)
-      bp_tile_loop<TW, TH, SB, MODE, kExact, true, true>(a, acc, count, tx0, tx1, ty0, ty1, b,
-                                                         ex, fx);
+      bp_tile_loop<TW, TH, SB, MODE, kExact, true, true, BLK>(a, acc, count, tx0, tx1, ty0, ty1, b,
+                                                         s_ex, magic);
   } else {
-    bp_tile_loop<TW, TH, SB, MODE, kExact, false, false>(a, acc, count, tx0, tx1, ty0, ty1, b,
-                                                         ex, fx);
+    bp_tile_loop<TW, TH, SB, MODE, kExact, false, false, BLK>(a, acc, count, tx0, tx1, ty0, ty1, b,
+                                                         s_ex, magic);
     if (tx0 == 0 && a.wraps)
-      bp_tile_loop<TW, TH, SB, MODE, kExact, false, true>(a, acc, count, tx0, tx1, ty0, ty1, b,
-                                                          ex, fx);
+      bp_tile_loop<TW, TH, SB, MODE, kExact, false, true, BLK>(a, acc, count, tx0, tx1, ty0, ty1, b,
+                                                          s_ex, magic);
   }
   __syncthreads();
   // coalesced write-out: plane by plane, row-contiguous
@@ -716,13 +756,14 @@ __device__ __forceinline__ void bp_tile_body(const TileArgs &a, int tile, int b,
     const unsigned *nterms = reinterpret_cast<const unsigned *>(acc) + SB * PLANE;
 #pragma unroll
     for (int k2 = 0; k2 < SB / 2; ++k2) {
-      for (int i = threadIdx.x; i < w_ * h_; i += kTileBlock) {
+      for (int i = threadIdx.x; i < w_ * h_; i += BLK) {
         const int ly = i / w_, lx = i - ly * w_;
         unsigned long long v = acc64[k2 * PLANE + ly * PITCH + lx];
-        // remove the magic offsets: n * (2^32 + 1) * bits(1.5 * 2^23), mod 2^64
+        // remove the magic offsets, n times both slices' bits, mod 2^64
         if (all_fixed)
           v -= (unsigned long long)nterms[ly * PITCH + lx] *
-               (((unsigned long long)kRoundMagicBits << 32) | kRoundMagicBits);
+               (((unsigned long long)__float_as_uint(magic[2 * k2 + 1]) << 32) |
+                __float_as_uint(magic[2 * k2]));
         const int lo = (int)(unsigned)v;
         const int hi = (int)(((long long)v - (long long)lo) >> 32);
         const int64_t o = (int64_t)(ty0 + ly) * N + tx0 + lx;
@@ -733,10 +774,10 @@ __device__ __forceinline__ void bp_tile_body(const TileArgs &a, int tile, int b,
           if (s >= a.S) break;
           const unsigned half = h ? (unsigned)(v >> 32) : (unsigned)v;
           float out;
-          if (!fx[q])
+          if (s_ex[q] == kNotFixed)
             out = __uint_as_float(half);
           else
-            out = (float)ldexp((double)(all_fixed ? (h ? hi : lo) : (int)half), -ex[q]);
+            out = (float)ldexp((double)(all_fixed ? (h ? hi : lo) : (int)half), -s_ex[q]);
           a.z[(int64_t)s * N * N + o] = out;
         }
       }
@@ -748,28 +789,28 @@ __device__ __forceinline__ void bp_tile_body(const TileArgs &a, int tile, int b,
     const int s = b * SB + q;
     if (MODE == kBpSino && s >= a.S) break;
     float *zs = a.z + (int64_t)s * N * N;
-    for (int i = threadIdx.x; i < w_ * h_; i += kTileBlock) {
+    for (int i = threadIdx.x; i < w_ * h_; i += BLK) {
       const int ly = i / w_, lx = i - ly * w_;
       const BpWord<MODE> v = acc[q * PLANE + ly * PITCH + lx];
       float out;
       if (MODE == kBpCount)
         out = (float)v;
-      else if (!fx[q])
+      else if (s_ex[q] == kNotFixed)
         out = __uint_as_float((unsigned)v);
       else if (MODE == kBpSino)
-        out = (float)ldexp((double)(int)v, -ex[q]);
+        out = (float)ldexp((double)(int)v, -s_ex[q]);
       else
-        out = (float)ldexp((double)(long long)v, -ex[q]);
+        out = (float)ldexp((double)(long long)v, -s_ex[q]);
       zs[(int64_t)(ty0 + ly) * N + tx0 + lx] = out;
     }
   }
 }
 
-template <int TW, int TH, int SB, int MODE, bool kExact>
-__global__ void __launch_bounds__(kTileBlock)
+template <int TW, int TH, int SB, int MODE, bool kExact, int BLK>
+__global__ void __launch_bounds__(BLK)
 k_bp_tile(TileArgs a) {
   extern __shared__ unsigned long long acc[];
-  bp_tile_body<TW, TH, SB, MODE, kExact>(a, blockIdx.x, blockIdx.y, acc);
+  bp_tile_body<TW, TH, SB, MODE, kExact, BLK>(a, blockIdx.x, blockIdx.y, acc);
 }
 
 // Per-slice maximum of |w| over w [P][C][S] (float bits, atomicMax on the
@@ -1153,7 +1194,7 @@ k_bp_batch(const BatchSliceDev *__restrict__ d, BatchQueues q, int it) {
     a.denmax = sd.denmax;
     a.z = sd.z;
     a.wraps = sd.wraps;
-    bp_tile_body<TW, TH, 1, kBpSino, kExact>(a, item - start[k], 0, acc);
+    bp_tile_body<TW, TH, 1, kBpSino, kExact, kTileBlock>(a, item - start[k], 0, acc);
   }
 }
 
@@ -1342,7 +1383,7 @@ hipError_t fwd_exact(bool exact, int mode, const Geometry &g, const RayInfo *ray
 
 constexpr size_t kLdsBytes = 160 * 1024;
 
-template <int TW, int TH, int SB, int MODE, bool E>
+template <int TW, int TH, int SB, int MODE, bool E, int BLK>
 hipError_t bp_launch(TileArgs a, int nbatch, hipStream_t st) {
   const int N = a.g.N;
   const int tiles = ((N + TW - 1) / TW) * ((N + TH - 1) / TH);
@@ -1350,25 +1391,55 @@ hipError_t bp_launch(TileArgs a, int nbatch, hipStream_t st) {
   // stage the per-angle column counts in LDS when they fit
   a.count_lds = (lds + (size_t)a.P * sizeof(int) <= kLdsBytes / 2) ? 1 : 0;
   if (a.count_lds) lds += (size_t)a.P * sizeof(int);
-  auto kern = k_bp_tile<TW, TH, SB, MODE, E>;
+  auto kern = k_bp_tile<TW, TH, SB, MODE, E, BLK>;
   if (lds > 65536) {
     hipError_t e = hipFuncSetAttribute((const void *)kern,
                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e != hipSuccess) return e;
   }
-  hipLaunchKernelGGL(kern, dim3(tiles, nbatch), dim3(kTileBlock), lds, st, a);
+  hipLaunchKernelGGL(kern, dim3(tiles, nbatch), dim3(BLK), lds, st, a);
   return hipGetLastError();
+}
+
+// Lanes of a tile's workgroup: the fewest of 256, 512 and 1024 that leave a CU
+// with 24 wavefronts (or what the vector registers allow), counting the
+// workgroups there are and those whose accumulators fit its LDS; 1024 only
+// where tiles are scarce, since a workgroup ends with its slowest lane.  One
+// launch with 256 / 512 / 1024 lanes (us):
+//   1 slice, 16x16, 256^2, 180 angles      92 /    53 /    41
+//   1 slice, 32x32, 1024^2, 720 angles   1415 /  1229 /  1412
+//   1 slice, 64x64, 2048^2, 1500 angles  9233 /  8173 /  9309
+//   5 slices, 32x32x8, 1024^2, 720       2800 /  1810 /  2189
+//   12 slices, 16x16x16, 2048^2, 1500   24855 / 29672 / 37040
+int tile_block(int N, int P, int TW, int TH, int SB, int nbatch) {
+  const int64_t tiles = (int64_t)((N + TW - 1) / TW) * ((N + TH - 1) / TH) * nbatch;
+  const double per_cu = tiles / 256.0;
+  if (per_cu <= 1.0) return 1024;  // a CU holds one such workgroup
+  const size_t lds = (size_t)TH * (TW + 1) * 4 * (SB + (SB > 1 ? 1 : 0)) + (size_t)P * sizeof(int);
+  const int waves = SB <= 8 ? 28 : (SB <= 16 ? 20 : 12);  // by vector registers
+  const int want = waves < 24 ? waves : 24;
+  const double resident = std::fmin(per_cu, std::fmin((double)(kLdsBytes / lds), waves / 4.0));
+  return resident * 4 >= want ? 256 : 512;
 }
 
 template <int TW, int TH, int SB>
 hipError_t bp_mode(int mode, bool exact, const TileArgs &a, int nbatch, hipStream_t st) {
-  if (mode == kBpSino)
-    return exact ? bp_launch<TW, TH, SB, kBpSino, true>(a, nbatch, st)
-                 : bp_launch<TW, TH, SB, kBpSino, false>(a, nbatch, st);
+  if (mode == kBpSino) {
+    const int blk = tile_block(a.g.N, a.P, TW, TH, SB, nbatch);
+    if constexpr (SB <= 16)
+      if (blk == 1024)
+        return exact ? bp_launch<TW, TH, SB, kBpSino, true, 1024>(a, nbatch, st)
+                     : bp_launch<TW, TH, SB, kBpSino, false, 1024>(a, nbatch, st);
+    if (blk >= 512)
+      return exact ? bp_launch<TW, TH, SB, kBpSino, true, 512>(a, nbatch, st)
+                   : bp_launch<TW, TH, SB, kBpSino, false, 512>(a, nbatch, st);
+    return exact ? bp_launch<TW, TH, SB, kBpSino, true, 256>(a, nbatch, st)
+                 : bp_launch<TW, TH, SB, kBpSino, false, 256>(a, nbatch, st);
+  }
   if (mode == kBpOnes)
-    return exact ? bp_launch<TW, TH, 1, kBpOnes, true>(a, 1, st)
-                 : bp_launch<TW, TH, 1, kBpOnes, false>(a, 1, st);
-  return bp_launch<TW, TH, 1, kBpCount, true>(a, 1, st);
+    return exact ? bp_launch<TW, TH, 1, kBpOnes, true, 256>(a, 1, st)
+                 : bp_launch<TW, TH, 1, kBpOnes, false, 256>(a, 1, st);
+  return bp_launch<TW, TH, 1, kBpCount, true, 256>(a, 1, st);
 }
 
 }  // namespace
