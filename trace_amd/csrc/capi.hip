@@ -223,10 +223,18 @@ int ensure_den(trace_handle *h) {
 
 // Slices per thread of the ordered backprojector: up to 32 in the tile form
 // and 8 in the per-pixel form, a divisor of the slice-batched copy's batch
-// for kOrdNum.
-static int ordered_batch(int mode, int S, int xsb, bool tile) {
+// for kOrdNum.  A tile is one wavefront, so small images take shallower
+// batches: they walk their rays more often but fill the GPU.  1536 wavefronts
+// are six per compute unit.  PML num, the tables' 16 or 32 slices per thread
+// against the batch chosen here: 21 slices 111 x 111, 708 angles 1460 -> 1233
+// us; 58 slices 94 x 94, 645 angles 1490 -> 1163; 9 slices 201 x 201, 1219
+// angles 2550 -> 2166.
+static int ordered_batch(int mode, int S, int N, int xsb, bool tile) {
   int sb = tile ? 32 : 8;
   while (sb > 1 && sb / 2 >= S) sb /= 2;
+  const int64_t tiles = (int64_t)((N + 7) / 8) * ((N + 7) / 8);
+  if (tile)
+    while (sb > 1 && tiles * nbatch(S, sb) < 1536) sb /= 2;
   if (mode == kOrdNum)
     while (sb > 1 && (xsb % sb) != 0) sb /= 2;
   return sb;
@@ -258,7 +266,7 @@ int backproject_ordered(trace_handle *h, int mode, const float *w, float *z, int
     if (int rc = ordered_den(h, h->z)) return rc;
   if (mode == kOrdNum && !h->xb) return fail(TRACE_E_INVALID, "no slice-batched image copy");
   const bool tile = h->ord_tile == 1;
-  const int sb = ordered_batch(mode, h->geo.S, h->xb_sb, tile);
+  const int sb = ordered_batch(mode, h->geo.S, h->geo.N, h->xb_sb, tile);
   // the tile form's overflow flag was checked on this geometry by the den pass
   unsigned *ovf = tile ? reinterpret_cast<unsigned *>(h->flag) : nullptr;
   TIMED(phase, launch_bp_ordered(h->geo, h->rays, mode, h->exact, w, h->xb, h->xb_sb, sb, z,

@@ -35,15 +35,22 @@
 // lanes first walk the four projections' columns through the tile at once
 // (one (projection, column) pair per lane, as the LDS tile backprojector
 // does) and drop every segment's length into an LDS slot keyed by (pixel,
-// projection, column - the pixel's first candidate column, segment number
-// of that ray in that pixel); then each lane sums its own pixel's slots in
-// (projection, column, segment) order.  A pixel sees at most three
-// candidate columns per projection (its projected width is at most sqrt 2
-// plus twice the 0.45-pixel margin), and a ray puts at most two segments in
-// one pixel on the geometries measured (two where it grazes a corner); a
-// geometry that would need more slots sets a flag when den is computed, and
-// the handle then keeps the per-pixel form.  Geometries with wrapped
-// segments use the per-pixel form.
+// projection, column modulo 3, segment number of that ray in that pixel);
+// then each lane sums its own pixel's slots in (projection, column, segment)
+// order.  A pixel sees at most three candidate columns per projection (its
+// projected width is at most sqrt 2 plus twice the 0.45-pixel margin), so
+// the column modulo 3 tells them apart, and a ray puts at most two segments
+// in one pixel, one after the other, on the geometries measured (two where
+// it grazes a corner); a geometry that would need more sets a flag when den
+// is computed, and the handle then keeps the per-pixel form.  Geometries
+// with wrapped segments use the per-pixel form.
+//
+// The walks bound the one-slice form, the sums the deeper ones.  Filing a
+// segment waits for nothing: its slot is the lane's own (the ray's column
+// modulo 3, and whether the segment before it fell in the same pixel), and
+// its presence is counted without reading the count back.  With the slot
+// from a table of first columns and the number from the count, two LDS round
+// trips a segment, the column sums of 2048^2 / 1500 took @D0 ms instead of @D1.
 #include <hip/hip_runtime.h>
 
 #include "internal.h"
@@ -212,6 +219,20 @@ constexpr int kOWave = 64;
 // projection slot (0 .. kOA-1) of a lane's phase-1 pair
 __device__ __forceinline__ int ai1_of(int lane) { return lane / kORanks; }
 
+// Column slot of a column (>= -3): its remainder modulo 3.
+__device__ __forceinline__ int column_slot(int c) { return (int)((unsigned)(c + 3) % kOSlots); }
+
+// Segments per column slot of a pixel's count word (a nibble per segment:
+// 0 or 1), two bits each, the slots in turn from m0 on.
+__device__ __forceinline__ unsigned slot_counts(unsigned word, int m0) {
+  const unsigned n = (word & 0x010101u) + ((word >> 4) & 0x010101u);  // a byte per slot
+  const unsigned r = n | (n << 24);                                   // slot 3 = slot 0
+  const unsigned n0 = (r >> (8 * m0)) & 3u;
+  const unsigned n1 = (m0 == 2 ? n : r >> (8 * m0 + 8)) & 3u;
+  const unsigned n2 = (m0 == 0 ? n >> 16 : (m0 == 1 ? n : n >> 8)) & 3u;
+  return n0 | (n1 << 2) | (n2 << 4);
+}
+
 template <int SB>
 struct OrdTileLds {
   static constexpr int kWPitch = SB >= 4 ? SB + 4 : SB;  // row pitch of s_w (bank spread)
@@ -222,13 +243,11 @@ __global__ void __launch_bounds__(kOWave)
 k_bp_ordered_tile(OrdArgs a, unsigned *__restrict__ overflow) {
   static_assert(SB <= kWeightPad, "a slice batch of weights past the last row must be allocated");
   constexpr int WP = OrdTileLds<SB>::kWPitch;
-  __shared__ unsigned s_cnt[kOA][kOWave];                  // byte counter per column slot
+  // segments filed, a nibble per (column slot, segment number)
+  __shared__ unsigned s_cnt[kOA][kOWave];
   __shared__ float s_len[kOA][kOSlots * kODups][kOWave];
   __shared__ float s_w[MODE == kOrdDen ? 1 : kOA * kORanks * WP];
   __shared__ int s_cmin[kOA];
-  // first candidate column of each pixel for the round's projections,
-  // written by the pixel's lane one round ahead (double-buffered)
-  __shared__ int s_pc0[2][kOA][kOWave];
   const int N = a.g.N, C = a.g.C;
   const int tiles_x = (N + kOT - 1) / kOT;
   const int tile = (int)xcd_chunked(blockIdx.x, gridDim.x);
@@ -269,19 +288,22 @@ k_bp_ordered_tile(OrdArgs a, unsigned *__restrict__ overflow) {
     for (int ai = 0; ai < kOA; ++ai) nxt[ai] = a.ang[min(p + ai, a.P - 1)];
     fang = a.ang[min(p + ai1_of(lane), a.P - 1)];
   };
-  // this lane's pixel's first candidate column for projections p .. p+kOA-1
-  auto pixel_columns = [&](int p, int buf) {
+  // this lane's pixel's first candidate column for a round's projections, and
+  // that column modulo 3 (columns are not negative where a ray exists)
+  int pc0[kOA], pm0[kOA];
+  auto pixel_columns = [&](int p) {
 #pragma unroll
     for (int ai = 0; ai < kOA; ++ai) {
-      int pc0 = 0, pc1;
-      if (p + ai < a.P) tile_columns(nxt[ai], pcx0, pcx1, pcy0, pcy1, a.yi0, pc0, pc1);
-      s_pc0[buf][ai][lane] = pc0;
+      int c0 = 0, c1;
+      if (p + ai < a.P) tile_columns(nxt[ai], pcx0, pcx1, pcy0, pcy1, a.yi0, c0, c1);
+      pc0[ai] = c0;
+      pm0[ai] = column_slot(c0);
     }
   };
 #pragma unroll
   for (int ai = 0; ai < kOA; ++ai) s_cnt[ai][lane] = 0;
   load_angles(0);
-  pixel_columns(0, 0);
+  pixel_columns(0);
   __syncthreads();
   const int ai1 = ai1_of(lane), k1 = lane % kORanks;  // phase-1 pair of this lane
   // The lane's phase-1 pair of a round, fetched one round ahead: its ray
@@ -324,7 +346,7 @@ k_bp_ordered_tile(OrdArgs a, unsigned *__restrict__ overflow) {
   };
   Pair cur;
   fetch(ai1, fang, cur);
-  for (int p0 = 0, buf = 0; p0 < a.P; p0 += kOA, buf ^= 1) {
+  for (int p0 = 0; p0 < a.P; p0 += kOA) {
     load_angles(p0 + kOA);
     // phase 1: walk the pairs, file each segment of the tile in its slot
     const int p = p0 + ai1;
@@ -338,23 +360,21 @@ k_bp_ordered_tile(OrdArgs a, unsigned *__restrict__ overflow) {
 #pragma unroll
           for (int q = 0; q < SB; ++q) dst[q] = b * SB + q < a.S ? cur.w[q] : 0.f;
         }
+        const int slot = column_slot(c);
+        float *len0 = &s_len[ai1][slot * kODups][0];
+        const unsigned one0 = 1u << (8 * slot);
+        int last = -1, again = 0;  // the pixel filed last, and its segment number
         traverse_window<kExact, true>(a.g, cur.ray, cur.quadrant, tx0, tx1, ty0, ty1,
                                       [&](int ix, int iy, float l, float) {
           const unsigned lx = (unsigned)(ix - tx0), ly = (unsigned)(iy - ty0);
           if (lx < (unsigned)(tx1 - tx0) && ly < (unsigned)(ty1 - ty0)) {
             const int lp = (int)(ly * kOT + lx);
-            const int slot = c - s_pc0[buf][ai1][lp];
-            if ((unsigned)slot >= (unsigned)kOSlots) {
-              atomicOr(overflow, 1u);
-              return;
-            }
-            const unsigned old = atomicAdd(&s_cnt[ai1][lp], 1u << (8 * slot));
-            const int dup = (int)((old >> (8 * slot)) & 0xffu);
-            if (dup >= kODups) {
-              atomicOr(overflow, 2u);
-              return;
-            }
-            s_len[ai1][slot * kODups + dup][lp] = l;
+            // a third segment (or a return to a pixel left) counts past 1 in
+            // its nibble, which phase 2 reports
+            again = lp == last ? 1 : 0;
+            last = lp;
+            len0[again * kOWave + lp] = l;
+            atomicAdd(&s_cnt[ai1][lp], again ? one0 << 4 : one0);
           }
         });
       }
@@ -367,8 +387,10 @@ k_bp_ordered_tile(OrdArgs a, unsigned *__restrict__ overflow) {
     // wavefront runs as many iterations as its busiest pixel has segments
     // rather than one per slot that any lane uses; with few slices the
     // decoding would cost more than it saves, and the loops nest.
-    auto add = [&](int ai, int kbase, int slot, int d) {
-      const float l = s_len[ai][slot * kODups + d][lane];
+    // `slot` counts from the pixel's first column, m0 is that one's place
+    auto add = [&](int ai, int kbase, int m0, int slot, int d) {
+      const int at = m0 + slot - (m0 + slot >= kOSlots ? kOSlots : 0);
+      const float l = s_len[ai][at * kODups + d][lane];
       if (MODE == kOrdDen) {
         acc[0] = acc[0] + l;
       } else {
@@ -384,20 +406,16 @@ k_bp_ordered_tile(OrdArgs a, unsigned *__restrict__ overflow) {
     };
     if (pix_ok && SB >= 8) {
       static_assert(kOSlots == 3 && kODups <= 3, "two-bit counts of three slots");
-      unsigned cnt[kOA];  // n0 | n1 << 2 | n2 << 4 per projection
+      unsigned cnt[kOA];  // n0 | n1 << 2 | n2 << 4 per projection, from its first column on
       int kb[kOA], end[kOA];
       int total = 0;
 #pragma unroll
       for (int ai = 0; ai < kOA; ++ai) {
-        const unsigned word = s_cnt[ai][lane];
-        s_cnt[ai][lane] = 0;
-        const unsigned n0 = min(word & 0xffu, (unsigned)kODups);
-        const unsigned n1 = min((word >> 8) & 0xffu, (unsigned)kODups);
-        const unsigned n2 = min((word >> 16) & 0xffu, (unsigned)kODups);
-        cnt[ai] = n0 | (n1 << 2) | (n2 << 4);
-        total += (int)(n0 + n1 + n2);
+        const unsigned n = slot_counts(s_cnt[ai][lane], pm0[ai]);
+        cnt[ai] = n;
+        total += (int)((n & 3u) + ((n >> 2) & 3u) + (n >> 4));
         end[ai] = total;
-        kb[ai] = s_pc0[buf][ai][lane] - s_cmin[ai];
+        kb[ai] = pc0[ai] - s_cmin[ai];
       }
       for (int k = 0; k < total; ++k) {
         // projection of the k-th segment, and its rank r within it
@@ -406,30 +424,35 @@ k_bp_ordered_tile(OrdArgs a, unsigned *__restrict__ overflow) {
         for (int i = 0; i < kOA - 1; ++i)
           if (k >= end[i]) ai = i + 1, base = end[i];
         unsigned c = cnt[0];
-        int kbase = kb[0];
+        int kbase = kb[0], m0 = pm0[0];
 #pragma unroll
         for (int i = 1; i < kOA; ++i)
-          if (ai == i) c = cnt[i], kbase = kb[i];
+          if (ai == i) c = cnt[i], kbase = kb[i], m0 = pm0[i];
         const int r = k - base;
         const int n0 = (int)(c & 3u), n01 = n0 + (int)((c >> 2) & 3u);
         const int slot = (r >= n0) + (r >= n01);
-        add(ai, kbase, slot, r - (slot == 0 ? 0 : (slot == 1 ? n0 : n01)));
+        add(ai, kbase, m0, slot, r - (slot == 0 ? 0 : (slot == 1 ? n0 : n01)));
       }
     } else if (pix_ok) {
 #pragma unroll
       for (int ai = 0; ai < kOA; ++ai) {
         const unsigned word = s_cnt[ai][lane];
         if (word == 0) continue;
-        s_cnt[ai][lane] = 0;
-        const int kbase = s_pc0[buf][ai][lane] - s_cmin[ai];
+        const unsigned n = slot_counts(word, pm0[ai]);
+        const int kbase = pc0[ai] - s_cmin[ai];
 #pragma unroll
         for (int slot = 0; slot < kOSlots; ++slot) {
-          const int n = min((int)((word >> (8 * slot)) & 0xffu), kODups);
-          for (int d = 0; d < n; ++d) add(ai, kbase, slot, d);
+          const int ns = (int)((n >> (2 * slot)) & 3u);
+          for (int d = 0; d < ns; ++d) add(ai, kbase, pm0[ai], slot, d);
         }
       }
     }
-    pixel_columns(p0 + kOA, buf ^ 1);
+#pragma unroll
+    for (int ai = 0; ai < kOA; ++ai) {
+      if (s_cnt[ai][lane] & 0xEEEEEEEEu) atomicOr(overflow, 1u);
+      s_cnt[ai][lane] = 0;
+    }
+    pixel_columns(p0 + kOA);
     __syncthreads();
   }
   if (!pix_ok) return;
