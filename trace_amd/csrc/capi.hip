@@ -360,6 +360,12 @@ float mov_of(int C, float center) {
   return mov;
 }
 
+// Whether two buffers of floats share memory.
+bool overlap(const float *a, size_t na, const float *b, size_t nb) {
+  const auto pa = reinterpret_cast<uintptr_t>(a), pb = reinterpret_cast<uintptr_t>(b);
+  return pa < pb + nb * sizeof(float) && pb < pa + na * sizeof(float);
+}
+
 // Launch shapes compiled into the library (kernels.hip, launch_backproject).
 bool fwd_shape_supported(int sb, int lanes) {
 #define TRACE_FWD_MATCH(SB_, LPR_) \
@@ -383,21 +389,19 @@ bool tile_shape_supported(int tw, int th, int sb) {
 }
 
 
-// Forward projection of xb into weights w (mode kFwdOutSIRT/EM) or y
-// (kFwdOutY), with max |w| per slice folded into h->maxw.
-int forward(trace_handle *h, int mode, const float *sino, float *out) {
-  if (mode != kFwdOutY)
-    TIMED(TRACE_PHASE_SETUP,
-          launch_fill(reinterpret_cast<float *>(h->maxw), h->geo.S, 0.f, h->stream));
+// Forward projection of the slice-batched image xb into weights w (mode
+// kFwdOutSIRT/EM) or y (kFwdOutY), with max |w| per slice folded into h->maxw,
+// which holds zeros beforehand (the image updates clear it).
+int forward(trace_handle *h, int mode, const float *xb, const float *sino, float *out) {
   if (forward_staged(h)) {
     if (int rc = ensure_staged(h)) return rc;
     TIMED(TRACE_PHASE_FORWARD, launch_forward_staged(h->geo, h->rays, h->staged, mode, h->exact,
-                                                     h->xb, sino, out, h->maxw, h->stream));
+                                                     xb, sino, out, h->maxw, h->stream));
     return TRACE_OK;
   }
   const int sb = forward_batch(h);
   TIMED(TRACE_PHASE_FORWARD, launch_forward(h->geo, h->rays, sb, h->fwd_bundle,
-                                            forward_lanes(h, sb), mode, h->exact, h->xb, sino,
+                                            forward_lanes(h, sb), mode, h->exact, xb, sino,
                                             out, h->maxw, h->stream));
   return TRACE_OK;
 }
@@ -715,9 +719,12 @@ int trace_reconstruct(trace_handle_t *h, trace_alg_t alg, int iters,
   if (int rc = ensure_rays(h)) return rc;
   if (int rc = ensure_den(h)) return rc;
   const bool reg = (alg == TRACE_PML || alg == TRACE_APMLR);
-  if (int rc = ensure_work(h, reg)) return rc;
-  hipStream_t st = h->stream;
   const int sb = forward_batch(h);
+  // with one slice to a batch the image is its own slice-batched copy
+  const bool copied = reg || sb > 1;
+  if (int rc = ensure_work(h, reg, copied)) return rc;
+  hipStream_t st = h->stream;
+  TIMED(TRACE_PHASE_SETUP, launch_fill(reinterpret_cast<float *>(h->maxw), S, 0.f, st));
   const int nslots = nbatch(S, sb) * sb;
   const int fmode = (alg == TRACE_SIRT) ? kFwdOutSIRT : kFwdOutEM;
 
@@ -729,12 +736,14 @@ int trace_reconstruct(trace_handle_t *h, trace_alg_t alg, int iters,
                    : backproject(h, kBpOutSino, h->w, h->z, TRACE_PHASE_BACK);
   };
   if (alg == TRACE_SIRT || alg == TRACE_MLEM) {
-    TIMED(TRACE_PHASE_SETUP, launch_pack(recon, S, 0, 0.f, NN, nslots, sb, h->xb, st));
+    if (copied)
+      TIMED(TRACE_PHASE_SETUP, launch_pack(recon, S, 0, 0.f, NN, nslots, sb, h->xb, st));
     for (int it = 0; it < iters; ++it) {
-      if (int rc = forward(h, fmode, sino, h->w)) return rc;
+      if (int rc = forward(h, fmode, copied ? h->xb : recon, sino, h->w)) return rc;
       if (int rc = back()) return rc;
       TIMED(TRACE_PHASE_UPDATE,
-            launch_update_em(alg == TRACE_SIRT, recon, h->z, h->den, S, NN, sb, h->xb, st));
+            launch_update_em(alg == TRACE_SIRT, recon, h->z, h->den, S, NN, sb, h->xb, h->maxw,
+                             st));
     }
     return TRACE_OK;
   }
@@ -742,10 +751,10 @@ int trace_reconstruct(trace_handle_t *h, trace_alg_t alg, int iters,
     float *cur = recon, *alt = h->xa;
     TIMED(TRACE_PHASE_SETUP, launch_pack(cur, S, 0, 0.f, NN, nslots, sb, h->xb, st));
     for (int it = 0; it < iters; ++it) {
-      if (int rc = forward(h, fmode, sino, h->w)) return rc;
+      if (int rc = forward(h, fmode, h->xb, sino, h->w)) return rc;
       if (int rc = back()) return rc;
       TIMED(TRACE_PHASE_UPDATE, launch_update_pml(cur, alt, h->z, h->den, S, g.N, prm->beta,
-                                                  ord_num, sb, nslots, h->xb, st));
+                                                  ord_num, sb, nslots, h->xb, h->maxw, st));
       std::swap(cur, alt);
     }
     if (cur != recon)
@@ -765,11 +774,11 @@ int trace_reconstruct(trace_handle_t *h, trace_alg_t alg, int iters,
   HIP_TRY(hipMemcpyAsync(pa + NN, recon, sizeof(float) * S * NN, hipMemcpyDeviceToDevice, st));
   TIMED(TRACE_PHASE_SETUP, launch_pack(pa, S + 2, off, 0.f, NN, nslots, sb, h->xb, st));
   for (int it = 0; it < iters; ++it) {
-    if (int rc = forward(h, kFwdOutEM, sino, h->w)) return rc;
+    if (int rc = forward(h, kFwdOutEM, h->xb, sino, h->w)) return rc;
     if (int rc = back()) return rc;
     TIMED(TRACE_PHASE_UPDATE, launch_update_apmlr(pa, pb, h->z, h->den, S, g.N, rp, w,
                                                   prm->apmlr_compat, ord_num, sb, nslots,
-                                                  h->xb, st));
+                                                  h->xb, h->maxw, st));
     std::swap(pa, pb);
   }
   HIP_TRY(hipMemcpyAsync(recon, pa + NN, sizeof(float) * S * NN, hipMemcpyDeviceToDevice, st));
@@ -815,12 +824,17 @@ int trace_forward(trace_handle_t *h, const float *x, float *y) {
   if (!x || !y) return fail(TRACE_E_INVALID, "null buffer");
   HIP_TRY(hipSetDevice(h->device));
   if (int rc = ensure_rays(h)) return rc;
-  if (int rc = ensure_work(h, false)) return rc;
   const Geometry &g = h->geo;
   const int sb = forward_batch(h);
-  TIMED(TRACE_PHASE_SETUP,
-        launch_pack(x, g.S, 0, 0.f, g.NN(), nbatch(g.S, sb) * sb, sb, h->xb, h->stream));
-  return forward(h, kFwdOutY, nullptr, y);
+  // with one slice to a batch the image is projected where it lies, unless
+  // the projections overwrite it
+  const bool copied =
+      sb > 1 || overlap(x, (size_t)g.S * g.NN(), y, (size_t)g.S * g.rays_per_slice());
+  if (int rc = ensure_work(h, false, copied)) return rc;
+  if (copied)
+    TIMED(TRACE_PHASE_SETUP,
+          launch_pack(x, g.S, 0, 0.f, g.NN(), nbatch(g.S, sb) * sb, sb, h->xb, h->stream));
+  return forward(h, kFwdOutY, copied ? h->xb : x, nullptr, y);
 }
 
 int trace_forward_noalloc(trace_handle_t *h, const float *x, float *y) {
@@ -857,8 +871,15 @@ int trace_adjoint(trace_handle_t *h, const float *r, float *z) {
   if (int rc = ensure_den(h)) return rc;  // fixed-point scale of A^T
   TIMED(TRACE_PHASE_SETUP,
         launch_fill(reinterpret_cast<float *>(h->maxw), h->geo.S, 0.f, h->stream));
-  TIMED(TRACE_PHASE_SETUP,
-        launch_to_pcs(r, h->geo.P, h->geo.S, h->geo.C, h->w, h->maxw, h->stream));
+  const Geometry &g = h->geo;
+  // one slice lies as the backprojector reads it; deeper tiles read past the
+  // last row, which only h->w allows
+  if (g.S == 1 && (h->tile.sb == 1 || h->backprojector != 0) &&
+      !overlap(r, (size_t)g.rays_per_slice(), z, (size_t)g.NN())) {
+    TIMED(TRACE_PHASE_SETUP, launch_absmax_slices(r, g.P, 1, g.C, h->maxw, h->stream));
+    return backproject(h, kBpOutSino, r, z, TRACE_PHASE_BACK);
+  }
+  TIMED(TRACE_PHASE_SETUP, launch_to_pcs(r, g.P, g.S, g.C, h->w, h->maxw, h->stream));
   return backproject(h, kBpOutSino, h->w, z, TRACE_PHASE_BACK);
 }
 

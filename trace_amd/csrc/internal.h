@@ -27,6 +27,15 @@ __device__ __forceinline__ int64_t xcd_chunked(int64_t b, int64_t nb) {
 // and lgkmcnt, bits 11:8, at their maxima, i.e. not waited for).
 __device__ __forceinline__ void wait_vector_loads() { __builtin_amdgcn_s_waitcnt(0x0F70); }
 
+// Raises *p (bits of a non-negative float) to m.  Every workgroup of a launch
+// does, and atomics on one address complete one after the other, about 4 ns
+// apart, so the value is read first: few workgroups then find a larger one.
+// With an atomic per wavefront and slice, and no reading, the 23 x 5000 of 23
+// slices 59 x 59 at 1361 angles took 471 us, ten times the projections (43 us).
+__device__ __forceinline__ void raise_max(unsigned *p, unsigned m) {
+  if (m > __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(p, m);
+}
+
 // Floats allocated after the [P][C][S] weights: the ordered tile kernel
 // reads a whole slice batch (up to 32 floats) from every row, so the last
 // row's partial batch stays inside the allocation.
@@ -147,6 +156,10 @@ struct BatchQueues {
   X(32, 32, 1) X(64, 64, 1) X(32, 32, 2) X(16, 16, 2) X(16, 16, 1)          \
   X(16, 16, 32) X(32, 32, 16) X(32, 16, 16) X(24, 24, 16)
 
+// (slot batch, slices per thread) of the regularised updates.
+#define TRACE_UPDATE_SHAPES(X)                                             \
+  X(1, 1) X(2, 2) X(4, 4) X(8, 8) X(16, 16) X(32, 32) X(8, 4) X(16, 4) X(32, 4)
+
 // Backprojection in the reference's summation order (ordered.hip): w
 // [P][C][S] weights, xb the slice-batched image the ray pass read (xsb
 // slices per slot batch; kOrdNum only), sb slices per thread (a divisor of
@@ -170,17 +183,19 @@ hipError_t launch_to_pcs(const float *r, int P, int S, int C, float *w, unsigned
 hipError_t launch_pack(const float *src, int nsrc, int off, float fill, int64_t NN,
                        int nslots, int sb, float *xb, hipStream_t st);
 hipError_t launch_update_em(bool sirt, float *x, const float *z, const float *den, int S,
-                            int64_t NN, int sb, float *xb, hipStream_t st);
+                            int64_t NN, int sb, float *xb, unsigned *maxw, hipStream_t st);
 hipError_t launch_fill(float *p, int64_t n, float v, hipStream_t st);
+// Every update also zeroes maxw[0..S) for the next projection.
 // num_direct: z holds num summed as the reference does (launch_bp_ordered,
 // kOrdNum); otherwise z = A^T w and num = -x * z.
 hipError_t launch_update_pml(const float *x, float *xn, const float *z, const float *den,
                              int S, int N, float beta, bool num_direct, int sb, int nslots,
-                             float *xb, hipStream_t st);
+                             float *xb, unsigned *maxw, hipStream_t st);
 hipError_t launch_update_apmlr(const float *xpad, float *xnpad, const float *z,
                                const float *den, int S, int N, const RegParams &p,
                                const StencilWeights &w, int compat, bool num_direct,
-                               int sb, int nslots, float *xb, hipStream_t st);
+                               int sb, int nslots, float *xb, unsigned *maxw,
+                               hipStream_t st);
 hipError_t launch_batch_reset(const BatchQueues &q, hipStream_t st);
 hipError_t launch_batch_forward(const BatchSliceDev *d, const BatchQueues &q, int it,
                                 int bundle_angles, bool exact, int grid, hipStream_t st);

@@ -107,8 +107,8 @@ __device__ __forceinline__ void store_slices(float *__restrict__ p, const float 
 //   SIRT  w = (p - y)/a2, a2 = sum len^2    (sirt.cc:47-52)
 //   EM    w = p/y                           (mlem.cc:50, pml.cc:236)
 // to w[p][c][s] (slices innermost, read as a block by the backprojector) and
-// fold max |w| over the rays with a segment in the image per slice into
-// maxw (bits; zeroed beforehand).
+// fold max |w| over the rays with a segment in the image per slice into the
+// workgroup's s_max[SB] (LDS, bits; zeroed beforehand).
 // LPR lanes per ray (1, 2 or 4): the lanes of one ray repeat its walk and
 // each gathers and sums SB/LPR of the batch's slices, so a gather touches
 // LPR-fold fewer distinct cache lines per wavefront instruction (the
@@ -168,9 +168,8 @@ __device__ __forceinline__ void forward_bundle(const GridInfo &g, const AngleInf
                                                const RayInfo *__restrict__ rays, int P, int S,
                                                int ba_log2, const float *__restrict__ xb,
                                                const float *__restrict__ sino,
-                                               float *__restrict__ out,
-                                               unsigned *__restrict__ maxw, int64_t bundle,
-                                               int b) {
+                                               float *__restrict__ out, unsigned *s_max,
+                                               int64_t bundle, int b) {
   static_assert(LPR == 1 || LPR == 2 || LPR == 4, "lanes per ray: 1, 2 or 4");
   static_assert(SB % LPR == 0, "slice batch must split evenly over the lanes of a ray");
   constexpr int SBL = SB / LPR;  // slices per lane
@@ -277,7 +276,7 @@ __device__ __forceinline__ void forward_bundle(const GridInfo &g, const AngleInf
       // max over the lanes holding the same slice (same sub)
       for (int off = 32; off >= LPR; off >>= 1)
         m = max(m, (unsigned)__shfl_down((int)m, off, 64));
-      if (lane < LPR && s < S) atomicMax(maxw + s, m);
+      if (lane < LPR) atomicMax(s_max + sub * SBL + k, m);
     }
   }
 }
@@ -288,27 +287,66 @@ k_forward(GridInfo g, const AngleInfo *__restrict__ ang, const RayInfo *__restri
           int P, int S, int ba_log2, const float *__restrict__ xb,
           const float *__restrict__ sino, float *__restrict__ out,
           unsigned *__restrict__ maxw) {
+  __shared__ unsigned s_max[SB];
+  if (MODE != kFwdY) {
+    if (threadIdx.x < SB) s_max[threadIdx.x] = 0;
+    __syncthreads();
+  }
   forward_bundle<SB, MODE, kExact, LPR, kWide>(
-      g, ang, rays, P, S, ba_log2, xb, sino, out, maxw,
+      g, ang, rays, P, S, ba_log2, xb, sino, out, s_max,
       xcd_chunked(blockIdx.x, gridDim.x) * (kRayBlock / 64) + (threadIdx.x >> 6), blockIdx.y);
+  if (MODE != kFwdY) {
+    __syncthreads();
+    const int s = blockIdx.y * SB + threadIdx.x;
+    if (threadIdx.x < SB && s < S) raise_max(maxw + s, s_max[threadIdx.x]);
+  }
 }
 
 // w[p][c][s] = r[p][s][c], folding max |r| per slice into maxw (zeroed
-// beforehand).  One block row per (p, s).
+// beforehand).  A workgroup transposes blocks of 64 columns x up to 32 slices
+// through LDS (rows of 64 floats in, of the slices out) and raises the maxima
+// once: 5 slices of 725 columns at 401 angles 96 -> 20 us; before, a workgroup
+// took one (p, s) and stored every S-th float.
+constexpr int kTransS = 32;
 __global__ void __launch_bounds__(256)
 k_to_pcs(const float *__restrict__ r, int P, int S, int C, float *__restrict__ w,
          unsigned *__restrict__ maxw) {
-  const int64_t ps = blockIdx.x;  // p * S + s
-  const int s = (int)(ps % S);
-  const int64_t p = ps / S;
-  unsigned m = 0;
-  for (int c = threadIdx.x; c < C; c += 256) {
-    const float v = r[ps * C + c];
-    w[(p * C + c) * S + s] = v;
-    m = max(m, __float_as_uint(__builtin_fabsf(v)));
+  __shared__ float t[kTransS][65];
+  __shared__ unsigned s_max[kTransS];
+  const int s0 = blockIdx.y * kTransS, ns = min(kTransS, S - s0);
+  const int nc = (C + 63) / 64;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  unsigned m[kTransS / 4] = {};
+  for (int64_t i = blockIdx.x; i < (int64_t)P * nc; i += gridDim.x) {
+    const int64_t p = i / nc;
+    const int c0 = (int)(i % nc) * 64, cn = min(64, C - c0);
+    if (lane < cn) {
+#pragma unroll
+      for (int j = 0; j < kTransS / 4; ++j) {
+        const int s = wave + 4 * j;
+        if (s < ns) {
+          const float v = r[(p * S + s0 + s) * C + c0 + lane];
+          t[s][lane] = v;
+          m[j] = max(m[j], __float_as_uint(__builtin_fabsf(v)));
+        }
+      }
+    }
+    __syncthreads();
+    float *dst = w + (p * C + c0) * S + s0;
+    for (int e = threadIdx.x; e < cn * ns; e += 256) {
+      const int c = e / ns, s = e - c * ns;
+      dst[(int64_t)c * S + s] = t[s][c];
+    }
+    __syncthreads();
   }
-  for (int off = 32; off > 0; off >>= 1) m = max(m, (unsigned)__shfl_down((int)m, off, 64));
-  if ((threadIdx.x & 63) == 0) atomicMax(maxw + s, m);
+#pragma unroll
+  for (int j = 0; j < kTransS / 4; ++j) {
+    for (int off = 32; off > 0; off >>= 1)
+      m[j] = max(m[j], (unsigned)__shfl_down((int)m[j], off, 64));
+    if (lane == 0) s_max[wave + 4 * j] = m[j];
+  }
+  __syncthreads();
+  if (threadIdx.x < ns) raise_max(maxw + s0 + threadIdx.x, s_max[threadIdx.x]);
 }
 
 // ------------------------------------------------------- backprojector --
@@ -823,8 +861,14 @@ k_absmax_slices(const float *__restrict__ w, int P, int S, int C, unsigned *__re
   for (int64_t i = (int64_t)blockIdx.x * kPixBlock + threadIdx.x; i < n;
        i += (int64_t)gridDim.x * kPixBlock)
     m = max(m, __float_as_uint(__builtin_fabsf(w[i * S + s])));
+  __shared__ unsigned s_max[kPixBlock / 64];
   for (int off = 32; off > 0; off >>= 1) m = max(m, (unsigned)__shfl_down((int)m, off, 64));
-  if ((threadIdx.x & 63) == 0) atomicMax(maxw + s, m);
+  if ((threadIdx.x & 63) == 0) s_max[threadIdx.x >> 6] = m;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int k = 1; k < kPixBlock / 64; ++k) m = max(m, s_max[k]);
+    raise_max(maxw + s, m);
+  }
 }
 
 // ------------------------------------------------------- pack / update --
@@ -849,14 +893,24 @@ k_pack(const float *__restrict__ src, int nsrc, int off, float fill, int64_t NN,
   store_slices<SB>(dst, v);
 }
 
+// The updates run between the backprojector, which reads the slices' largest
+// weights, and the next projection, which gathers them anew: their first
+// workgroup clears them (a launch for it took 4 us an iteration).
+__device__ __forceinline__ void clear_max(unsigned *maxw, int S) {
+  if ((blockIdx.x | blockIdx.y | blockIdx.z) == 0)
+    for (int s = threadIdx.x; s < S; s += kPixBlock) maxw[s] = 0;
+}
+
 // SIRT (sirt.cc:21-33) / MLEM (mlem.cc:21-34) update of a batch of slices
-// at pixel j, also refreshing the batched copy.
+// at pixel j, also refreshing the batched copy (with one slice to a batch x
+// is that copy).
 template <int SB, bool kSIRT>
 __global__ void __launch_bounds__(kPixBlock)
 k_update_em(float *__restrict__ x, const float *__restrict__ z, const float *__restrict__ den,
-            int S, int64_t NN, float *__restrict__ xb) {
+            int S, int64_t NN, float *__restrict__ xb, unsigned *__restrict__ maxw) {
   const int64_t j = (int64_t)blockIdx.x * kPixBlock + threadIdx.x;
   const int b = blockIdx.y;
+  clear_max(maxw, S);
   if (j >= NN) return;
   const float d = den[j];
   float v[SB];
@@ -873,8 +927,7 @@ k_update_em(float *__restrict__ x, const float *__restrict__ z, const float *__r
       v[q] = xv;
     }
   }
-  float *dst = xb + ((int64_t)b * NN + j) * SB;
-  store_slices<SB>(dst, v);
+  if (SB > 1) store_slices<SB>(xb + ((int64_t)b * NN + j) * SB, v);
 }
 
 __global__ void k_fill(float *__restrict__ p, int64_t n, float v) {
@@ -932,17 +985,17 @@ constexpr int kInnerDy[8] = {0, 0, 1, -1, 1, 1, -1, -1};
 constexpr float kPmlAxial = 0.1464466094f;
 constexpr float kPmlDiag = 0.10355339059f;
 
-// PML stencil and update of the SB slices of batch b at one pixel.
-template <int SB, bool kInner>
+// PML stencil and update of the VB slices from s0 on at one pixel.
+template <int VB, bool kInner>
 __device__ __forceinline__ void pml_pixel(const float *__restrict__ x, float *__restrict__ xn,
                                           const float *__restrict__ z, int S, int N,
                                           int64_t NN, int64_t pix, int cls, float d,
-                                          float beta, int num_direct, int b, float (&v)[SB]) {
+                                          float beta, int num_direct, int s0, float (&v)[VB]) {
   const float *w = c_pml_w[cls == 0 ? 0 : (cls <= 4 ? 1 : 2)];
   const int cnt = c_nbn[cls];
 #pragma unroll
-  for (int q = 0; q < SB; ++q) {
-    const int s = b * SB + q;
+  for (int q = 0; q < VB; ++q) {
+    const int s = s0 + q;
     v[q] = 0.f;
     if (s < S) {
       const int64_t j = (int64_t)s * NN + pix;
@@ -978,28 +1031,29 @@ __device__ __forceinline__ void pml_pixel(const float *__restrict__ x, float *__
 // num_direct, z holds num as the reference sums it (ordered.hip); otherwise
 // z = A^T w and num = -x * z (the x factor of pml.cc:243 taken out of the
 // sum).
-// A thread owns pixel (m, n) of the SB slices of slot batch b and also
-// writes the slice-batched copy xb of the new image for the next ray pass
-// (slot t = slice t; padding slots hold 0).
-template <int SB>
+// A thread owns a pixel of VB of the SB slices of a slot batch and also
+// writes their part of the slice-batched copy xb of the new image for the next
+// ray pass (slot t = slice t; padding slots hold 0).
+template <int SB, int VB>
 __global__ void __launch_bounds__(kPixBlock)
 k_update_pml(const float *__restrict__ x, float *__restrict__ xn,
              const float *__restrict__ z, const float *__restrict__ den,
-             int S, int N, float beta, int num_direct, float *__restrict__ xb) {
-  const int m = blockIdx.x * kPixBlock + threadIdx.x;
-  const int n = blockIdx.y;
-  const int b = blockIdx.z;
-  if (m >= N) return;
+             int S, int N, float beta, int num_direct, float *__restrict__ xb,
+             unsigned *__restrict__ maxw) {
+  const int pix = blockIdx.x * kPixBlock + threadIdx.x;
+  const int s0 = blockIdx.y * VB;
+  clear_max(maxw, S);
+  if (pix >= N * N) return;
   const int64_t NN = (int64_t)N * N;
-  const int64_t pix = (int64_t)n * N + m;
+  const int n = pix / N, m = pix - n * N;
   const int cls = pixel_class(m, n, N);
   const float d = den[pix];
-  float v[SB];
+  float v[VB];
   if (cls == 0)
-    pml_pixel<SB, true>(x, xn, z, S, N, NN, pix, cls, d, beta, num_direct, b, v);
+    pml_pixel<VB, true>(x, xn, z, S, N, NN, pix, cls, d, beta, num_direct, s0, v);
   else
-    pml_pixel<SB, false>(x, xn, z, S, N, NN, pix, cls, d, beta, num_direct, b, v);
-  store_slices<SB>(xb + ((int64_t)b * NN + pix) * SB, v);
+    pml_pixel<VB, false>(x, xn, z, S, N, NN, pix, cls, d, beta, num_direct, s0, v);
+  store_slices<VB>(xb + ((int64_t)(s0 / SB) * NN + pix) * SB + s0 % SB, v);
 }
 
 struct ApmlrArgs {
@@ -1010,21 +1064,21 @@ struct ApmlrArgs {
   int num_direct;  // z holds num (ordered.hip), not A^T w
 };
 
-// APMLR stencil and update of the slots of batch b at one pixel (see
+// APMLR stencil and update of the VB slots from t0 on at one pixel (see
 // k_update_apmlr).
-template <int SB, bool kInner>
+template <int VB, bool kInner>
 __device__ __forceinline__ void apmlr_pixel(const float *__restrict__ xp,
                                             float *__restrict__ xnp,
                                             const float *__restrict__ z, int S, int N,
                                             int64_t NN, int64_t pix, int cls, float d,
-                                            const ApmlrArgs &a, int b, float (&v)[SB]) {
+                                            const ApmlrArgs &a, int t0, float (&v)[VB]) {
   const int cnt = kInner ? 8 : c_nbn[cls];
   const int off = a.compat ? 0 : 1;
   const float tb = 2.0f * a.p.beta;
   const float tb1 = 2.0f * a.p.beta1;
 #pragma unroll
-  for (int q = 0; q < SB; ++q) {
-    const int pi = b * SB + q + off;  // padded slice of slot b*SB+q
+  for (int q = 0; q < VB; ++q) {
+    const int pi = t0 + q + off;  // padded slice of slot t0 + q
     float val = 0.f;
     if (pi >= 1 && pi <= S) {
       const int s = pi - 1;
@@ -1082,29 +1136,30 @@ __device__ __forceinline__ void apmlr_pixel(const float *__restrict__ xp,
 // update (apmlr.cc:3-26) over ghost-padded images [S+2][N][N]; real slice s
 // lives at padded index s+1.  The ray pass of slice s used padded slice s
 // (compat, apmlr.cc:1082-1084) or s+1, which also supplies num's x factor.
-// Thread (pixel, slot batch b): slot t of the batched copy holds padded
-// slice t + off (off = 0 compat, 1 otherwise); real slices are updated,
+// Thread (pixel, VB slots of a slot batch): slot t of the batched copy holds
+// padded slice t + off (off = 0 compat, 1 otherwise); real slices are updated,
 // ghosts (padded 0 and S+1, constant) are copied, slots past S+1 hold 0.
 // The grid covers every real slice even when its slot lies past nslots.
-template <int SB>
+template <int SB, int VB>
 __global__ void __launch_bounds__(kPixBlock)
 k_update_apmlr(const float *__restrict__ xp, float *__restrict__ xnp,
                const float *__restrict__ z, const float *__restrict__ den,
-               int S, int N, ApmlrArgs a, float *__restrict__ xb) {
-  const int m = blockIdx.x * kPixBlock + threadIdx.x;
-  const int n = blockIdx.y;
-  const int b = blockIdx.z;
-  if (m >= N) return;
+               int S, int N, ApmlrArgs a, float *__restrict__ xb,
+               unsigned *__restrict__ maxw) {
+  const int pix = blockIdx.x * kPixBlock + threadIdx.x;
+  const int t0 = blockIdx.y * VB;
+  clear_max(maxw, S);
+  if (pix >= N * N) return;
   const int64_t NN = (int64_t)N * N;
-  const int64_t pix = (int64_t)n * N + m;
+  const int n = pix / N, m = pix - n * N;
   const int cls = pixel_class(m, n, N);
   const float d = den[pix];
-  float v[SB];
+  float v[VB];
   if (cls == 0)
-    apmlr_pixel<SB, true>(xp, xnp, z, S, N, NN, pix, cls, d, a, b, v);
+    apmlr_pixel<VB, true>(xp, xnp, z, S, N, NN, pix, cls, d, a, t0, v);
   else
-    apmlr_pixel<SB, false>(xp, xnp, z, S, N, NN, pix, cls, d, a, b, v);
-  if (b * SB < a.nslots) store_slices<SB>(xb + ((int64_t)b * NN + pix) * SB, v);
+    apmlr_pixel<VB, false>(xp, xnp, z, S, N, NN, pix, cls, d, a, t0, v);
+  if (t0 < a.nslots) store_slices<VB>(xb + ((int64_t)(t0 / SB) * NN + pix) * SB + t0 % SB, v);
 }
 
 // ------------------------------------------------------------- batched --
@@ -1144,6 +1199,8 @@ __global__ void __launch_bounds__(kRayBlock)
 k_forward_batch(const BatchSliceDev *__restrict__ d, BatchQueues q, int it, int ba_log2) {
   const int *start = q.start[0];
   const int total = start[q.n];
+  __shared__ unsigned s_max[1];
+  if (threadIdx.x == 0) s_max[0] = 0;  // the next barrier: batch_next_item's
   for (;;) {
     const int item = batch_next_item(q.counters + 0);
     if (item >= total) break;
@@ -1153,7 +1210,7 @@ k_forward_batch(const BatchSliceDev *__restrict__ d, BatchQueues q, int it, int 
     const int64_t bundle = (int64_t)(item - start[k]) * (kRayBlock / 64) + (threadIdx.x >> 6);
     auto run = [&](auto mode, auto wide) {
       forward_bundle<1, decltype(mode)::value, kExact, 1, decltype(wide)::value>(
-          sd.g, sd.ang, sd.rays, sd.P, 1, ba_log2, sd.x, sd.sino, sd.w, sd.maxw, bundle, 0);
+          sd.g, sd.ang, sd.rays, sd.P, 1, ba_log2, sd.x, sd.sino, sd.w, s_max, bundle, 0);
     };
     using std::integral_constant;
     if (wide_image(sd.g.N, 1)) {
@@ -1163,6 +1220,11 @@ k_forward_batch(const BatchSliceDev *__restrict__ d, BatchQueues q, int it, int 
       run(integral_constant<int, kFwdSIRT>(), std::false_type());
     } else {
       run(integral_constant<int, kFwdEM>(), std::false_type());
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      raise_max(sd.maxw, s_max[0]);
+      s_max[0] = 0;
     }
   }
 }
@@ -1522,15 +1584,17 @@ hipError_t launch_pack(const float *src, int nsrc, int off, float fill, int64_t 
 }
 
 hipError_t launch_update_em(bool sirt, float *x, const float *z, const float *den, int S,
-                            int64_t NN, int sb, float *xb, hipStream_t st) {
+                            int64_t NN, int sb, float *xb, unsigned *maxw, hipStream_t st) {
   const int nb = (S + sb - 1) / sb;
   dim3 grid(blocks_for(NN, kPixBlock), nb), block(kPixBlock);
 #define TRACE_UPD_CASE(SB_)                                                                   \
   case SB_:                                                                                   \
     if (sirt)                                                                                 \
-      hipLaunchKernelGGL((k_update_em<SB_, true>), grid, block, 0, st, x, z, den, S, NN, xb); \
+      hipLaunchKernelGGL((k_update_em<SB_, true>), grid, block, 0, st, x, z, den, S, NN, xb, \
+                         maxw);                                                               \
     else                                                                                      \
-      hipLaunchKernelGGL((k_update_em<SB_, false>), grid, block, 0, st, x, z, den, S, NN, xb); \
+      hipLaunchKernelGGL((k_update_em<SB_, false>), grid, block, 0, st, x, z, den, S, NN, xb, \
+                         maxw);                                                               \
     break;
   switch (sb) {
     TRACE_UPD_CASE(1)
@@ -1551,53 +1615,52 @@ hipError_t launch_fill(float *p, int64_t n, float v, hipStream_t st) {
   return hipGetLastError();
 }
 
+// Slices per thread of the regularised updates: the slot batch, or 4 of it
+// where that leaves fewer than 8192 wavefronts, since a thread takes its slices
+// one after the other (some 10 divisions and a square root each).  All / 4
+// slices (us): APMLR 14 slices 82^2 58 / 18, 9 slices 511^2 59 / 39; PML 20
+// slices 151^2 45 / 14.  Where the wavefronts are there anyway whole lines of
+// the copy are written (PML 32 slices 1024^2 274).
+static bool update_split(int N, int sb, int slots) {
+  return sb > 4 && (int64_t)blocks_for((int64_t)N * N, kPixBlock) * ((slots + sb - 1) / sb) < 2048;
+}
+
 hipError_t launch_update_pml(const float *x, float *xn, const float *z, const float *den,
                              int S, int N, float beta, bool num_direct, int sb, int nslots,
-                             float *xb, hipStream_t st) {
-  dim3 grid(blocks_for(N, kPixBlock), N, nslots / sb);
-#define TRACE_PML_CASE(SB_)                                                              \
-  case SB_:                                                                              \
-    hipLaunchKernelGGL(k_update_pml<SB_>, grid, dim3(kPixBlock), 0, st, x, xn, z, den, S, \
-                       N, beta, num_direct ? 1 : 0, xb);                                  \
-    break;
-  switch (sb) {
-    TRACE_PML_CASE(1)
-    TRACE_PML_CASE(2)
-    TRACE_PML_CASE(4)
-    TRACE_PML_CASE(8)
-    TRACE_PML_CASE(16)
-    TRACE_PML_CASE(32)
-    default: return hipErrorInvalidValue;
+                             float *xb, unsigned *maxw, hipStream_t st) {
+  const unsigned bx = blocks_for((int64_t)N * N, kPixBlock);
+  const int vb = update_split(N, sb, nslots) ? 4 : sb;
+  const dim3 grid(bx, nslots / vb);
+#define TRACE_PML_CASE(SB_, VB_)                                                           \
+  if (sb == SB_ && vb == VB_) {                                                            \
+    hipLaunchKernelGGL((k_update_pml<SB_, VB_>), grid, dim3(kPixBlock), 0, st, x, xn, z,   \
+                       den, S, N, beta, num_direct ? 1 : 0, xb, maxw);                     \
+    return hipGetLastError();                                                              \
   }
+  TRACE_UPDATE_SHAPES(TRACE_PML_CASE)
 #undef TRACE_PML_CASE
-  return hipGetLastError();
+  return hipErrorInvalidValue;
 }
 
 hipError_t launch_update_apmlr(const float *xpad, float *xnpad, const float *z,
                                const float *den, int S, int N, const RegParams &p,
                                const StencilWeights &w, int compat, bool num_direct,
-                               int sb, int nslots, float *xb, hipStream_t st) {
-  // batches: every slot of the copy and every real slice's slot
+                               int sb, int nslots, float *xb, unsigned *maxw, hipStream_t st) {
+  // slots: those of the copy and every real slice's
   const int off = compat ? 0 : 1;
   const int need = (nslots > S + 1 - off) ? nslots : S + 1 - off;
-  dim3 grid(blocks_for(N, kPixBlock), N, (need + sb - 1) / sb);
+  const int vb = update_split(N, sb, need) ? 4 : sb;
+  const dim3 grid(blocks_for((int64_t)N * N, kPixBlock), (need + vb - 1) / vb);
   ApmlrArgs a{w, p, compat, nslots, num_direct ? 1 : 0};
-#define TRACE_APMLR_CASE(SB_)                                                         \
-  case SB_:                                                                           \
-    hipLaunchKernelGGL(k_update_apmlr<SB_>, grid, dim3(kPixBlock), 0, st, xpad, xnpad, z, \
-                       den, S, N, a, xb);                                              \
-    break;
-  switch (sb) {
-    TRACE_APMLR_CASE(1)
-    TRACE_APMLR_CASE(2)
-    TRACE_APMLR_CASE(4)
-    TRACE_APMLR_CASE(8)
-    TRACE_APMLR_CASE(16)
-    TRACE_APMLR_CASE(32)
-    default: return hipErrorInvalidValue;
+#define TRACE_APMLR_CASE(SB_, VB_)                                                         \
+  if (sb == SB_ && vb == VB_) {                                                            \
+    hipLaunchKernelGGL((k_update_apmlr<SB_, VB_>), grid, dim3(kPixBlock), 0, st, xpad,     \
+                       xnpad, z, den, S, N, a, xb, maxw);                                  \
+    return hipGetLastError();                                                              \
   }
+  TRACE_UPDATE_SHAPES(TRACE_APMLR_CASE)
 #undef TRACE_APMLR_CASE
-  return hipGetLastError();
+  return hipErrorInvalidValue;
 }
 
 hipError_t launch_batch_reset(const BatchQueues &q, hipStream_t st) {
@@ -1727,15 +1790,17 @@ hipError_t launch_count_segments(const Geometry &g, const RayInfo *rays,
 
 hipError_t launch_to_pcs(const float *r, int P, int S, int C, float *w, unsigned *maxw,
                          hipStream_t st) {
-  hipLaunchKernelGGL(k_to_pcs, dim3((unsigned)((int64_t)P * S)), dim3(256), 0, st, r, P, S, C,
-                     w, maxw);
+  const int64_t blocks = (int64_t)P * ((C + 63) / 64);
+  hipLaunchKernelGGL(k_to_pcs,
+                     dim3((unsigned)(blocks < 2048 ? blocks : 2048), (S + kTransS - 1) / kTransS),
+                     dim3(256), 0, st, r, P, S, C, w, maxw);
   return hipGetLastError();
 }
 
 hipError_t launch_absmax_slices(const float *w, int P, int S, int C, unsigned *maxw,
                                 hipStream_t st) {
   int64_t n = (int64_t)P * C;
-  unsigned bx = blocks_for(n, kPixBlock);
+  unsigned bx = blocks_for(n, 4 * kPixBlock);
   if (bx > 512) bx = 512;
   hipLaunchKernelGGL(k_absmax_slices, dim3(bx, S), dim3(kPixBlock), 0, st, w, P, S, C, maxw);
   return hipGetLastError();

@@ -305,6 +305,12 @@ __device__ __forceinline__ void forward_staged(
     cur = nxt;
   }
 
+  // the staged pixels are done with: the first words hold the slices' maxima
+  unsigned *s_max = reinterpret_cast<unsigned *>(slab);
+  if (MODE != kFwdOutY) {
+    if (threadIdx.x < SB) s_max[threadIdx.x] = 0;
+    __syncthreads();
+  }
 #pragma unroll
   for (int k = 0; k < SB; ++k) {
     const int s = b * SB + k;
@@ -325,8 +331,13 @@ __device__ __forceinline__ void forward_staged(
     if (MODE != kFwdOutY) {
       for (int off = 32; off >= 1; off >>= 1)
         m = max(m, (unsigned)__shfl_down((int)m, off, 64));
-      if (lane == 0 && s < S) atomicMax(maxw + s, m);
+      if (lane == 0) atomicMax(s_max + k, m);
     }
+  }
+  if (MODE != kFwdOutY) {
+    __syncthreads();
+    const int s = b * SB + threadIdx.x;
+    if (threadIdx.x < SB && s < S) raise_max(maxw + s, s_max[threadIdx.x]);
   }
 }
 
