@@ -400,6 +400,11 @@ int forward(trace_handle *h, int mode, const float *xb, const float *sino, float
     return TRACE_OK;
   }
   const int sb = forward_batch(h);
+  if (const int lanes = split_lanes(h->geo, sb)) {
+    TIMED(TRACE_PHASE_FORWARD, launch_forward_split(h->geo, h->rays, sb, lanes, mode, h->exact, xb,
+                                                    sino, out, h->maxw, h->stream));
+    return TRACE_OK;
+  }
   TIMED(TRACE_PHASE_FORWARD, launch_forward(h->geo, h->rays, sb, h->fwd_bundle,
                                             forward_lanes(h, sb), mode, h->exact, xb, sino,
                                             out, h->maxw, h->stream));

@@ -172,6 +172,14 @@ hipError_t launch_bp_ordered(const Geometry &g, const RayInfo *rays, int mode, b
                              bool wraps, unsigned *tile_overflow, hipStream_t st);
 bool ordered_sb_supported(int mode, int sb, int xsb);
 
+// Forward projection with `lanes` lanes per ray (split.hip): sb slices to a
+// slot of xb.  split_lanes: how many a launch should take, 0 for the whole-ray
+// form.
+int split_lanes(const Geometry &g, int sb);
+hipError_t launch_forward_split(const Geometry &g, const RayInfo *rays, int sb, int lanes,
+                                int mode, bool exact, const float *xb, const float *sino,
+                                float *out, unsigned *maxw, hipStream_t st);
+
 hipError_t launch_backproject(const Geometry &g, const RayInfo *rays, const int *count,
                               const TileShape &ts, int mode, bool exact, const float *w,
                               const unsigned *maxw, float maxlen, float denmax, float *z,
