@@ -221,20 +221,12 @@ int ensure_den(trace_handle *h) {
   return TRACE_OK;
 }
 
-// Slices per thread of the ordered backprojector: up to 32 in the tile form
-// and 8 in the per-pixel form, a divisor of the slice-batched copy's batch
-// for kOrdNum.  A tile is one wavefront, so small images take shallower
-// batches: they walk their rays more often but fill the GPU.  1536 wavefronts
-// are six per compute unit.  PML num, the tables' 16 or 32 slices per thread
-// against the batch chosen here: 21 slices 111 x 111, 708 angles 1460 -> 1233
-// us; 58 slices 94 x 94, 645 angles 1490 -> 1163; 9 slices 201 x 201, 1219
-// angles 2550 -> 2166.
-static int ordered_batch(int mode, int S, int N, int xsb, bool tile) {
+// Slices per workgroup of the ordered backprojector's tile form, up to 32, and
+// per thread of the per-pixel form, up to 8; a divisor of the slice-batched
+// copy's batch for kOrdNum.
+static int ordered_batch(int mode, int S, int xsb, bool tile) {
   int sb = tile ? 32 : 8;
   while (sb > 1 && sb / 2 >= S) sb /= 2;
-  const int64_t tiles = (int64_t)((N + 7) / 8) * ((N + 7) / 8);
-  if (tile)
-    while (sb > 1 && tiles * nbatch(S, sb) < 1536) sb /= 2;
   if (mode == kOrdNum)
     while (sb > 1 && (xsb % sb) != 0) sb /= 2;
   return sb;
@@ -242,21 +234,34 @@ static int ordered_batch(int mode, int S, int N, int xsb, bool tile) {
 
 int ordered_den(trace_handle *h, float *out) {
   if (int rc = ensure_rays(h)) return rc;
-  if (h->ord_tile != 0 && !h->wraps) {
-    unsigned *ovf = reinterpret_cast<unsigned *>(h->flag);
+  unsigned *ovf = reinterpret_cast<unsigned *>(h->flag);
+  auto launch = [&](int form) {
+    return launch_bp_ordered(h->geo, h->rays, kOrdDen, h->exact, nullptr, nullptr, 1, 1, out,
+                             h->wraps, form > 0 ? ovf : nullptr, form == 2, h->stream);
+  };
+  hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+  (void)hipStreamIsCapturing(h->stream, &capture);
+  // decided before; or undecided where nothing can be read back: the form that
+  // always serves
+  if (h->ord_tile >= 0 || capture != hipStreamCaptureStatusNone) {
+    TIMED(TRACE_PHASE_SETUP, launch(h->ord_tile < 0 ? 0 : h->ord_tile));
+    return TRACE_OK;
+  }
+  // the plain tile form, the one for rays on grid lines, the per-pixel form: the
+  // first that has the slots
+  for (int form = h->wraps ? 2 : 1; form <= 2; ++form) {
     HIP_TRY(hipMemsetAsync(ovf, 0, sizeof(unsigned), h->stream));
-    TIMED(TRACE_PHASE_SETUP, launch_bp_ordered(h->geo, h->rays, kOrdDen, h->exact, nullptr,
-                                               nullptr, 1, 1, out, false, ovf, h->stream));
+    TIMED(TRACE_PHASE_SETUP, launch(form));
     unsigned f = 0;
     HIP_TRY(hipMemcpyAsync(&f, ovf, sizeof(f), hipMemcpyDeviceToHost, h->stream));
     HIP_TRY(hipStreamSynchronize(h->stream));
-    h->ord_tile = f ? 0 : 1;
-    if (!f) return TRACE_OK;
-  } else {
-    h->ord_tile = 0;
+    if (!f) {
+      h->ord_tile = form;
+      return TRACE_OK;
+    }
   }
-  TIMED(TRACE_PHASE_SETUP, launch_bp_ordered(h->geo, h->rays, kOrdDen, h->exact, nullptr, nullptr,
-                                             1, 1, out, h->wraps, nullptr, h->stream));
+  h->ord_tile = 0;
+  TIMED(TRACE_PHASE_SETUP, launch(0));
   return TRACE_OK;
 }
 
@@ -265,12 +270,12 @@ int backproject_ordered(trace_handle *h, int mode, const float *w, float *z, int
   if (h->ord_tile < 0)  // decided by the den pass (same walks, same slots)
     if (int rc = ordered_den(h, h->z)) return rc;
   if (mode == kOrdNum && !h->xb) return fail(TRACE_E_INVALID, "no slice-batched image copy");
-  const bool tile = h->ord_tile == 1;
-  const int sb = ordered_batch(mode, h->geo.S, h->geo.N, h->xb_sb, tile);
+  const bool tile = h->ord_tile >= 1;
+  const int sb = ordered_batch(mode, h->geo.S, h->xb_sb, tile);
   // the tile form's overflow flag was checked on this geometry by the den pass
   unsigned *ovf = tile ? reinterpret_cast<unsigned *>(h->flag) : nullptr;
   TIMED(phase, launch_bp_ordered(h->geo, h->rays, mode, h->exact, w, h->xb, h->xb_sb, sb, z,
-                                 h->wraps, ovf, h->stream));
+                                 h->wraps, ovf, h->ord_tile == 2, h->stream));
   return TRACE_OK;
 }
 

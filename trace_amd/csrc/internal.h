@@ -164,12 +164,14 @@ struct BatchQueues {
 // [P][C][S] weights, xb the slice-batched image the ray pass read (xsb
 // slices per slot batch; kOrdNum only), sb slices per thread (a divisor of
 // xsb for kOrdNum; at most 8 in the per-pixel form).  With tile_overflow
-// non-null the tile form runs (geometries without wrapped segments) and
-// ORs a nonzero value into *tile_overflow when a pixel needs more LDS
-// slots than it has; without, the per-pixel form.
+// non-null the tile form runs (with grid_rays the one for geometries with rays
+// on grid lines, wrapped segments among them) and ORs a nonzero value into
+// *tile_overflow when a pixel needs more LDS slots than it has; without, the
+// per-pixel form.
 hipError_t launch_bp_ordered(const Geometry &g, const RayInfo *rays, int mode, bool exact,
                              const float *w, const float *xb, int xsb, int sb, float *out,
-                             bool wraps, unsigned *tile_overflow, hipStream_t st);
+                             bool wraps, unsigned *tile_overflow, bool grid_rays,
+                             hipStream_t st);
 bool ordered_sb_supported(int mode, int sb, int xsb);
 
 // Forward projection with `lanes` lanes per ray (split.hip): sb slices to a

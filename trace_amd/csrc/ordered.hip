@@ -50,7 +50,7 @@
 // modulo 3, and whether the segment before it fell in the same pixel), and
 // its presence is counted without reading the count back.  With the slot
 // from a table of first columns and the number from the count, two LDS round
-// trips a segment, the column sums of 2048^2 / 1500 took @D0 ms instead of @D1.
+// trips a segment, the column sums of 2048^2 / 1500 took 45.3 ms instead of 37.1.
 #include <hip/hip_runtime.h>
 
 #include "internal.h"
@@ -466,6 +466,337 @@ k_bp_ordered_tile(OrdArgs a, unsigned *__restrict__ overflow) {
     if (b * SB + q < a.S) a.out[(int64_t)(b * SB + q) * NN + j] = acc[q];
 }
 
+// LDS of W wavefronts summing SB slices.
+template <int SB, int W, bool kGrid>
+struct OrdSharedLds {
+  static constexpr int kPitch = SB >= 4 ? SB + 4 : SB;  // row pitch of w (bank spread)
+  static constexpr int kDups = kGrid ? 3 : kODups;  // segments per ray and pixel
+  static constexpr int kOwn = kOA * kOSlots * kDups;
+  static constexpr int kTerms = kOwn + (kGrid ? kOA * kDups : 0);  // and wrapped ones
+  static constexpr int kRows = kOA * kORanks + (kGrid ? kOA : 0);
+  float len[W][kTerms][kOWave];            // segment lengths in their slots
+  float w[W][kRows][kPitch];               // weights of the round's rays
+  unsigned cnt[W][kOA][kOWave];            // presence counts and columns (see the kernel)
+  unsigned total[W][kOWave];               // segments of a pixel, per wavefront's projections
+  unsigned short code[W][kTerms][kOWave];  // their places in order: len row | w row << 8
+  unsigned edge[kGrid ? W : 1][kOA][kOT]; // wrapped segments of a row, and 1 << 8 if first
+};
+
+// The tile form for small images: a workgroup of W wavefronts per (tile, slice
+// batch).  With one wavefront a tile, an image of few tiles spends its time in
+// rounds that follow one another, four projections each, and splitting the
+// batch to have more wavefronts repeats the walks.  Here each wavefront files
+// the segments of its own four projections of a round and lists their places in
+// order, then each sums SB / W of the slices over the 4 W projections,
+// ascending.  A large image is served better by one wavefront a tile, which
+// holds less LDS and waits for no other.
+//
+// kGrid: the geometry may have rays on grid lines.  A crossing of such a ray
+// can be computed tens of pixels away, so the ray comes back to pixels it has
+// left, and its segments are numbered by the count so far.  On the right edge
+// line its segments wrap (ix == N) into column 0, whose tiles also take the
+// flagged rays through the strip left of the edge, a column a projection at
+// most, and list a wrapped segment before or after the pixel's own by its
+// column.  Anything else sets the overflow flag, and the per-pixel form is used.
+template <int SB, int W, int MODE, bool kExact, bool kGrid>
+__global__ void __launch_bounds__(kOWave * W)
+k_bp_ordered_shared(OrdArgs a, unsigned *__restrict__ overflow) {
+  static_assert(SB <= kWeightPad, "a slice batch of weights past the last row must be allocated");
+  constexpr int SBW = SB > W ? SB / W : 1;  // slices a wavefront sums
+  using Lds = OrdSharedLds<SB, W, kGrid>;
+  extern __shared__ __align__(16) unsigned char s_raw[];
+  auto &lds = *reinterpret_cast<Lds *>(s_raw);
+  const int N = a.g.N, C = a.g.C;
+  const int tiles_x = (N + kOT - 1) / kOT;
+  const int tile = (int)xcd_chunked(blockIdx.x, gridDim.x);
+  const int tx0 = (tile % tiles_x) * kOT, ty0 = (tile / tiles_x) * kOT;
+  const int tx1 = min(tx0 + kOT, N), ty1 = min(ty0 + kOT, N);
+  const int b = blockIdx.y;
+  const int lane = threadIdx.x % kOWave;
+  const int wv = __builtin_amdgcn_readfirstlane((int)threadIdx.x / kOWave);
+  const int64_t NN = (int64_t)N * N;
+  // the pixel this lane sums, and its first slice
+  const int px = tx0 + (lane % kOT), py = ty0 + (lane / kOT);
+  const bool pix_ok = px < N && py < N && wv * SBW < SB;
+  const int s0 = b * SB + wv * SBW;
+  const float pcx0 = grid_line(N, px), pcx1 = grid_line(N, px + 1);
+  const float pcy0 = grid_line(N, py), pcy1 = grid_line(N, py + 1);
+  float acc[SBW], xv[SBW];
+#pragma unroll
+  for (int q = 0; q < SBW; ++q) acc[q] = 0.f, xv[q] = 0.f;
+  if (MODE == kOrdNum && pix_ok) {
+    const float *src =
+        a.xb + ((int64_t)(s0 / a.xsb) * NN + (int64_t)py * N + px) * a.xsb + s0 % a.xsb;
+#pragma unroll
+    for (int q = 0; q < SBW; ++q) xv[q] = src[q];
+  }
+  // Wait for the pixel's values here, once.  Otherwise the compiler waits
+  // for them where phase 3 first reads them, inside the loop, and its
+  // in-order counter then also waits for the next round's prefetch issued
+  // just before, which serialises every round on that fetch.
+  wait_vector_loads();
+  const float x0 = grid_line(N, tx0), x1 = grid_line(N, tx1);
+  const float y0 = grid_line(N, ty0), y1 = grid_line(N, ty1);
+  const int ai1 = lane / kORanks, k1 = lane % kORanks;  // phase-1 pair of this lane
+  // The angle records of the next round are loaded at the start of a round
+  // (nxt: this wavefront's four projections, for the pixels' columns; fang:
+  // this lane's phase-1 projection, for its pair), so that they have arrived
+  // by the time they are used and their wait never covers the pair prefetch.
+  AngleInfo nxt[kOA], fang;
+  auto load_angles = [&](int p) {
+#pragma unroll
+    for (int ai = 0; ai < kOA; ++ai) nxt[ai] = a.ang[min(p + ai, a.P - 1)];
+    fang = a.ang[min(p + ai1, a.P - 1)];
+  };
+  // The lane's phase-1 pair of a round, fetched one round ahead: its ray
+  // table entry and weights mostly miss L2, so the next round's loads are
+  // issued before this round's sums and arrive while they run.
+  struct Pair {
+    int c, cmin, quadrant;
+    bool ok;
+    RayInfo ray;
+    float w[SB];
+  };
+  // Every lane issues the same loads on every path (row 0 when it has no
+  // pair; a whole slice batch of weights, which the kWeightPad floats after
+  // the weights keep in bounds for the last row): with one path, the
+  // compiler's wait for a load covers that load and the older ones only, so
+  // the prefetch is never waited for before its use.
+  auto fetch = [&](int p, const AngleInfo &ang, Pair &q) {
+    int cmin, cmax;
+    tile_columns(ang, x0, x1, y0, y1, a.yi0, cmin, cmax);
+    q.cmin = cmin;
+    q.quadrant = ang.quadrant;
+    q.c = cmin + k1;
+    q.ok = p < a.P && q.c <= cmax && q.c >= 0 && q.c < C;
+    const int64_t t = q.ok ? (int64_t)p * C + q.c : 0;
+    q.ray = a.rays[t];
+    if (MODE != kOrdDen) {
+      const float *wr = a.w + t * a.S + b * SB;
+      if constexpr (SB % 4 == 0) {
+#pragma unroll
+        for (int i = 0; i < SB; i += 4) {
+          float4 v;
+          __builtin_memcpy(&v, wr + i, sizeof v);  // rows are 4-byte aligned
+          q.w[i] = v.x, q.w[i + 1] = v.y, q.w[i + 2] = v.z, q.w[i + 3] = v.w;
+        }
+      } else {
+#pragma unroll
+        for (int i = 0; i < SB; ++i) q.w[i] = wr[i];
+      }
+    }
+  };
+  Pair cur;
+  // Count words of a round: in the low 24 bits a byte per column slot, with a
+  // nibble per segment number (kGrid: the number of segments); above them the pixel's first candidate column counted from
+  // the tile's (plus one), and that column modulo 3.
+  auto start_counts = [&](int p) {
+#pragma unroll
+    for (int ai = 0; ai < kOA; ++ai) {
+      int c0 = 0, c1;
+      if (p + ai < a.P) tile_columns(nxt[ai], pcx0, pcx1, pcy0, pcy1, a.yi0, c0, c1);
+      const int cmin = __builtin_amdgcn_readlane(cur.cmin, ai * kORanks);
+      lds.cnt[wv][ai][lane] =
+          ((unsigned)(c0 - cmin + 1) << 26) | ((unsigned)column_slot(c0) << 24);
+    }
+    if (kGrid && lane < kOA * kOT) lds.edge[wv][lane / kOT][lane % kOT] = 0;
+  };
+  // Files the wrapped segments of this wavefront's projections: lane (ai1, k1)
+  // takes the k1-th column through the strip.
+  auto file_wrapped = [&](int p0, int p, const AngleInfo &ang) {
+    int emin, emax;
+    tile_columns(ang, grid_line(N, N - 1), grid_line(N, N), grid_line(N, ty0 - 1), y1, a.yi0, emin,
+                 emax);
+    const int c = emin + k1;
+    bool ok = p < a.P && c <= emax && c >= 0 && c < C;
+    const int64_t t = ok ? (int64_t)p * C + c : 0;
+    const RayInfo ray = a.rays[t];
+    ok = ok && (ray.alo & kRayWraps);
+    const uint64_t mine = (__ballot(ok) >> (ai1 * kORanks)) & 0xFFFFu;
+    if (!ok) return;
+    int cmin, cmax;
+    tile_columns(ang, x0, x1, y0, y1, a.yi0, cmin, cmax);
+    if (emax - emin >= kORanks || __popcll(mine) > 1 || (c >= cmin && c <= cmax)) {
+      atomicOr(overflow, 1u);
+      return;
+    }
+    if (MODE != kOrdDen) {
+      const float *wr = a.w + t * a.S + b * SB;
+      float *dst = lds.w[wv][kOA * kORanks + ai1];
+      for (int q = 0; q < SB; ++q) dst[q] = b * SB + q < a.S ? wr[q] : 0.f;
+    }
+    traverse_window<kExact, true>(a.g, ray, ang.quadrant, N - 1, N, ty0 - 1, ty1,
+                                  [&](int ix, int iy, float l, float) {
+      const unsigned ly = (unsigned)(iy + 1 - ty0);
+      if (ix == N && ly < (unsigned)(ty1 - ty0)) {
+        unsigned &n = lds.edge[wv][ai1][ly];
+        const unsigned k = n & 0xFFu;
+        if (k < Lds::kDups) lds.len[wv][Lds::kOwn + ai1 * Lds::kDups + k][ly * kOT] = l;
+        n = (n + 1) | (c < cmin ? 0x100u : 0u);
+      }
+    });
+  };
+  constexpr int kRound = kOA * W;  // projections per round
+  AngleInfo fcur;  // this round's fang
+  load_angles(wv * kOA);
+  fcur = fang;
+  fetch(wv * kOA + ai1, fang, cur);
+  start_counts(wv * kOA);
+  for (int r0 = 0; r0 < a.P; r0 += kRound) {
+    const int p0 = r0 + wv * kOA;  // this wavefront's first projection
+    if (kGrid) fcur = fang;
+    load_angles(p0 + kRound);
+    // phase 1: walk the pairs, file each segment of the tile in its slot
+    const int p = p0 + ai1;
+    if (p < a.P && cur.ok) {
+      const int c = cur.c;
+      if (MODE != kOrdDen) {
+        // slots past the stack's last slice (read from the next row) add 0
+        float *dst = lds.w[wv][lane];
+#pragma unroll
+        for (int q = 0; q < SB; ++q) dst[q] = b * SB + q < a.S ? cur.w[q] : 0.f;
+      }
+      const int slot = column_slot(c);
+      float *len0 = lds.len[wv][(ai1 * kOSlots + slot) * Lds::kDups];
+      const unsigned one0 = 1u << (8 * slot);
+      int last = -1, again = 0;  // the pixel filed last, and its segment number
+      traverse_window<kExact, true>(a.g, cur.ray, cur.quadrant, tx0, tx1, ty0, ty1,
+                                    [&](int ix, int iy, float l, float) {
+        const unsigned lx = (unsigned)(ix - tx0), ly = (unsigned)(iy - ty0);
+        if (lx < (unsigned)(tx1 - tx0) && ly < (unsigned)(ty1 - ty0)) {
+          const int lp = (int)(ly * kOT + lx);
+          unsigned *cnt = &lds.cnt[wv][ai1][lp];
+          if constexpr (kGrid) {
+            // only this lane counts in its slot's byte
+            const int k = (int)((*cnt >> (8 * slot)) & 0xFFu);
+            if (k < Lds::kDups) len0[k * kOWave + lp] = l;
+            if (k <= Lds::kDups) atomicAdd(cnt, one0);
+          } else {
+            // a third segment (or a return to a pixel left) counts past 1 in
+            // its nibble, which phase 2 reports
+            again = lp == last ? 1 : 0;
+            last = lp;
+            len0[again * kOWave + lp] = l;
+            atomicAdd(cnt, again ? one0 << 4 : one0);
+          }
+        }
+      });
+    }
+    if (kGrid && tx0 == 0) file_wrapped(p0, p, fcur);
+    // Phase 2: each lane lists the places of its pixel's segments of this
+    // wavefront's projections in order, (projection, column, segment)
+    // ascending.  Only this wavefront has filed there, and its LDS accesses
+    // take effect in the order they are issued.
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    {
+      unsigned short *dst = &lds.code[wv][0][lane];
+      int n = 0;
+#pragma unroll
+      for (int ai = 0; ai < kOA; ++ai) {
+        const unsigned word = lds.cnt[wv][ai][lane];
+        if (!kGrid && (word & 0x00EEEEEEu)) atomicOr(overflow, 1u);
+        unsigned wrapped = 0;
+        if (kGrid && lane % kOT == 0) wrapped = lds.edge[wv][ai][lane / kOT];
+        if ((wrapped & 0xFFu) > Lds::kDups) atomicOr(overflow, 1u);
+        auto list_wrapped = [&]() {
+          for (unsigned k = 0; k < (wrapped & 0xFFu) && k < Lds::kDups; ++k) {
+            *dst = (unsigned short)((Lds::kOwn + ai * Lds::kDups + k) |
+                                    ((kOA * kORanks + ai) << 8));
+            dst += kOWave, ++n;
+          }
+        };
+        if (kGrid && (wrapped & 0x100u)) list_wrapped();
+        unsigned at = (word >> 24) & 3u;            // slot of the candidate column
+        unsigned row = ai * kORanks + (word >> 26) - 1;  // and its pair
+#pragma unroll
+        for (int k = 0; k < kOSlots; ++k) {
+          const unsigned has = word >> (8 * at);
+          const unsigned code = (ai * kOSlots + at) * Lds::kDups | (row << 8);
+          if constexpr (kGrid) {
+            const unsigned m = has & 0xFFu;
+            if (m > Lds::kDups) atomicOr(overflow, 1u);
+            for (unsigned d = 0; d < m && d < Lds::kDups; ++d) {
+              *dst = (unsigned short)(code + d);
+              dst += kOWave, ++n;
+            }
+          } else {
+            if (has & 0x01u) {
+              *dst = (unsigned short)code;
+              dst += kOWave, ++n;
+            }
+            if (has & 0x10u) {
+              *dst = (unsigned short)(code + 1);
+              dst += kOWave, ++n;
+            }
+          }
+          at = at == kOSlots - 1 ? 0 : at + 1;
+          ++row;
+        }
+        if (kGrid && wrapped && !(wrapped & 0x100u)) list_wrapped();
+      }
+      lds.total[wv][lane] = n;
+    }
+    __syncthreads();
+    fetch(p0 + kRound + ai1, fang, cur);  // next round's pair, in flight during phase 3
+    // phase 3: each lane adds its pixel's segments, the wavefronts' projections
+    // in turn; as many iterations as the busiest pixel has segments
+    if (pix_ok) {
+      for (int g = 0; g < W; ++g) {
+        const int n = (int)lds.total[g][lane];
+        const unsigned short *src = &lds.code[g][0][lane];
+        const float *len = &lds.len[g][0][lane];
+        const float *wg = &lds.w[g][0][MODE == kOrdDen ? 0 : wv * SBW];
+        for (int k = 0; k < n; ++k) {
+          const unsigned code = *src;
+          src += kOWave;
+          const float l = len[(code & 0xFFu) * kOWave];
+          if (MODE == kOrdDen) {
+            acc[0] = acc[0] + l;
+          } else {
+            const float *wr = wg + (code >> 8) * Lds::kPitch;
+#pragma unroll
+            for (int q = 0; q < SBW; ++q) {
+              if (MODE == kOrdEM)
+                acc[q] = acc[q] + l * wr[q];
+              else
+                acc[q] = acc[q] - (xv[q] * l) * wr[q];
+            }
+          }
+        }
+      }
+    }
+    __syncthreads();
+    start_counts(p0 + kRound);
+  }
+  if (!pix_ok) return;
+  const int64_t j = (int64_t)py * N + px;
+  if (MODE == kOrdDen) {
+    a.out[j] = acc[0];
+    return;
+  }
+#pragma unroll
+  for (int q = 0; q < SBW; ++q)
+    if (s0 + q < a.S) a.out[(int64_t)(s0 + q) * NN + j] = acc[q];
+}
+
+template <int SB, int W, int MODE, bool kGrid>
+hipError_t ord_shared_launch(const OrdArgs &a, bool exact, unsigned *overflow, hipStream_t st) {
+  const int N = a.g.N;
+  const int tiles = ((N + kOT - 1) / kOT) * ((N + kOT - 1) / kOT);
+  const int nb = MODE == kOrdDen ? 1 : (a.S + SB - 1) / SB;
+  constexpr size_t lds = sizeof(OrdSharedLds<SB, W, kGrid>);
+  static_assert(lds <= 160 * 1024, "a workgroup's LDS");
+  auto kern = exact ? k_bp_ordered_shared<SB, W, MODE, true, kGrid>
+                    : k_bp_ordered_shared<SB, W, MODE, false, kGrid>;
+  if (lds > 65536) {
+    const hipError_t e = hipFuncSetAttribute(
+        (const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    if (e != hipSuccess) return e;
+  }
+  hipLaunchKernelGGL(kern, dim3(tiles, nb), dim3(kOWave * W), lds, st, a, overflow);
+  return hipGetLastError();
+}
+
 template <int SB, int MODE>
 hipError_t ord_tile_launch(const OrdArgs &a, bool exact, unsigned *overflow, hipStream_t st) {
   const int N = a.g.N;
@@ -482,6 +813,22 @@ hipError_t ord_tile_launch(const OrdArgs &a, bool exact, unsigned *overflow, hip
 
 }  // namespace
 
+// Wavefronts per tile: more where the tiles alone leave the GPU's SIMDs idle.
+// One launch with 1 / 4 / 8, PML num (us):
+//    59^2,  700 angles   1 slice 967 / 344 /  237   32 slices 1344 /  445 /  340
+//   151^2,  400                  590 / 213 /  269              792 /  279 /  377
+//   300^2,  300                  471 / 345 /  589              686 /  610 /  802
+//   400^2,  300                  547 / 622 /  997             1220 / 1005 / 1358
+//   511^2,  200                  498 / 639 / 1110              916 / 1102 / 1487
+// Geometries with rays on grid lines always share (129^2, 110 angles, 11 slices:
+// 175 us, 745 in the per-pixel form; den of 125^2, 122 angles 94, per pixel 2131).
+int ordered_waves(int N, int S, int sb, bool grid_rays) {
+  const int64_t tiles =
+      (int64_t)((N + kOT - 1) / kOT) * ((N + kOT - 1) / kOT) * ((S + sb - 1) / sb);
+  if (grid_rays) return 4;
+  return tiles <= 128 ? 8 : (tiles <= (sb == 32 ? 3000 : 1536) ? 4 : 1);
+}
+
 bool ordered_sb_supported(int mode, int sb, int xsb) {
   if (mode == kOrdDen) return true;
   if (sb != 1 && sb != 2 && sb != 4 && sb != 8 && sb != 16 && sb != 32) return false;
@@ -490,7 +837,8 @@ bool ordered_sb_supported(int mode, int sb, int xsb) {
 
 hipError_t launch_bp_ordered(const Geometry &g, const RayInfo *rays, int mode, bool exact,
                              const float *w, const float *xb, int xsb, int sb, float *out,
-                             bool wraps, unsigned *tile_overflow, hipStream_t st) {
+                             bool wraps, unsigned *tile_overflow, bool grid_rays,
+                             hipStream_t st) {
   OrdArgs a;
   a.g = g.grid;
   a.ang = g.d_ang;
@@ -505,8 +853,27 @@ hipError_t launch_bp_ordered(const Geometry &g, const RayInfo *rays, int mode, b
   a.wraps = wraps ? 1 : 0;
   if (!ordered_sb_supported(mode, sb, xsb)) return hipErrorInvalidValue;
   if (tile_overflow) {
-    // tile form (no wrapped segments)
-    if (wraps) return hipErrorInvalidValue;
+    // tile form; wrapped segments need the grid-ray one
+    if (wraps && !grid_rays) return hipErrorInvalidValue;
+    const int waves = ordered_waves(g.N, mode == kOrdDen ? 1 : g.S, sb, grid_rays);
+#define TRACE_ORDS_CASE(SB_, W_, GRID_)                                                     \
+  if (waves == W_ && grid_rays == GRID_) {                                                      \
+    if (mode == kOrdDen)                                                                     \
+      return ord_shared_launch<1, W_, kOrdDen, GRID_>(a, exact, tile_overflow, st);         \
+    if (sb == SB_)                                                                           \
+      return mode == kOrdNum                                                                 \
+                 ? ord_shared_launch<SB_, W_, kOrdNum, GRID_>(a, exact, tile_overflow, st)  \
+                 : ord_shared_launch<SB_, W_, kOrdEM, GRID_>(a, exact, tile_overflow, st);  \
+  }
+#define TRACE_ORDS_WAVES(W_, GRID_)                                                         \
+  TRACE_ORDS_CASE(1, W_, GRID_) TRACE_ORDS_CASE(2, W_, GRID_) TRACE_ORDS_CASE(4, W_, GRID_) \
+  TRACE_ORDS_CASE(8, W_, GRID_) TRACE_ORDS_CASE(16, W_, GRID_) TRACE_ORDS_CASE(32, W_, GRID_)
+    TRACE_ORDS_WAVES(4, false)
+    TRACE_ORDS_WAVES(8, false)
+    TRACE_ORDS_WAVES(4, true)
+#undef TRACE_ORDS_WAVES
+#undef TRACE_ORDS_CASE
+    if (grid_rays) return hipErrorInvalidValue;
     if (mode == kOrdDen) return ord_tile_launch<1, kOrdDen>(a, exact, tile_overflow, st);
 #define TRACE_ORDT_CASE(SB_)                                                               \
   case SB_:                                                                                \
