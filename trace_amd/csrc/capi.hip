@@ -102,11 +102,8 @@ static void free_staged(trace_handle *h) {
 int ensure_rays(trace_handle *h) {
   if (h->rays_ready) return TRACE_OK;
   if (!h->rays) HIP_TRY(dev_alloc(&h->rays, (size_t)h->geo.rays_per_slice()));
-  TIMED(TRACE_PHASE_SETUP, launch_ray_info(h->geo, h->rays, h->stream));
   HIP_TRY(hipMemsetAsync(h->counters, 0, 4 * sizeof(unsigned long long), h->stream));
-  TIMED(TRACE_PHASE_SETUP, launch_count_segments(h->geo, h->rays, h->counters, h->counters + 1,
-                                                 reinterpret_cast<unsigned *>(h->counters + 2),
-                                                 h->counters + 3, h->stream));
+  TIMED(TRACE_PHASE_SETUP, launch_ray_info(h->geo, h->rays, h->counters, h->stream));
   unsigned long long c[4] = {0, 0, 0, 0};
   HIP_TRY(hipMemcpyAsync(c, h->counters, sizeof(c), hipMemcpyDeviceToHost, h->stream));
   HIP_TRY(hipStreamSynchronize(h->stream));
@@ -865,7 +862,7 @@ int trace_forward_noalloc(trace_handle_t *h, const float *x, float *y) {
   RayInfo *rays = static_cast<RayInfo *>(base);
   float *xb = reinterpret_cast<float *>(static_cast<unsigned char *>(base) + rays_b);
   // every scratch byte read below is written first on the same stream
-  HIP_TRY(launch_ray_info(g, rays, h->stream, false));
+  HIP_TRY(launch_ray_info(g, rays, nullptr, h->stream));
   HIP_TRY(launch_pack(x, g.S, 0, 0.f, g.NN(), nbatch(g.S, sb) * sb, sb, xb, h->stream));
   HIP_TRY(launch_forward(g, rays, sb, h->fwd_bundle, forward_lanes(h, sb), kFwdOutY, h->exact,
                          xb, nullptr, y, nullptr, h->stream));

@@ -101,7 +101,8 @@ int tile_count_bound(float sinq, float cosq, int TW, int TH);
 // Ray table; `flags` adds the window flags (kRayWhole, kRayWraps, kRay1D)
 // from one walk per ray, which the tile kernels need and whole-ray walks
 // do not.
-hipError_t launch_ray_info(const Geometry &g, RayInfo *rays, hipStream_t st, bool flags = true);
+hipError_t launch_ray_info(const Geometry &g, RayInfo *rays, unsigned long long *counts,
+                           hipStream_t st);
 hipError_t launch_forward(const Geometry &g, const RayInfo *rays, int sb, int bundle_angles,
                           int lanes_per_ray, int mode, bool exact, const float *xb,
                           const float *sino, float *out, unsigned *maxw, hipStream_t st);
@@ -224,9 +225,6 @@ hipError_t launch_dump_rays(const Geometry &g, const RayInfo *rays, int n, const
                             float *len2, hipStream_t st, bool exact);
 hipError_t launch_ray_sums(const Geometry &g, const RayInfo *rays, bool exact, float *len_sum,
                            float *len2_sum, hipStream_t st);
-hipError_t launch_count_segments(const Geometry &g, const RayInfo *rays,
-                                 unsigned long long *total, unsigned long long *oor,
-                                 unsigned *maxlen, unsigned long long *wraps, hipStream_t st);
 hipError_t launch_check_finite(const float *v, int64_t n, int *flag, hipStream_t st);
 
 }  // namespace trace_hip

@@ -47,17 +47,51 @@ __device__ __forceinline__ void atomic_add_f32(float *p, float v) {
 
 // ---------------------------------------------------------------- rays --
 
+// Ray table.  With `counts` also the rays' flags and the geometry's segment
+// statistics, from one walk of each ray: all segments, those outside the image,
+// the bits of the longest, and the rays with a wrapped one (zeroed beforehand).
+// Whole-ray walks (the forward projector) read neither.
 __global__ void __launch_bounds__(kRayBlock)
 k_ray_info(GridInfo g, const AngleInfo *__restrict__ ang, const float *__restrict__ yi,
-           int P, int flags, RayInfo *__restrict__ rays) {
+           int P, unsigned long long *__restrict__ counts, RayInfo *__restrict__ rays) {
   const int64_t t = (int64_t)blockIdx.x * kRayBlock + threadIdx.x;
-  if (t >= (int64_t)P * g.C) return;
-  const int c = (int)(t % g.C), p = (int)(t / g.C);
-  RayInfo r = make_ray(g, yi[c], ang[p].sinq, ang[p].cosq);
-  // the flags walk each ray once; whole-ray walks (the forward projector)
-  // do not read them
-  if (flags) r.alo |= ray_flags(g, r, ang[p].quadrant);
-  rays[t] = r;
+  const bool valid = t < (int64_t)P * g.C;
+  RayStats st;
+  unsigned wraps = 0;
+  if (valid) {
+    const int c = (int)(t % g.C), p = (int)(t / g.C);
+    RayInfo r = make_ray(g, yi[c], ang[p].sinq, ang[p].cosq);
+    if (counts) {
+      r.alo |= ray_flags(g, r, ang[p].quadrant, st);
+      wraps = (r.alo & kRayWraps) ? 1u : 0u;
+    }
+    rays[t] = r;
+  }
+  if (!counts) return;
+  __shared__ unsigned s_sum[3], s_longest;
+  if (threadIdx.x < 3) s_sum[threadIdx.x] = 0;
+  if (threadIdx.x == 3) s_longest = 0;
+  __syncthreads();
+  unsigned lb = __float_as_uint(st.longest);
+  for (int off = 32; off > 0; off >>= 1) {
+    st.segments += __shfl_down(st.segments, off, 64);
+    st.outside += __shfl_down(st.outside, off, 64);
+    wraps += __shfl_down(wraps, off, 64);
+    lb = max(lb, (unsigned)__shfl_down((int)lb, off, 64));
+  }
+  if ((threadIdx.x & 63) == 0) {
+    atomicAdd(s_sum + 0, st.segments);
+    atomicAdd(s_sum + 1, st.outside);
+    atomicAdd(s_sum + 2, wraps);
+    atomicMax(&s_longest, lb);
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    atomicAdd(counts + 0, (unsigned long long)s_sum[0]);
+    if (s_sum[1]) atomicAdd(counts + 1, (unsigned long long)s_sum[1]);
+    raise_max(reinterpret_cast<unsigned *>(counts + 2), s_longest);
+    if (s_sum[2]) atomicAdd(counts + 3, (unsigned long long)s_sum[2]);
+  }
 }
 
 // ------------------------------------------------------------- forward --
@@ -1359,42 +1393,6 @@ k_ray_sums(GridInfo g, const AngleInfo *__restrict__ ang, const RayInfo *__restr
   if (len2_sum) len2_sum[t] = a2;
 }
 
-// Segment statistics of one slice: total count, count outside the image,
-// and the bits of the longest segment under either length rounding.
-__global__ void __launch_bounds__(kRayBlock)
-k_count_segments(GridInfo g, const AngleInfo *__restrict__ ang,
-                 const RayInfo *__restrict__ rays, int P,
-                 unsigned long long *total, unsigned long long *oor, unsigned *maxlen,
-                 unsigned long long *wraps) {
-  const int64_t t = (int64_t)blockIdx.x * kRayBlock + threadIdx.x;
-  const int C = g.C;
-  unsigned cnt = 0, bad = 0, wr = 0;
-  float lmax = 0.f;
-  if (t < (int64_t)P * C) {
-    const int p = (int)(t / C);
-    const unsigned NN = (unsigned)g.N * (unsigned)g.N;
-    const RayInfo r = rays[t];
-    wr = (r.alo & kRayWraps) ? 1u : 0u;
-    cnt = traverse_full<true>(g, r, ang[p].quadrant, [&](int ix, int iy, float l, float l2) {
-      bad += ((unsigned)(ix + iy * g.N) >= NN) ? 1u : 0u;
-      lmax = fmaxf(lmax, fmaxf(l, __builtin_amdgcn_sqrtf(l2)));
-    });
-  }
-  unsigned lb = __float_as_uint(lmax);
-  for (int off = 32; off > 0; off >>= 1) {
-    cnt += __shfl_down(cnt, off, 64);
-    bad += __shfl_down(bad, off, 64);
-    wr += __shfl_down(wr, off, 64);
-    lb = max(lb, (unsigned)__shfl_down((int)lb, off, 64));
-  }
-  if ((threadIdx.x & 63) == 0) {
-    atomicAdd(total, (unsigned long long)cnt);
-    if (bad) atomicAdd(oor, (unsigned long long)bad);
-    if (wr && wraps) atomicAdd(wraps, (unsigned long long)wr);
-    atomicMax(maxlen, lb);
-  }
-}
-
 __global__ void k_check_finite(const float *__restrict__ v, int64_t n,
                                int *__restrict__ flag) {
   int64_t i = (int64_t)blockIdx.x * kPixBlock + threadIdx.x;
@@ -1519,10 +1517,11 @@ int tile_count_bound(float sinq, float cosq, int TW, int TH) {
   return (int)std::floor(len) + 1;
 }
 
-hipError_t launch_ray_info(const Geometry &g, RayInfo *rays, hipStream_t st, bool flags) {
+hipError_t launch_ray_info(const Geometry &g, RayInfo *rays, unsigned long long *counts,
+                           hipStream_t st) {
   const int64_t n = g.rays_per_slice();
   hipLaunchKernelGGL(k_ray_info, dim3(blocks_for(n, kRayBlock)), dim3(kRayBlock), 0, st,
-                     g.grid, g.d_ang, g.d_yi, g.P, flags ? 1 : 0, rays);
+                     g.grid, g.d_ang, g.d_yi, g.P, counts, rays);
   return hipGetLastError();
 }
 
@@ -1776,15 +1775,6 @@ hipError_t launch_ray_sums(const Geometry &g, const RayInfo *rays, bool exact, f
   else
     hipLaunchKernelGGL(k_ray_sums<false>, dim3(blocks_for(n, kRayBlock)), dim3(kRayBlock), 0, st,
                        g.grid, g.d_ang, rays, g.P, len_sum, len2_sum);
-  return hipGetLastError();
-}
-
-hipError_t launch_count_segments(const Geometry &g, const RayInfo *rays,
-                                 unsigned long long *total, unsigned long long *oor,
-                                 unsigned *maxlen, unsigned long long *wraps, hipStream_t st) {
-  const int64_t n = g.rays_per_slice();
-  hipLaunchKernelGGL(k_count_segments, dim3(blocks_for(n, kRayBlock)), dim3(kRayBlock), 0, st,
-                     g.grid, g.d_ang, rays, g.P, total, oor, maxlen, wraps);
   return hipGetLastError();
 }
 

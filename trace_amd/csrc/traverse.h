@@ -402,14 +402,22 @@ struct AxisCheck {
 // kRay1D: the same check fails on the second axis (columns for |islope| <=
 // 1, rows otherwise), so the ray's windows must not be intersected with a
 // window on that axis.
-__device__ __forceinline__ int ray_flags(const GridInfo &g, const RayInfo &r, int quadrant) {
+//
+// `stats` takes the ray's segments from the same walk.
+struct RayStats {
+  unsigned segments = 0, outside = 0;  // all of them, and those not in the image
+  float longest = 0.f;                 // under either rounding of the lengths
+};
+__device__ __forceinline__ int ray_flags(const GridInfo &g, const RayInfo &r, int quadrant,
+                                         RayStats &stats) {
   Walker w;
   w.init(r, g.N, quadrant);
   const bool sorted = w.a_sorted();  // unsorted rays are walked whole in any case
   w.seek(0, 0);
   const bool on_a = __builtin_fabsf(r.islope) <= 1.0f;
   AxisCheck prim(on_a), sec(!on_a);
-  bool wraps = false, hits = false;
+  bool wraps = false;
+  const unsigned NN = (unsigned)g.N * (unsigned)g.N;
   float px = 0.f, py = 0.f;
   const int n = w.alen + w.blen;
   for (int k = 0; k < n; ++k) {
@@ -417,16 +425,20 @@ __device__ __forceinline__ int ray_flags(const GridInfo &g, const RayInfo &r, in
     float qx, qy;
     w.next(qx, qy);
     if (k > 0) {
-      const int ix = (int)__builtin_fmaf(qx + px, 0.5f, g.mg);  // as segment()
-      const int iy = (int)__builtin_fmaf(qy + py, 0.5f, g.mg);
+      int ix, iy;
+      float l, l2;
+      segment<true>(px, py, qx, qy, g.mg, ix, iy, l, l2);
       wraps |= (ix == g.N);
-      hits |= (unsigned)(ix + iy * g.N) < (unsigned)g.N * (unsigned)g.N;
+      stats.outside += (unsigned)(ix + iy * g.N) >= NN ? 1u : 0u;
+      stats.longest = fmaxf(stats.longest, fmaxf(l, __builtin_amdgcn_sqrtf(l2)));
     }
     px = qx;
     py = qy;
     prim.point(takeA, qx, qy);
     sec.point(takeA, qx, qy);
   }
+  stats.segments = n < 2 ? 0u : (unsigned)(n - 1);
+  const bool hits = stats.outside < stats.segments;
   const bool whole = sorted && !prim.done(n);
   const bool one_axis = !sec.done(n);
   return (whole ? kRayWhole : 0) | (wraps ? kRayWraps : 0) | (one_axis ? kRay1D : 0) |
