@@ -59,21 +59,9 @@ int fail(int code, const std::string &msg) {
 
 int nbatch(int S, int sb) { return (S + sb - 1) / sb; }
 
-// Angle groups of the handle's slice batch (host only, once per batch).
-static const StagedLayout &layout_of(trace_handle *h) {
-  if (h->layout_sb != h->fwd_sb) {
-    h->layout = staged_layout(h->geo, h->ang.data(), h->fwd_sb);
-    h->layout_faster = staged_faster(h->geo, h->layout, h->fwd_sb);
-    h->layout_sb = h->fwd_sb;
-  }
-  return h->layout;
-}
-
 bool forward_staged(trace_handle *h) {
   if (h->fwd_staged == 0 || !staged_batch(h->fwd_sb)) return false;
-  if (h->fwd_staged == 1) return true;
-  (void)layout_of(h);
-  return h->layout_faster;
+  return h->fwd_staged == 1 || staged_faster(h->geo, h->fwd_sb);
 }
 
 int forward_batch(trace_handle *h) {
@@ -123,7 +111,7 @@ int ensure_staged(trace_handle *h) {
   if (pl.sb == sb) return TRACE_OK;
   if (int rc = ensure_rays(h)) return rc;
   const Geometry &g = h->geo;
-  const StagedLayout &lay = layout_of(h);
+  const StagedLayout lay = staged_layout(g, h->ang.data(), sb);
   free_staged(h);
   pl.H = lay.H;
   pl.ngroups = (int)lay.group.size();

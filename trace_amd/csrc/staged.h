@@ -41,8 +41,8 @@ struct StagedLayout {
   std::vector<int4> group;
 };
 StagedLayout staged_layout(const Geometry &g, const AngleInfo *ang, int sb);
-// Whether the staged form is the faster one for a geometry and its layout.
-bool staged_faster(const Geometry &g, const StagedLayout &lay, int sb);
+// Whether the staged form is the fastest one for a geometry at slice batch sb.
+bool staged_faster(const Geometry &g, int sb);
 
 hipError_t launch_staged_plan(const Geometry &g, const RayInfo *rays, StagedPlan &pl,
                               hipStream_t st);

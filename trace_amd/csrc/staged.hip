@@ -474,28 +474,26 @@ StagedLayout staged_layout(const Geometry &g, const AngleInfo *ang, int sb) {
   return best;
 }
 
-// Estimated times of one projection by the two forms, from launches of one
-// batch on uniform angles (us; sb 4 / 8 / 16 / 32, staged against whole):
-//   2048^2, 1500 angles   9011 / 10127 / 17371 / 24494   12422 / 19763 / 33321 / 50221
-//   1024^2,  720          1370 /  1518 /  2426 /  3532    1694 /  2347 /  3935 /  5558
-//   1024^2,  180           702 /   721 /   921 /  1523     785 /   860 /  1354 /  2275
-//    640^2,  480           606 /   682 /   893 /  1231     439 /   639 /  1072 /  1402
-//    512^2,  360           364 /   409 /   512 /   687     266 /   345 /   575 /   688
-//    300^2,  181           204 /   228 /   288 /   342      80 /    88 /   123 /   160
-// A staged launch takes a sweep per bundle in flight (bundles fill the 256
-// CUs in rounds; one alone waits for its slabs), a whole-ray launch its
-// segments' gathers and the longest ray's latency.
-bool staged_faster(const Geometry &g, const StagedLayout &lay, int sb) {
-  const int i = sb == 4 ? 0 : (sb == 8 ? 1 : (sb == 16 ? 2 : 3));
-  static const double sweep[] = {0.51, 0.64, 0.75, 0.98};   // us per pixel of the sweep
-  static const double round[] = {0.33, 0.37, 0.63, 0.90};   // and per round of bundles
-  static const double gather[] = {1.9, 2.6, 5.5, 8.0};      // 1e-6 us per segment
-  const int nb = (g.S + sb - 1) / sb;
-  const double bundles = (double)lay.group.size() * ((g.C + kStW - 1) / kStW) * nb;
-  const double staged = g.N * (sweep[i] + round[i] * bundles / 256);
-  const double segments = 1.2 * g.N * std::min(g.N, g.C) * (double)g.P;
-  const double whole = nb * segments * gather[i] * 1e-6 + 0.1 * g.N;
-  return staged < whole;
+// A staged launch sweeps every bundle through the image however few its rays
+// are, which takes 0.5 to 1 us a pixel of the side; the other forms take their
+// segments' gathers, which cost the more the further the image outgrows the
+// caches and the fewer the angles whose rays could share lines.  Over 185
+// geometries, N from 128 to 2048 and 30 to 1500 uniform angles, the side to the
+// power 1.5 times the angles told the faster form, or one within 1% on average
+// (between 1 and 2 the power matters little).  Staged against the better of the
+// others (us):
+//               4 slices      8 slices     16 slices      32 slices
+//   256^2, 1500    237 / 258     270 / 241     392 / 444     539 / 564
+//   600^2,  250    427 / 258     469 / 345     589 / 572    1020 / 684
+//   600^2, 1000    765 / 719     848 / 797    1363 / 1532   1922 / 2186
+//   900^2,  250    634 / 700     889 / 879     905 / 1319   1559 / 1833
+//  1300^2,   60   1012 / 385     906 / 612    1241 / 957    2136 / 1988
+//  1300^2,  250   1137 / 1493   1193 / 1982   2203 / 2892   3441 / 5599
+//  2048^2,  130   1753 / 2709   2136 / 3059   3996 / 4937   7017 / 11913
+//  2048^2, 1000   6299 / 9849   7084 / 15412
+bool staged_faster(const Geometry &g, int sb) {
+  const double side = std::min(g.N, g.C);
+  return side * std::sqrt(side) * g.P >= (sb <= 8 ? 8e6 : (sb == 16 ? 2.8e6 : 4.2e6));
 }
 
 hipError_t launch_staged_plan(const Geometry &g, const RayInfo *rays, StagedPlan &pl,
