@@ -157,7 +157,7 @@ struct BatchQueues {
   X(32, 32, 1) X(64, 64, 1) X(32, 32, 2) X(16, 16, 2) X(16, 16, 1)          \
   X(16, 16, 32) X(32, 32, 16) X(32, 16, 16) X(24, 24, 16)
 
-// (slot batch, slices per thread) of the regularised updates.
+// (slot batch, slices per thread) of the image updates.
 #define TRACE_UPDATE_SHAPES(X)                                             \
   X(1, 1) X(2, 2) X(4, 4) X(8, 8) X(16, 16) X(32, 32) X(8, 4) X(16, 4) X(32, 4)
 

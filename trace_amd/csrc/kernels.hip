@@ -935,22 +935,22 @@ __device__ __forceinline__ void clear_max(unsigned *maxw, int S) {
     for (int s = threadIdx.x; s < S; s += kPixBlock) maxw[s] = 0;
 }
 
-// SIRT (sirt.cc:21-33) / MLEM (mlem.cc:21-34) update of a batch of slices
+// SIRT (sirt.cc:21-33) / MLEM (mlem.cc:21-34) update of VB slices of a batch
 // at pixel j, also refreshing the batched copy (with one slice to a batch x
 // is that copy).
-template <int SB, bool kSIRT>
+template <int SB, int VB, bool kSIRT>
 __global__ void __launch_bounds__(kPixBlock)
 k_update_em(float *__restrict__ x, const float *__restrict__ z, const float *__restrict__ den,
             int S, int64_t NN, float *__restrict__ xb, unsigned *__restrict__ maxw) {
   const int64_t j = (int64_t)blockIdx.x * kPixBlock + threadIdx.x;
-  const int b = blockIdx.y;
+  const int s0 = blockIdx.y * VB;
   clear_max(maxw, S);
   if (j >= NN) return;
   const float d = den[j];
-  float v[SB];
+  float v[VB];
 #pragma unroll
-  for (int q = 0; q < SB; ++q) {
-    const int s = b * SB + q;
+  for (int q = 0; q < VB; ++q) {
+    const int s = s0 + q;
     v[q] = 0.f;
     if (s < S) {
       const int64_t o = (int64_t)s * NN + j;
@@ -961,7 +961,7 @@ k_update_em(float *__restrict__ x, const float *__restrict__ z, const float *__r
       v[q] = xv;
     }
   }
-  if (SB > 1) store_slices<SB>(xb + ((int64_t)b * NN + j) * SB, v);
+  if (SB > 1) store_slices<VB>(xb + ((int64_t)(s0 / SB) * NN + j) * SB + s0 % SB, v);
 }
 
 __global__ void k_fill(float *__restrict__ p, int64_t n, float v) {
@@ -1582,30 +1582,35 @@ hipError_t launch_pack(const float *src, int nsrc, int off, float fill, int64_t 
   return hipGetLastError();
 }
 
+// Slices per thread of the updates: the slot batch, or 4 of it where that
+// leaves too few workgroups, since a thread takes its slices one after the other
+// (APMLR some 10 divisions and a square root each: below 2048 workgroups, SIRT
+// and MLEM one division: below 512).  All / 4 slices (us): APMLR 14 slices 82^2
+// 58 / 18, 9 slices 511^2 59 / 39; PML 20 slices 151^2 45 / 14; SIRT 33 slices
+// 125^2 15 / 7; MLEM 7 slices 548^2 8 / 10.  Where the wavefronts are there
+// anyway whole lines of the copy are written.
+static bool update_split(int64_t NN, int sb, int slots, int blocks) {
+  return sb > 4 && (int64_t)blocks_for(NN, kPixBlock) * ((slots + sb - 1) / sb) < blocks;
+}
+
 hipError_t launch_update_em(bool sirt, float *x, const float *z, const float *den, int S,
                             int64_t NN, int sb, float *xb, unsigned *maxw, hipStream_t st) {
-  const int nb = (S + sb - 1) / sb;
-  dim3 grid(blocks_for(NN, kPixBlock), nb), block(kPixBlock);
-#define TRACE_UPD_CASE(SB_)                                                                   \
-  case SB_:                                                                                   \
-    if (sirt)                                                                                 \
-      hipLaunchKernelGGL((k_update_em<SB_, true>), grid, block, 0, st, x, z, den, S, NN, xb, \
-                         maxw);                                                               \
-    else                                                                                      \
-      hipLaunchKernelGGL((k_update_em<SB_, false>), grid, block, 0, st, x, z, den, S, NN, xb, \
-                         maxw);                                                               \
-    break;
-  switch (sb) {
-    TRACE_UPD_CASE(1)
-    TRACE_UPD_CASE(2)
-    TRACE_UPD_CASE(4)
-    TRACE_UPD_CASE(8)
-    TRACE_UPD_CASE(16)
-    TRACE_UPD_CASE(32)
-    default: return hipErrorInvalidValue;
+  const int nslots = (S + sb - 1) / sb * sb;
+  const int vb = update_split(NN, sb, nslots, 512) ? 4 : sb;
+  const dim3 grid(blocks_for(NN, kPixBlock), nslots / vb), block(kPixBlock);
+#define TRACE_UPD_CASE(SB_, VB_)                                                            \
+  if (sb == SB_ && vb == VB_) {                                                             \
+    if (sirt)                                                                               \
+      hipLaunchKernelGGL((k_update_em<SB_, VB_, true>), grid, block, 0, st, x, z, den, S,   \
+                         NN, xb, maxw);                                                     \
+    else                                                                                    \
+      hipLaunchKernelGGL((k_update_em<SB_, VB_, false>), grid, block, 0, st, x, z, den, S,  \
+                         NN, xb, maxw);                                                     \
+    return hipGetLastError();                                                               \
   }
+  TRACE_UPDATE_SHAPES(TRACE_UPD_CASE)
 #undef TRACE_UPD_CASE
-  return hipGetLastError();
+  return hipErrorInvalidValue;
 }
 
 hipError_t launch_fill(float *p, int64_t n, float v, hipStream_t st) {
@@ -1614,21 +1619,11 @@ hipError_t launch_fill(float *p, int64_t n, float v, hipStream_t st) {
   return hipGetLastError();
 }
 
-// Slices per thread of the regularised updates: the slot batch, or 4 of it
-// where that leaves fewer than 8192 wavefronts, since a thread takes its slices
-// one after the other (some 10 divisions and a square root each).  All / 4
-// slices (us): APMLR 14 slices 82^2 58 / 18, 9 slices 511^2 59 / 39; PML 20
-// slices 151^2 45 / 14.  Where the wavefronts are there anyway whole lines of
-// the copy are written (PML 32 slices 1024^2 274).
-static bool update_split(int N, int sb, int slots) {
-  return sb > 4 && (int64_t)blocks_for((int64_t)N * N, kPixBlock) * ((slots + sb - 1) / sb) < 2048;
-}
-
 hipError_t launch_update_pml(const float *x, float *xn, const float *z, const float *den,
                              int S, int N, float beta, bool num_direct, int sb, int nslots,
                              float *xb, unsigned *maxw, hipStream_t st) {
   const unsigned bx = blocks_for((int64_t)N * N, kPixBlock);
-  const int vb = update_split(N, sb, nslots) ? 4 : sb;
+  const int vb = update_split((int64_t)N * N, sb, nslots, 2048) ? 4 : sb;
   const dim3 grid(bx, nslots / vb);
 #define TRACE_PML_CASE(SB_, VB_)                                                           \
   if (sb == SB_ && vb == VB_) {                                                            \
@@ -1648,7 +1643,7 @@ hipError_t launch_update_apmlr(const float *xpad, float *xnpad, const float *z,
   // slots: those of the copy and every real slice's
   const int off = compat ? 0 : 1;
   const int need = (nslots > S + 1 - off) ? nslots : S + 1 - off;
-  const int vb = update_split(N, sb, need) ? 4 : sb;
+  const int vb = update_split((int64_t)N * N, sb, need, 2048) ? 4 : sb;
   const dim3 grid(blocks_for((int64_t)N * N, kPixBlock), (need + vb - 1) / vb);
   ApmlrArgs a{w, p, compat, nslots, num_direct ? 1 : 0};
 #define TRACE_APMLR_CASE(SB_, VB_)                                                         \
