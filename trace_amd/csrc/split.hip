@@ -66,8 +66,8 @@ k_forward_split(GridInfo g, const AngleInfo *__restrict__ ang, const RayInfo *__
   constexpr int R = L::kRays;
   constexpr int U = SB == 1 ? 8 : 4;  // gathers in flight
   static_assert(M % U == 0, "whole sets of gathers");
-  __shared__ float s_prod[kBlock / 64][L::kRays * L::kRay];
-  __shared__ float s_sq[kSq ? kBlock / 64 : 1][kSq ? L2::kRays * L2::kRay : 1];
+  __shared__ __align__(16) float s_prod[kBlock / 64][L::kRays * L::kRay];
+  __shared__ __align__(16) float s_sq[kSq ? kBlock / 64 : 1][kSq ? L2::kRays * L2::kRay : 1];
   __shared__ unsigned s_max[SB];
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   const int sub = lane / R, r = lane % R;
