@@ -155,6 +155,27 @@ int ensure_count(trace_handle *h) {
   return TRACE_OK;
 }
 
+// Partial accumulators and tickets for tiles that several workgroups share
+// (256 tickets: no more items are split).
+static int ensure_split(trace_handle *h, TileSplit &split) {
+  split.n = tile_splits(h->geo, h->tile);
+  if (split.n <= 1) return TRACE_OK;
+  constexpr size_t kTickets = 256;
+  const size_t words = kTickets + tile_split_words(h->geo, h->tile, split.n);
+  if (h->split_words < words) {
+    if (h->split) HIP_TRY(hipStreamSynchronize(h->stream));  // a launch may still use it
+    dev_free(h->split);
+    h->split = nullptr;
+    h->split_words = 0;
+    HIP_TRY(dev_alloc(&h->split, words));
+    h->split_words = words;
+    HIP_TRY(launch_fill(reinterpret_cast<float *>(h->split), kTickets, 0.f, h->stream));
+  }
+  split.ticket = h->split;
+  split.part = h->split + kTickets;
+  return TRACE_OK;
+}
+
 // A^T applied with the configured backprojector.  mode: kBpOutSino (w
 // [P][C][S] -> z [S][N][N], with h->maxw holding max |w| per slice, as left
 // by the forward projector or launch_to_pcs), kBpOutOnes / kBpOutCount
@@ -163,8 +184,11 @@ int backproject(trace_handle *h, int mode, const float *w, float *z, int phase) 
   if (int rc = ensure_rays(h)) return rc;
   if (h->backprojector == 0) {
     if (int rc = ensure_count(h)) return rc;
-    TIMED(phase, launch_backproject(h->geo, h->rays, h->count, h->tile, mode, h->exact, w,
-                                    h->maxw, h->maxlen, h->den_max, z, h->wraps, h->stream));
+    TileSplit split;
+    if (mode == kBpOutSino)
+      if (int rc = ensure_split(h, split)) return rc;
+    TIMED(phase, launch_backproject(h->geo, h->rays, h->count, h->tile, mode, h->exact, w, h->maxw,
+                                    h->maxlen, h->den_max, z, h->wraps, split, h->stream));
   } else {
     const int ns = (mode == kBpOutSino) ? h->geo.S : 1;
     TIMED(phase, launch_fill(z, (int64_t)ns * h->geo.NN(), 0.f, h->stream));
@@ -600,7 +624,8 @@ void trace_destroy(trace_handle_t *h) {
   for (void *p : {(void *)h->geo.d_ang, (void *)h->geo.d_yi, (void *)h->rays, (void *)h->count,
                   (void *)h->den, (void *)h->xb, (void *)h->w, (void *)h->z, (void *)h->xa,
                   (void *)h->xc, (void *)h->flag, (void *)h->counters, (void *)h->maxw,
-                  (void *)h->staged.order, (void *)h->staged.group, (void *)h->staged.range})
+                  (void *)h->split, (void *)h->staged.order, (void *)h->staged.group,
+                  (void *)h->staged.range})
     dev_free(p);
   delete h;
 }

@@ -133,6 +133,8 @@ struct trace_handle {
   unsigned long long *counters = nullptr;  // [4]: segments, outside image, max length bits,
                                            // rays with a segment at ix == N
   unsigned *maxw = nullptr;    // [S] bits of max |w| per slice
+  unsigned *split = nullptr;   // tickets and partial tiles (ensure_split)
+  size_t split_words = 0;
   float maxlen = 0.f;          // longest segment of the geometry
   float den_max = 0.f;         // bound on the sum of segment lengths per pixel
   int64_t nnz = 0, nnz_oor = 0;

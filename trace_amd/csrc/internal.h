@@ -183,10 +183,26 @@ hipError_t launch_forward_split(const Geometry &g, const RayInfo *rays, int sb, 
                                 int mode, bool exact, const float *xb, const float *sino,
                                 float *out, unsigned *maxw, hipStream_t st);
 
+// Workgroups that share a tile's angles (16 x 16 tiles, weights only), where
+// an image has at most half as many (tile, slice batch) items as the GPU has CUs
+// and one workgroup's lanes would take two pairs each, or more.  Each leaves its
+// accumulators in `part` and the last one adds them.  One launch, one workgroup /
+// several (us): 1 slice 81^2, 336 angles 63 / 31, 176^2, 300 58 / 42; 7 slices
+// 110^2, 500 151 / 72; 16 slices 81^2, 336 141 / 91; 33 slices 125^2, 122 90 / 84.
+// Too few angles: 7 slices 50^2, 60 26 / 31; tiles enough: 1 slice 256^2, 180
+// 39 / 62.
+struct TileSplit {
+  int n = 1;
+  unsigned *part = nullptr;    // [slice batch][tile][n][accumulator words]
+  unsigned *ticket = nullptr;  // [slice batch][tile], zero between launches
+};
+int tile_splits(const Geometry &g, const TileShape &ts);
+size_t tile_split_words(const Geometry &g, const TileShape &ts, int splits);
+
 hipError_t launch_backproject(const Geometry &g, const RayInfo *rays, const int *count,
                               const TileShape &ts, int mode, bool exact, const float *w,
                               const unsigned *maxw, float maxlen, float denmax, float *z,
-                              bool wraps, hipStream_t st);
+                              bool wraps, const TileSplit &split, hipStream_t st);
 hipError_t launch_absmax_slices(const float *w, int P, int S, int C, unsigned *maxw,
                                 hipStream_t st);
 hipError_t launch_to_pcs(const float *r, int P, int S, int C, float *w, unsigned *maxw,

@@ -401,6 +401,7 @@ struct TileArgs {
   float denmax;       // bound on sum of lengths per pixel (max of A^T 1), kBpSino
   float *z;           // [S][N][N] output (kBpOnes/kBpCount: [N][N])
   int wraps;          // some ray has a segment with ix == N (kRayWraps)
+  TileSplit split;    // workgroups of a tile (k_bp_tile_split)
 };
 
 // LDS accumulator layout of the tile backprojector: one plane per slice,
@@ -762,15 +763,23 @@ constexpr int bp_acc_words() {
 // dynamic LDS (bp_acc_words() words of BpWord<MODE>, then int count[P]
 // when a.count_lds); the body starts and ends with a workgroup barrier, so a
 // persistent workgroup may run it for one tile after another.
-template <int TW, int TH, int SB, int MODE, bool kExact, int BLK>
-__device__ __forceinline__ void bp_tile_body(const TileArgs &a, int tile, int b,
-                                             unsigned long long *lds) {
+//
+// kSplit: this workgroup has taken a share of the angles (a is narrowed to
+// it), `part` is its place among the a.split.n partial accumulators of the
+// tile, and the workgroup that finishes last adds the others' and writes out.
+// The words are integers, so their sum does not depend on the split.  A batch
+// with a non-finite slice is summed in float; `whole` then holds all angles
+// for the first workgroup.
+template <int TW, int TH, int SB, int MODE, bool kExact, int BLK, bool kSplit = false>
+__device__ __forceinline__ void bp_tile_body(TileArgs a, int tile, int b,
+                                             unsigned long long *lds, int part = 0,
+                                             const TileArgs *whole = nullptr) {
   BpWord<MODE> *acc = reinterpret_cast<BpWord<MODE> *>(lds);
   constexpr int PITCH = TilePitch<TW, TH>::kPitch;
   constexpr int PLANE = TilePitch<TW, TH>::kPlane;
   constexpr int WORDS = bp_acc_words<TW, TH, SB, MODE>();
   int *lcount = reinterpret_cast<int *>(acc + WORDS);
-  const int *count = a.count_lds ? lcount : a.count;
+  const int *count = !kSplit && a.count_lds ? lcount : a.count;
   const int N = a.g.N;
   const int tiles_x = (N + TW - 1) / TW;
   const int tx = tile % tiles_x, ty = tile / tiles_x;
@@ -778,7 +787,7 @@ __device__ __forceinline__ void bp_tile_body(const TileArgs &a, int tile, int b,
   const int tx1 = min(tx0 + TW, N), ty1 = min(ty0 + TH, N);
   __syncthreads();  // the previous tile's write-out has read acc and s_ex
   for (int i = threadIdx.x; i < WORDS; i += BLK) acc[i] = 0;
-  if (a.count_lds)
+  if (!kSplit && a.count_lds)
     for (int i = threadIdx.x; i < a.P; i += BLK) lcount[i] = a.count[i];
   // Per-slice scale exponents (kNotFixed: a float slice) in LDS, where the
   // write-out and the mixed form read them; the all-fixed loop takes the
@@ -798,6 +807,13 @@ __device__ __forceinline__ void bp_tile_body(const TileArgs &a, int tile, int b,
     fixed = fixed && (MODE != kBpSino || has_magic(e));
   }
   const bool all_fixed = __syncthreads_and(fixed);
+  if constexpr (kSplit) {
+    if (!all_fixed) {
+      if (part != 0) return;
+      a = *whole;
+    }
+    count = a.count;
+  }
   float magic[SB];
 #pragma unroll
   for (int q = 0; q < SB; ++q) {
@@ -821,6 +837,44 @@ __device__ __forceinline__ void bp_tile_body(const TileArgs &a, int tile, int b,
                                                           s_ex, magic);
   }
   __syncthreads();
+  if constexpr (kSplit) {
+    if (all_fixed) {
+      static_assert(sizeof(BpWord<MODE>) == 4, "32-bit words");
+      const int64_t item = (int64_t)b * gridDim.x + tile;
+      unsigned *parts = a.split.part + item * a.split.n * WORDS;
+      // Agent-scope stores and loads go past the XCDs' L2s to memory, and a
+      // store is complete there when the wavefront's counter reaches zero, which
+      // every wavefront waits for before the barrier and the ticket.  (With
+      // plain stores and a device fence each workgroup wrote its L2 back: one
+      // slice 81^2 at 336 angles 92 us a launch, 43 with one fence a workgroup,
+      // 31 so.)
+      for (int i = threadIdx.x; i < WORDS; i += BLK)
+        __hip_atomic_store(parts + (int64_t)part * WORDS + i, (unsigned)acc[i], __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_AGENT);
+      wait_vector_loads();  // loads and stores share the counter
+      __shared__ int s_last;
+      __syncthreads();
+      if (threadIdx.x == 0) {
+        s_last = atomicAdd(a.split.ticket + item, 1u) == (unsigned)(a.split.n - 1);
+        if (s_last) atomicExch(a.split.ticket + item, 0u);  // for the next launch
+      }
+      __syncthreads();
+      if (!s_last) return;
+      auto get = [](const unsigned *p) {
+        return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      };
+      constexpr int PAIRS = BpPacked<MODE, SB>::value ? SB / 2 * PLANE : 0;  // 64-bit words
+      unsigned long long *acc64 = reinterpret_cast<unsigned long long *>(acc);
+      for (int k = 0; k < a.split.n; ++k) {
+        if (k == part) continue;
+        const unsigned *src = parts + (int64_t)k * WORDS;
+        for (int i = threadIdx.x; i < PAIRS; i += BLK)
+          acc64[i] += ((unsigned long long)get(src + 2 * i + 1) << 32) | get(src + 2 * i);
+        for (int i = 2 * PAIRS + threadIdx.x; i < WORDS; i += BLK) acc[i] += get(src + i);
+      }
+      __syncthreads();
+    }
+  }
   // coalesced write-out: plane by plane, row-contiguous
   const int w_ = tx1 - tx0, h_ = ty1 - ty0;
   if (BpPacked<MODE, SB>::value) {
@@ -883,6 +937,24 @@ __global__ void __launch_bounds__(BLK)
 k_bp_tile(TileArgs a) {
   extern __shared__ unsigned long long acc[];
   bp_tile_body<TW, TH, SB, MODE, kExact, BLK>(a, blockIdx.x, blockIdx.y, acc);
+}
+
+// The angles of a tile shared among a.split.n workgroups (blockIdx.z), for
+// images with fewer tiles than the GPU has CUs.
+template <int TW, int TH, int SB, bool kExact, int BLK>
+__global__ void __launch_bounds__(BLK)
+k_bp_tile_split(TileArgs all) {
+  extern __shared__ unsigned long long acc[];
+  TileArgs a = all;
+  const int per = (all.P + all.split.n - 1) / all.split.n;
+  const int p0 = (int)blockIdx.z * per;
+  a.P = min(per, all.P - p0);  // at least one (tile_splits)
+  a.ang += p0;
+  a.count += p0;
+  a.rays += (int64_t)p0 * a.g.C;
+  a.w += (int64_t)p0 * a.g.C * a.S;
+  bp_tile_body<TW, TH, SB, kBpSino, kExact, BLK, true>(a, blockIdx.x, blockIdx.y, acc,
+                                                       (int)blockIdx.z, &all);
 }
 
 // Per-slice maximum of |w| over w [P][C][S] (float bits, atomicMax on the
@@ -1482,8 +1554,23 @@ int tile_block(int N, int P, int TW, int TH, int SB, int nbatch) {
   return resident * 4 >= want ? 256 : 512;
 }
 
+template <int SB, bool E>
+hipError_t bp_split_launch(const TileArgs &a, int nbatch, hipStream_t st) {
+  constexpr int BLK = kTileBlock;
+  const int tiles = ((a.g.N + 15) / 16) * ((a.g.N + 15) / 16);
+  constexpr size_t lds = (size_t)bp_acc_words<16, 16, SB, kBpSino>() * sizeof(unsigned);
+  static_assert(lds <= 65536, "no attribute needed");
+  hipLaunchKernelGGL((k_bp_tile_split<16, 16, SB, E, BLK>), dim3(tiles, nbatch, a.split.n),
+                     dim3(BLK), lds, st, a);
+  return hipGetLastError();
+}
+
 template <int TW, int TH, int SB>
 hipError_t bp_mode(int mode, bool exact, const TileArgs &a, int nbatch, hipStream_t st) {
+  if constexpr (TW == 16 && TH == 16)
+    if (mode == kBpSino && a.split.n > 1)
+      return exact ? bp_split_launch<SB, true>(a, nbatch, st)
+                   : bp_split_launch<SB, false>(a, nbatch, st);
   if (mode == kBpSino) {
     const int blk = tile_block(a.g.N, a.P, TW, TH, SB, nbatch);
     if constexpr (SB <= 16)
@@ -1539,11 +1626,33 @@ hipError_t launch_forward(const Geometry &g, const RayInfo *rays, int sb, int bu
   return hipErrorInvalidValue;
 }
 
+int tile_splits(const Geometry &g, const TileShape &ts) {
+  if (ts.tw != 16 || ts.th != 16) return 1;
+  const int64_t items = (int64_t)((g.N + 15) / 16) * ((g.N + 15) / 16) * ((g.S + ts.sb - 1) / ts.sb);
+  const int64_t pairs = (int64_t)g.P * 22;  // (angle, column) pairs of a tile
+  if (items > 128 || pairs < 2048) return 1;
+  // up to four workgroups of 256 lanes a CU, a pair for every lane, and at most
+  // 32768 words for the last one to add up
+  int64_t n = 1024 / items;
+  const int64_t words = 32768 / ((ts.sb + 1) * TilePitch<16, 16>::kPlane);
+  n = n < pairs / kTileBlock ? n : pairs / kTileBlock;
+  n = n < words ? n : words;
+  if (n < 2) return 1;
+  const int64_t per = (g.P + n - 1) / n;
+  return (int)((g.P + per - 1) / per);
+}
+
+size_t tile_split_words(const Geometry &g, const TileShape &ts, int splits) {
+  const size_t items = (size_t)((g.N + 15) / 16) * ((g.N + 15) / 16) * ((g.S + ts.sb - 1) / ts.sb);
+  return items * splits * (ts.sb + 1) * TilePitch<16, 16>::kPlane;
+}
+
 hipError_t launch_backproject(const Geometry &g, const RayInfo *rays, const int *count,
                               const TileShape &ts, int mode, bool exact, const float *w,
                               const unsigned *maxw, float maxlen, float denmax, float *z,
-                              bool wraps, hipStream_t st) {
+                              bool wraps, const TileSplit &split, hipStream_t st) {
   TileArgs a;
+  a.split = split;
   a.wraps = wraps ? 1 : 0;
   a.maxw = maxw;
   a.maxlen = maxlen;
