@@ -178,7 +178,7 @@ def _code_only(text: str) -> str:
 # The device code: the kernels and what they include.  Host files (the
 # C-ABI, the batch set-up) choose launch shapes, which every counter record
 # names separately.
-KERNEL_SOURCES = ("internal.h", "kernels.hip", "ordered.hip", "staged.h", "staged.hip",
+KERNEL_SOURCES = ("internal.h", "kernels.hip", "ordered.hip", "split.hip", "staged.h", "staged.hip",
                   "traverse.h")
 
 
