@@ -155,13 +155,35 @@ int ensure_count(trace_handle *h) {
   return TRACE_OK;
 }
 
+// Slices of one launch whose batch is the smallest power of two that holds
+// them, at most 32.
+static int batch_for(int n) {
+  int sb = 1;
+  while (sb < n && sb < 32) sb *= 2;
+  return sb;
+}
+
+// Slices of the stack's first launch.  Where the last of its 32-slice batches
+// would be at most half full, a second launch takes what is left in a batch of
+// its own; not on images so small (below least_side) that two launches one after
+// the other fill the GPU worse than the two batches of one.  One / two launches,
+// 33, 40 and 48 slices (us), adjoint 256^2, 200 angles 291 / 210, 296 / 237,
+// 297 / 258; 1024^2, 240 3678 / 2479, 3669 / 2651, 3717 / 3122; PML num 1024^2,
+// 240 7733 / 5675, 6346, 6692; 512^2, 360 3002 / 2411, 2777, 2935; 320^2, 60
+// 274 / 277, 295, 303.  17 slices in 16 and 1 gain 6% at most and lose where they
+// are ordered.
+static int head_slices(const trace_handle *h, int sb, int least_side) {
+  const int S = h->geo.S, rest = S % 32;
+  return sb == 32 && S > 32 && rest >= 1 && rest <= 16 && h->geo.N >= least_side ? S - rest : S;
+}
+
 // Partial accumulators and tickets for tiles that several workgroups share
 // (256 tickets: no more items are split).
-static int ensure_split(trace_handle *h, TileSplit &split) {
-  split.n = tile_splits(h->geo, h->tile);
+static int ensure_split(trace_handle *h, const TileShape &tile, int n, TileSplit &split) {
+  split.n = tile_splits(h->geo, tile, n);
   if (split.n <= 1) return TRACE_OK;
   constexpr size_t kTickets = 256;
-  const size_t words = kTickets + tile_split_words(h->geo, h->tile, split.n);
+  const size_t words = kTickets + tile_split_words(h->geo, tile, n, split.n);
   if (h->split_words < words) {
     if (h->split) HIP_TRY(hipStreamSynchronize(h->stream));  // a launch may still use it
     dev_free(h->split);
@@ -184,11 +206,19 @@ int backproject(trace_handle *h, int mode, const float *w, float *z, int phase) 
   if (int rc = ensure_rays(h)) return rc;
   if (h->backprojector == 0) {
     if (int rc = ensure_count(h)) return rc;
-    TileSplit split;
-    if (mode == kBpOutSino)
-      if (int rc = ensure_split(h, split)) return rc;
-    TIMED(phase, launch_backproject(h->geo, h->rays, h->count, h->tile, mode, h->exact, w, h->maxw,
-                                    h->maxlen, h->den_max, z, h->wraps, split, h->stream));
+    const int S = mode == kBpOutSino ? h->geo.S : 1;
+    const int head = mode == kBpOutSino && h->tile_default ? head_slices(h, h->tile.sb, 256) : S;
+    for (int s0 = 0; s0 < S; s0 += head) {
+      TileShape tile = h->tile;
+      const int n = s0 == 0 ? head : S - head;
+      if (head < S) tile.sb = batch_for(n);
+      TileSplit split;
+      if (mode == kBpOutSino)
+        if (int rc = ensure_split(h, tile, n, split)) return rc;
+      TIMED(phase, launch_backproject(h->geo, h->rays, h->count, tile, mode, h->exact, w, h->maxw,
+                                      h->maxlen, h->den_max, z, h->wraps, split, s0, n,
+                                      h->stream));
+    }
   } else {
     const int ns = (mode == kBpOutSino) ? h->geo.S : 1;
     TIMED(phase, launch_fill(z, (int64_t)ns * h->geo.NN(), 0.f, h->stream));
@@ -246,7 +276,7 @@ int ordered_den(trace_handle *h, float *out) {
   unsigned *ovf = reinterpret_cast<unsigned *>(h->flag);
   auto launch = [&](int form) {
     return launch_bp_ordered(h->geo, h->rays, kOrdDen, h->exact, nullptr, nullptr, 1, 1, out,
-                             h->wraps, form > 0 ? ovf : nullptr, form == 2, h->stream);
+                             h->wraps, form > 0 ? ovf : nullptr, form == 2, 0, 1, h->stream);
   };
   hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
   (void)hipStreamIsCapturing(h->stream, &capture);
@@ -283,8 +313,13 @@ int backproject_ordered(trace_handle *h, int mode, const float *w, float *z, int
   const int sb = ordered_batch(mode, h->geo.S, h->xb_sb, tile);
   // the tile form's overflow flag was checked on this geometry by the den pass
   unsigned *ovf = tile ? reinterpret_cast<unsigned *>(h->flag) : nullptr;
-  TIMED(phase, launch_bp_ordered(h->geo, h->rays, mode, h->exact, w, h->xb, h->xb_sb, sb, z,
-                                 h->wraps, ovf, h->ord_tile == 2, h->stream));
+  const int S = h->geo.S, head = head_slices(h, sb, 400);
+  for (int s0 = 0; s0 < S; s0 += head) {
+    const int n = s0 == 0 ? head : S - head;
+    TIMED(phase, launch_bp_ordered(h->geo, h->rays, mode, h->exact, w, h->xb, h->xb_sb,
+                                   head < S ? batch_for(n) : sb, z, h->wraps, ovf,
+                                   h->ord_tile == 2, s0, n, h->stream));
+  }
   return TRACE_OK;
 }
 
@@ -708,6 +743,7 @@ int trace_set_launch_shape(trace_handle_t *h, int fwd_batch, int tile_w, int til
   h->fwd_sb = fwd_batch;
   if (!fwd_shape_supported(fwd_batch, h->fwd_lanes)) h->fwd_lanes = 1;
   h->tile = TileShape{tile_w, tile_h, tile_batch};
+  h->tile_default = false;
   return TRACE_OK;
 }
 

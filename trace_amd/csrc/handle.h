@@ -112,6 +112,7 @@ struct trace_handle {
   int fwd_staged = -1;    // TRACE_OPT_FWD_STAGED: 0 or 1 as set, -1 chosen by staged_faster
   trace_hip::StagedPlan staged;  // slab plan of the staged forward projector
   trace_hip::TileShape tile{16, 16, 16};
+  bool tile_default = true;  // not set by the caller
   trace_hip::RayInfo *rays = nullptr;     // [P][C]
   bool rays_ready = false;
   int *count = nullptr;        // [P] columns-per-tile bound for count_shape

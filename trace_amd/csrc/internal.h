@@ -168,11 +168,11 @@ struct BatchQueues {
 // non-null the tile form runs (with grid_rays the one for geometries with rays
 // on grid lines, wrapped segments among them) and ORs a nonzero value into
 // *tile_overflow when a pixel needs more LDS slots than it has; without, the
-// per-pixel form.
+// per-pixel form.  Slices [s0, s0 + n) of the stack, s0 a multiple of sb.
 hipError_t launch_bp_ordered(const Geometry &g, const RayInfo *rays, int mode, bool exact,
                              const float *w, const float *xb, int xsb, int sb, float *out,
                              bool wraps, unsigned *tile_overflow, bool grid_rays,
-                             hipStream_t st);
+                             int s0, int n, hipStream_t st);
 bool ordered_sb_supported(int mode, int sb, int xsb);
 
 // Forward projection with `lanes` lanes per ray (split.hip): sb slices to a
@@ -196,13 +196,16 @@ struct TileSplit {
   unsigned *part = nullptr;    // [slice batch][tile][n][accumulator words]
   unsigned *ticket = nullptr;  // [slice batch][tile], zero between launches
 };
-int tile_splits(const Geometry &g, const TileShape &ts);
-size_t tile_split_words(const Geometry &g, const TileShape &ts, int splits);
+int tile_splits(const Geometry &g, const TileShape &ts, int n_slices);
+size_t tile_split_words(const Geometry &g, const TileShape &ts, int n_slices, int splits);
+
+// Slices [s0, s0 + n) of the stack (s0 = 0, n = 1 for column sums and counts).
 
 hipError_t launch_backproject(const Geometry &g, const RayInfo *rays, const int *count,
                               const TileShape &ts, int mode, bool exact, const float *w,
                               const unsigned *maxw, float maxlen, float denmax, float *z,
-                              bool wraps, const TileSplit &split, hipStream_t st);
+                              bool wraps, const TileSplit &split, int s0, int n,
+                              hipStream_t st);
 hipError_t launch_absmax_slices(const float *w, int P, int S, int C, unsigned *maxw,
                                 hipStream_t st);
 hipError_t launch_to_pcs(const float *r, int P, int S, int C, float *w, unsigned *maxw,

@@ -392,7 +392,8 @@ struct TileArgs {
   const AngleInfo *ang;
   const RayInfo *rays;
   const int *count;   // [P] upper bound of the columns touching any tile
-  int P, S;
+  int P, S;           // S: slices of a row of w
+  int n;              // slices from w, maxw and z on
   int count_lds;      // 1: count[] is staged in LDS after the accumulators
   float yi0;          // detector coordinate of column 0
   const float *w;     // [P][C][S] weights (kBpSino)
@@ -539,7 +540,7 @@ __device__ __forceinline__ void bp_tile_loop(const TileArgs &a, BpWord<MODE> *ac
   const float y0 = grid_line(N, wy0), y1 = grid_line(N, wy1);
   // the strip's column range is at most one wider than a tile's
   constexpr int extra = EDGE ? 1 : 0;
-  const bool full = (b + 1) * SB <= a.S;  // no slot past the stack's last slice
+  const bool full = (b + 1) * SB <= a.n;  // no slot past the stack's last slice
   // Lane t takes flat slots t, t + BLK, ... of the tile's (angle,
   // column) pairs.  One slice (kRank): slot f is rank r = f / P of angle
   // p = f % P, rank r being the r-th of the angle's column slots counted
@@ -662,7 +663,7 @@ __device__ __forceinline__ void bp_tile_loop(const TileArgs &a, BpWord<MODE> *ac
 #pragma unroll
         for (int q = 0; q < SB; ++q) {
           // slots past the stack's last slice (read from the next row) add 0
-          const float wq = full || b * SB + q < a.S ? cur.w[q] : 0.f;
+          const float wq = full || b * SB + q < a.n ? cur.w[q] : 0.f;
           nz |= __float_as_uint(wq);
           wv[q] = (!ALLFX && ex[q] != kNotFixed) ? ldexpf(wq, ex[q]) : wq;
         }
@@ -799,7 +800,7 @@ __device__ __forceinline__ void bp_tile_body(TileArgs a, int tile, int b,
     const int s = b * SB + (int)threadIdx.x;
     int e;
     if (MODE == kBpSino)
-      e = weight_exponent((s < a.S) ? __uint_as_float(a.maxw[s]) : 0.f, a.denmax, a.maxlen,
+      e = weight_exponent((s < a.n) ? __uint_as_float(a.maxw[s]) : 0.f, a.denmax, a.maxlen,
                           fixed);
     else
       e = fixed_exponent(1.0f, a.maxlen, fixed);
@@ -897,7 +898,7 @@ __device__ __forceinline__ void bp_tile_body(TileArgs a, int tile, int b,
         for (int h = 0; h < 2; ++h) {
           const int q = 2 * k2 + h;
           const int s = b * SB + q;
-          if (s >= a.S) break;
+          if (s >= a.n) break;
           const unsigned half = h ? (unsigned)(v >> 32) : (unsigned)v;
           float out;
           if (s_ex[q] == kNotFixed)
@@ -913,7 +914,7 @@ __device__ __forceinline__ void bp_tile_body(TileArgs a, int tile, int b,
 #pragma unroll
   for (int q = 0; q < SB; ++q) {
     const int s = b * SB + q;
-    if (MODE == kBpSino && s >= a.S) break;
+    if (MODE == kBpSino && s >= a.n) break;
     float *zs = a.z + (int64_t)s * N * N;
     for (int i = threadIdx.x; i < w_ * h_; i += BLK) {
       const int ly = i / w_, lx = i - ly * w_;
@@ -1353,7 +1354,7 @@ k_bp_batch(const BatchSliceDev *__restrict__ d, BatchQueues q, int it) {
     a.rays = sd.rays;
     a.count = sd.count;
     a.P = sd.P;
-    a.S = 1;
+    a.S = a.n = 1;
     a.count_lds = 1;
     a.yi0 = sd.yi0;
     a.w = sd.w;
@@ -1626,9 +1627,9 @@ hipError_t launch_forward(const Geometry &g, const RayInfo *rays, int sb, int bu
   return hipErrorInvalidValue;
 }
 
-int tile_splits(const Geometry &g, const TileShape &ts) {
+int tile_splits(const Geometry &g, const TileShape &ts, int n_slices) {
   if (ts.tw != 16 || ts.th != 16) return 1;
-  const int64_t items = (int64_t)((g.N + 15) / 16) * ((g.N + 15) / 16) * ((g.S + ts.sb - 1) / ts.sb);
+  const int64_t items = (int64_t)((g.N + 15) / 16) * ((g.N + 15) / 16) * ((n_slices + ts.sb - 1) / ts.sb);
   const int64_t pairs = (int64_t)g.P * 22;  // (angle, column) pairs of a tile
   if (items > 128 || pairs < 2048) return 1;
   // up to four workgroups of 256 lanes a CU, a pair for every lane, and at most
@@ -1642,19 +1643,20 @@ int tile_splits(const Geometry &g, const TileShape &ts) {
   return (int)((g.P + per - 1) / per);
 }
 
-size_t tile_split_words(const Geometry &g, const TileShape &ts, int splits) {
-  const size_t items = (size_t)((g.N + 15) / 16) * ((g.N + 15) / 16) * ((g.S + ts.sb - 1) / ts.sb);
+size_t tile_split_words(const Geometry &g, const TileShape &ts, int n_slices, int splits) {
+  const size_t items = (size_t)((g.N + 15) / 16) * ((g.N + 15) / 16) * ((n_slices + ts.sb - 1) / ts.sb);
   return items * splits * (ts.sb + 1) * TilePitch<16, 16>::kPlane;
 }
 
 hipError_t launch_backproject(const Geometry &g, const RayInfo *rays, const int *count,
                               const TileShape &ts, int mode, bool exact, const float *w,
                               const unsigned *maxw, float maxlen, float denmax, float *z,
-                              bool wraps, const TileSplit &split, hipStream_t st) {
+                              bool wraps, const TileSplit &split, int s0, int n,
+                              hipStream_t st) {
   TileArgs a;
   a.split = split;
   a.wraps = wraps ? 1 : 0;
-  a.maxw = maxw;
+  a.maxw = maxw ? maxw + s0 : nullptr;
   a.maxlen = maxlen;
   a.denmax = denmax;
   a.g = g.grid;
@@ -1663,10 +1665,11 @@ hipError_t launch_backproject(const Geometry &g, const RayInfo *rays, const int 
   a.count = count;
   a.P = g.P;
   a.S = g.S;
+  a.n = n;
   a.yi0 = g.yi0;
-  a.w = w;
-  a.z = z;
-  const int nb = (g.S + ts.sb - 1) / ts.sb;
+  a.w = w ? w + s0 : nullptr;
+  a.z = z + (int64_t)s0 * g.NN();
+  const int nb = (n + ts.sb - 1) / ts.sb;
 #define TRACE_BP_CASE(TW_, TH_, SB_)                              \
   if (ts.tw == TW_ && ts.th == TH_ && ts.sb == SB_)               \
     return bp_mode<TW_, TH_, SB_>(mode, exact, a, nb, st);

@@ -68,7 +68,8 @@ struct OrdArgs {
   GridInfo g;
   const AngleInfo *ang;
   const RayInfo *rays;
-  int P, S;
+  int P, S;         // S: slices of a row of w
+  int n;            // slices from w, xb and out on
   float yi0;
   const float *w;   // [P][C][S] per-ray weights (kOrdNum, kOrdEM)
   const float *xb;  // [S/xsb][N*N][xsb] image the ray pass read (kOrdNum)
@@ -144,7 +145,7 @@ k_bp_ordered(OrdArgs a) {
       if (MODE != kOrdDen) {
         const float *wr = a.w + t * a.S + b * SB;
 #pragma unroll
-        for (int q = 0; q < SB; ++q) wv[q] = (b * SB + q < a.S) ? wr[q] : 0.f;
+        for (int q = 0; q < SB; ++q) wv[q] = (b * SB + q < a.n) ? wr[q] : 0.f;
       }
       auto visit = [&](int ix, int iy, float l, float) {
         const bool wrap = (ix == N);
@@ -186,7 +187,7 @@ k_bp_ordered(OrdArgs a) {
       const int s = b * SB + q;
       if (MODE == kOrdDen)
         a.out[j] = acc[i][0];
-      else if (s < a.S)
+      else if (s < a.n)
         a.out[(int64_t)s * NN + j] = acc[i][q];
     }
   }
@@ -197,7 +198,7 @@ hipError_t ord_launch(const OrdArgs &a, bool exact, hipStream_t st) {
   const int N = a.g.N;
   const int sxn = (N + PW - 1) / PW, syn = (N + PH - 1) / PH;
   const int blocks = ((sxn + kOrdStrips - 1) / kOrdStrips) * ((syn + kOrdStrips - 1) / kOrdStrips);
-  const int nb = MODE == kOrdDen ? 1 : (a.S + SB - 1) / SB;
+  const int nb = MODE == kOrdDen ? 1 : (a.n + SB - 1) / SB;
   if (exact)
     hipLaunchKernelGGL((k_bp_ordered<PW, PH, SB, MODE, true>), dim3(blocks, nb),
                        dim3(kOrdBlock), 0, st, a);
@@ -358,7 +359,7 @@ k_bp_ordered_tile(OrdArgs a, unsigned *__restrict__ overflow) {
           // slots past the stack's last slice (read from the next row) add 0
           float *dst = s_w + (ai1 * kORanks + k1) * WP;
 #pragma unroll
-          for (int q = 0; q < SB; ++q) dst[q] = b * SB + q < a.S ? cur.w[q] : 0.f;
+          for (int q = 0; q < SB; ++q) dst[q] = b * SB + q < a.n ? cur.w[q] : 0.f;
         }
         const int slot = column_slot(c);
         float *len0 = &s_len[ai1][slot * kODups][0];
@@ -463,7 +464,7 @@ k_bp_ordered_tile(OrdArgs a, unsigned *__restrict__ overflow) {
   }
 #pragma unroll
   for (int q = 0; q < SB; ++q)
-    if (b * SB + q < a.S) a.out[(int64_t)(b * SB + q) * NN + j] = acc[q];
+    if (b * SB + q < a.n) a.out[(int64_t)(b * SB + q) * NN + j] = acc[q];
 }
 
 // LDS of W wavefronts summing SB slices.
@@ -623,7 +624,7 @@ k_bp_ordered_shared(OrdArgs a, unsigned *__restrict__ overflow) {
     if (MODE != kOrdDen) {
       const float *wr = a.w + t * a.S + b * SB;
       float *dst = lds.w[wv][kOA * kORanks + ai1];
-      for (int q = 0; q < SB; ++q) dst[q] = b * SB + q < a.S ? wr[q] : 0.f;
+      for (int q = 0; q < SB; ++q) dst[q] = b * SB + q < a.n ? wr[q] : 0.f;
     }
     traverse_window<kExact, true>(a.g, ray, ang.quadrant, N - 1, N, ty0 - 1, ty1,
                                   [&](int ix, int iy, float l, float) {
@@ -654,7 +655,7 @@ k_bp_ordered_shared(OrdArgs a, unsigned *__restrict__ overflow) {
         // slots past the stack's last slice (read from the next row) add 0
         float *dst = lds.w[wv][lane];
 #pragma unroll
-        for (int q = 0; q < SB; ++q) dst[q] = b * SB + q < a.S ? cur.w[q] : 0.f;
+        for (int q = 0; q < SB; ++q) dst[q] = b * SB + q < a.n ? cur.w[q] : 0.f;
       }
       const int slot = column_slot(c);
       float *len0 = lds.len[wv][(ai1 * kOSlots + slot) * Lds::kDups];
@@ -776,14 +777,14 @@ k_bp_ordered_shared(OrdArgs a, unsigned *__restrict__ overflow) {
   }
 #pragma unroll
   for (int q = 0; q < SBW; ++q)
-    if (s0 + q < a.S) a.out[(int64_t)(s0 + q) * NN + j] = acc[q];
+    if (s0 + q < a.n) a.out[(int64_t)(s0 + q) * NN + j] = acc[q];
 }
 
 template <int SB, int W, int MODE, bool kGrid>
 hipError_t ord_shared_launch(const OrdArgs &a, bool exact, unsigned *overflow, hipStream_t st) {
   const int N = a.g.N;
   const int tiles = ((N + kOT - 1) / kOT) * ((N + kOT - 1) / kOT);
-  const int nb = MODE == kOrdDen ? 1 : (a.S + SB - 1) / SB;
+  const int nb = MODE == kOrdDen ? 1 : (a.n + SB - 1) / SB;
   constexpr size_t lds = sizeof(OrdSharedLds<SB, W, kGrid>);
   static_assert(lds <= 160 * 1024, "a workgroup's LDS");
   auto kern = exact ? k_bp_ordered_shared<SB, W, MODE, true, kGrid>
@@ -801,7 +802,7 @@ template <int SB, int MODE>
 hipError_t ord_tile_launch(const OrdArgs &a, bool exact, unsigned *overflow, hipStream_t st) {
   const int N = a.g.N;
   const int tiles = ((N + kOT - 1) / kOT) * ((N + kOT - 1) / kOT);
-  const int nb = MODE == kOrdDen ? 1 : (a.S + SB - 1) / SB;
+  const int nb = MODE == kOrdDen ? 1 : (a.n + SB - 1) / SB;
   if (exact)
     hipLaunchKernelGGL((k_bp_ordered_tile<SB, MODE, true>), dim3(tiles, nb), dim3(kOWave), 0, st,
                        a, overflow);
@@ -838,24 +839,27 @@ bool ordered_sb_supported(int mode, int sb, int xsb) {
 hipError_t launch_bp_ordered(const Geometry &g, const RayInfo *rays, int mode, bool exact,
                              const float *w, const float *xb, int xsb, int sb, float *out,
                              bool wraps, unsigned *tile_overflow, bool grid_rays,
-                             hipStream_t st) {
+                             int s0, int n, hipStream_t st) {
   OrdArgs a;
   a.g = g.grid;
   a.ang = g.d_ang;
   a.rays = rays;
   a.P = g.P;
   a.S = g.S;
+  a.n = n;
   a.yi0 = g.yi0;
-  a.w = w;
-  a.xb = xb;
+  a.w = w ? w + s0 : nullptr;
+  // a slot batch of the copy, and the slots within it (the kernels step from
+  // there by sb, which divides xsb)
+  a.xb = xb ? xb + (int64_t)(s0 / xsb) * g.NN() * xsb + s0 % xsb : nullptr;
   a.xsb = xsb;
-  a.out = out;
+  a.out = out + (int64_t)s0 * g.NN();
   a.wraps = wraps ? 1 : 0;
   if (!ordered_sb_supported(mode, sb, xsb)) return hipErrorInvalidValue;
   if (tile_overflow) {
     // tile form; wrapped segments need the grid-ray one
     if (wraps && !grid_rays) return hipErrorInvalidValue;
-    const int waves = ordered_waves(g.N, mode == kOrdDen ? 1 : g.S, sb, grid_rays);
+    const int waves = ordered_waves(g.N, mode == kOrdDen ? 1 : n, sb, grid_rays);
 #define TRACE_ORDS_CASE(SB_, W_, GRID_)                                                     \
   if (waves == W_ && grid_rays == GRID_) {                                                      \
     if (mode == kOrdDen)                                                                     \
