@@ -108,7 +108,8 @@ typedef struct trace_handle trace_handle_t;
                                  16 slices, 2 at 5-16, else 1): the lanes
                                  of a ray split its slice batch; compiled for
                                  batches 8, 16 and 32 (2 lanes) and 16, 32
-                                 (4 lanes) */
+                                 (4 lanes).  Launches of few rays, whose lanes
+                                 share a ray's walk instead, do not read it */
 
 #define TRACE_OPT_ORDERED_SUMS 6 /* order of the backprojected float sums:
                                     0: every sum in 32-bit fixed point
@@ -134,7 +135,8 @@ typedef struct trace_handle trace_handle_t;
                                   similar direction x 64 columns sweep the
                                   image in slabs staged in LDS; 0: every ray
                                   reads its pixels from HBM (the form used at
-                                  other slice batches).  Until it is set, the
+                                  other slice batches; where rays are few,
+                                  several lanes share the walk of each).  Until it is set, the
                                   faster of the two for the geometry; reads
                                   as 1 then */
 

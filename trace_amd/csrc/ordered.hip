@@ -42,8 +42,9 @@
 // the column modulo 3 tells them apart, and a ray puts at most two segments
 // in one pixel, one after the other, on the geometries measured (two where
 // it grazes a corner); a geometry that would need more sets a flag when den
-// is computed, and the handle then keeps the per-pixel form.  Geometries
-// with wrapped segments use the per-pixel form.
+// is computed.  Geometries with rays on grid lines need more, and have
+// wrapped segments: a variant of the shared form below serves them, and what
+// overflows there too keeps the per-pixel form.
 //
 // The walks bound the one-slice form, the sums the deeper ones.  Filing a
 // segment waits for nothing: its slot is the lane's own (the ray's column
