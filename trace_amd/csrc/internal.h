@@ -44,11 +44,14 @@ constexpr int kWeightPad = 32;
 // Pixel blocks (of 256 pixels) per work item of the batched image update.
 constexpr int kBatchUpdateBlocks = 16;
 
-// A slice batch of an N x N image of 2^32 bytes or more: past the reach of
-// the buffer resource and 32-bit offsets the forward projector gathers with.
-// One slice has a form for it; deeper batches are cut until they fit.
+// A slice batch of an N x N image too large for the buffer resource and the
+// 32-bit offsets the forward projector gathers with.  One slice has a form for
+// it; deeper batches are cut until they fit.  A segment on the far grid lines has
+// an index up to N^2 + N: its offset too must stay below 2^32, past the
+// resource's range, where it reads 0 (at 23170^2 with 2 slices and 11585^2 with
+// 8 the image fits but such an offset would wrap to a pixel of row 0).
 __host__ __device__ inline bool wide_image(int N, int sb) {
-  return (uint64_t)N * (uint64_t)N * (uint64_t)sb * 4 >= (uint64_t(1) << 32);
+  return ((uint64_t)N * (uint64_t)N + (uint64_t)N + 1) * (uint64_t)sb * 4 > (uint64_t(1) << 32);
 }
 
 enum Alg { kSIRT = 0, kMLEM = 1, kPML = 2, kAPMLR = 3 };
