@@ -59,9 +59,19 @@ int fail(int code, const std::string &msg) {
 
 int nbatch(int S, int sb) { return (S + sb - 1) / sb; }
 
+// Whether the handle's stream is being captured into a graph: nothing can be
+// allocated, copied from the host or read back then.
+static bool capturing(trace_handle *h) {
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(h->stream, &status) != hipSuccess) (void)hipGetLastError();
+  return status != hipStreamCaptureStatusNone;
+}
+
+// A capture that finds no plan takes another form (the same sums).
 bool forward_staged(trace_handle *h) {
   if (h->fwd_staged == 0 || !staged_batch(h->fwd_sb)) return false;
-  return h->fwd_staged == 1 || staged_faster(h->geo, h->fwd_sb);
+  if (h->fwd_staged != 1 && !staged_faster(h->geo, h->fwd_sb)) return false;
+  return h->staged.sb == h->fwd_sb || !capturing(h);
 }
 
 int forward_batch(trace_handle *h) {
@@ -178,13 +188,18 @@ static int head_slices(const trace_handle *h, int sb, int least_side) {
 }
 
 // Partial accumulators and tickets for tiles that several workgroups share
-// (256 tickets: no more items are split).
+// (256 tickets: no more items are split).  In a capture that would need more of
+// them than there are, one workgroup takes a tile (the same sums).
 static int ensure_split(trace_handle *h, const TileShape &tile, int n, TileSplit &split) {
   split.n = tile_splits(h->geo, tile, n);
   if (split.n <= 1) return TRACE_OK;
   constexpr size_t kTickets = 256;
   const size_t words = kTickets + tile_split_words(h->geo, tile, n, split.n);
   if (h->split_words < words) {
+    if (capturing(h)) {
+      split.n = 1;
+      return TRACE_OK;
+    }
     if (h->split) HIP_TRY(hipStreamSynchronize(h->stream));  // a launch may still use it
     dev_free(h->split);
     h->split = nullptr;
@@ -278,11 +293,9 @@ int ordered_den(trace_handle *h, float *out) {
     return launch_bp_ordered(h->geo, h->rays, kOrdDen, h->exact, nullptr, nullptr, 1, 1, out,
                              h->wraps, form > 0 ? ovf : nullptr, form == 2, 0, 1, h->stream);
   };
-  hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-  (void)hipStreamIsCapturing(h->stream, &capture);
   // decided before; or undecided where nothing can be read back: the form that
   // always serves
-  if (h->ord_tile >= 0 || capture != hipStreamCaptureStatusNone) {
+  if (h->ord_tile >= 0 || capturing(h)) {
     TIMED(TRACE_PHASE_SETUP, launch(h->ord_tile < 0 ? 0 : h->ord_tile));
     return TRACE_OK;
   }
@@ -923,7 +936,9 @@ int trace_adjoint(trace_handle_t *h, const float *r, float *z) {
   if (!h) return fail(TRACE_E_INVALID, "handle is null");
   if (!r || !z) return fail(TRACE_E_INVALID, "null buffer");
   HIP_TRY(hipSetDevice(h->device));
-  if (int rc = ensure_work(h, false)) return rc;
+  // the copy of the image is not read here, but allocated for the projections
+  // that may follow under capture (a one-slice reconstruction leaves none behind)
+  if (int rc = ensure_work(h, false, !capturing(h))) return rc;
   if (int rc = ensure_den(h)) return rc;  // fixed-point scale of A^T
   TIMED(TRACE_PHASE_SETUP,
         launch_fill(reinterpret_cast<float *>(h->maxw), h->geo.S, 0.f, h->stream));
