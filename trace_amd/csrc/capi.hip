@@ -302,6 +302,7 @@ int ordered_den(trace_handle *h, float *out) {
   // the plain tile form, the one for rays on grid lines, the per-pixel form: the
   // first that has the slots
   for (int form = h->wraps ? 2 : 1; form <= 2; ++form) {
+    if (form == 2 && !ordered_grid_rays_fit(h->geo.N)) break;
     HIP_TRY(hipMemsetAsync(ovf, 0, sizeof(unsigned), h->stream));
     TIMED(TRACE_PHASE_SETUP, launch(form));
     unsigned f = 0;

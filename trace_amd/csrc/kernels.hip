@@ -1548,6 +1548,8 @@ int tile_block(int N, int P, int TW, int TH, int SB, int nbatch) {
   const int64_t tiles = (int64_t)((N + TW - 1) / TW) * ((N + TH - 1) / TH) * nbatch;
   const double per_cu = tiles / 256.0;
   if (per_cu <= 1.0) return 1024;  // a CU holds one such workgroup
+  // a launch holds fewer than 2^32 lanes (8x8 tiles from 23171^2 on)
+  if (tiles / nbatch * 512 >= (int64_t(1) << 32)) return 256;
   const size_t lds = (size_t)TH * (TW + 1) * 4 * (SB + (SB > 1 ? 1 : 0)) + (size_t)P * sizeof(int);
   const int waves = SB <= 8 ? 28 : (SB <= 16 ? 20 : 12);  // by vector registers
   const int want = waves < 24 ? waves : 24;

@@ -831,6 +831,13 @@ int ordered_waves(int N, int S, int sb, bool grid_rays) {
   return tiles <= 128 ? 8 : (tiles <= (sb == 32 ? 3000 : 1536) ? 4 : 1);
 }
 
+// A launch holds fewer than 2^32 lanes: four wavefronts a tile reach that from
+// 32761^2 on, where geometries with rays on grid lines keep the per-pixel form.
+bool ordered_grid_rays_fit(int N) {
+  const int64_t side = (N + kOT - 1) / kOT;
+  return side * side * kOWave * ordered_waves(N, 1, 1, true) < (int64_t(1) << 32);
+}
+
 bool ordered_sb_supported(int mode, int sb, int xsb) {
   if (mode == kOrdDen) return true;
   if (sb != 1 && sb != 2 && sb != 4 && sb != 8 && sb != 16 && sb != 32) return false;
