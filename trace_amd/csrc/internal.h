@@ -192,8 +192,8 @@ hipError_t launch_forward_split(const Geometry &g, const RayInfo *rays, int sb, 
 // an image has at most half as many (tile, slice batch) items as the GPU has CUs
 // and one workgroup's lanes would take two pairs each, or more.  Each leaves its
 // accumulators in `part` and the last one adds them.  One launch, one workgroup /
-// several (us): 1 slice 81^2, 336 angles 63 / 31, 176^2, 300 58 / 42; 7 slices
-// 110^2, 500 151 / 72; 16 slices 81^2, 336 141 / 91; 33 slices 125^2, 122 90 / 84.
+// several (us): 1 slice 81^2, 336 angles 65 / 34, 176^2, 300 60 / 43; 7 slices
+// 110^2, 500 151 / 73; 16 slices 81^2, 336 145 / 93; 33 slices 125^2, 122 91 / 85.
 // Too few angles: 7 slices 50^2, 60 26 / 31; tiles enough: 1 slice 256^2, 180
 // 39 / 62.
 struct TileSplit {

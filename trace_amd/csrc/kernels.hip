@@ -843,12 +843,12 @@ __device__ __forceinline__ void bp_tile_body(TileArgs a, int tile, int b,
       static_assert(sizeof(BpWord<MODE>) == 4, "32-bit words");
       const int64_t item = (int64_t)b * gridDim.x + tile;
       unsigned *parts = a.split.part + item * a.split.n * WORDS;
-      // Agent-scope stores and loads go past the XCDs' L2s to memory, and a
-      // store is complete there when the wavefront's counter reaches zero, which
-      // every wavefront waits for before the barrier and the ticket.  (With
-      // plain stores and a device fence each workgroup wrote its L2 back: one
-      // slice 81^2 at 336 angles 92 us a launch, 43 with one fence a workgroup,
-      // 31 so.)
+      // Every wavefront's stores are complete at the barrier; the release on the
+      // ticket then publishes the workgroup's words to the GPU, and the acquire
+      // of the workgroup that takes the last ticket sees those of all before it
+      // (each ticket's release goes on in the read-modify-writes that follow it).
+      // The words go past the XCD's L2 besides (agent scope), which leaves the
+      // release little to write back.
       for (int i = threadIdx.x; i < WORDS; i += BLK)
         __hip_atomic_store(parts + (int64_t)part * WORDS + i, (unsigned)acc[i], __ATOMIC_RELAXED,
                            __HIP_MEMORY_SCOPE_AGENT);
@@ -856,8 +856,13 @@ __device__ __forceinline__ void bp_tile_body(TileArgs a, int tile, int b,
       __shared__ int s_last;
       __syncthreads();
       if (threadIdx.x == 0) {
-        s_last = atomicAdd(a.split.ticket + item, 1u) == (unsigned)(a.split.n - 1);
-        if (s_last) atomicExch(a.split.ticket + item, 0u);  // for the next launch
+        unsigned *ticket = a.split.ticket + item;
+        s_last = __hip_atomic_fetch_add(ticket, 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT) ==
+                 (unsigned)(a.split.n - 1);
+        if (s_last) {
+          __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+          atomicExch(ticket, 0u);  // for the next launch
+        }
       }
       __syncthreads();
       if (!s_last) return;
