@@ -196,10 +196,10 @@ def kernel_source_hash(d: str | None = None) -> str:
 
 
 def fwd_staged(pj) -> bool:
-    """True when the projector's forward launches run the slab-staged form
-    (32-slice batches and TRACE_OPT_FWD_STAGED on)."""
+    """True when the projector's forward launches run the slab-staged form at
+    32-slice batches."""
     from trace_amd import _capi
-    return pj.launch_shape()[0] == 32 and pj.get_option(_capi.TRACE_OPT_FWD_STAGED) == 1
+    return pj.launch_shape()[0] == 32 and pj.fwd_form() == _capi.TRACE_FORM_STAGED
 
 
 def fwd_shape(pj) -> list:

@@ -136,9 +136,24 @@ typedef struct trace_handle trace_handle_t;
                                   image in slabs staged in LDS; 0: every ray
                                   reads its pixels from HBM (the form used at
                                   other slice batches; where rays are few,
-                                  several lanes share the walk of each).  Until it is set, the
-                                  faster of the two for the geometry; reads
-                                  as 1 then */
+                                  several lanes share the walk of each).
+                                  Until it is set, the faster of the two for
+                                  the geometry; reads as 1 then */
+#define TRACE_OPT_FWD_FORM 9 /* read only: the form the next projection takes
+                                at the present launch shape (TRACE_FORM_*);
+                                only the whole-ray one reads the lanes and the
+                                bundle */
+#define TRACE_OPT_BACK_REST 10 /* 1: where a stack's last batch of 32 slices
+                                  would be at most half full, the slices past
+                                  the batch before it are backprojected in a
+                                  launch of their own (same bits); 0: one
+                                  launch.  1 until trace_set_launch_shape,
+                                  which sets 0 */
+
+/* Forms of the forward projector (TRACE_OPT_FWD_FORM). */
+#define TRACE_FORM_WHOLE 0  /* whole rays, TRACE_OPT_FWD_LANES lanes each */
+#define TRACE_FORM_STAGED 1 /* slabs staged in LDS */
+#define TRACE_FORM_SPLIT 2  /* several lanes share a ray's walk */
 
 /* Kernel phases reported by trace_phase_times. */
 #define TRACE_PHASE_FORWARD 0 /* forward projection and per-ray weights */
@@ -165,7 +180,8 @@ int trace_get_option(trace_handle_t *h, int option, int *value);
 /* Launch shape: slices per forward-projector ray (1, 2, 4, 8, 16 or 32; the
  * lanes per ray are kept when the batch has that form, else reset to 1) and the
  * backprojector's image tile (tile_w x tile_h pixels, tile_batch slices per
- * workgroup).  Only the shapes compiled into the library are accepted
+ * workgroup; one launch for the whole stack until TRACE_OPT_BACK_REST is set
+ * again).  Only the shapes compiled into the library are accepted
  * (TRACE_E_UNSUPPORTED otherwise); trace_amd.autotune picks among them.
  * No reference counterpart (the reference's work unit is fixed at one
  * sinogram row, sirt_main.cc:172). */

@@ -31,6 +31,11 @@ TRACE_OPT_FWD_LANES = 5
 TRACE_OPT_ORDERED_SUMS = 6
 TRACE_OPT_ORDERED_TILE = 7
 TRACE_OPT_FWD_STAGED = 8
+TRACE_OPT_FWD_FORM = 9
+TRACE_OPT_BACK_REST = 10
+TRACE_FORM_WHOLE = 0
+TRACE_FORM_STAGED = 1
+TRACE_FORM_SPLIT = 2
 PHASES = ("forward", "back", "update", "setup")
 
 

@@ -81,6 +81,11 @@ int forward_batch(trace_handle *h) {
   return sb;
 }
 
+int forward_form(trace_handle *h) {
+  if (forward_staged(h)) return TRACE_FORM_STAGED;
+  return split_lanes(h->geo, forward_batch(h)) ? TRACE_FORM_SPLIT : TRACE_FORM_WHOLE;
+}
+
 const char *last_error() { return g_err.c_str(); }
 void clear_error() { g_err.clear(); }
 
@@ -222,7 +227,7 @@ int backproject(trace_handle *h, int mode, const float *w, float *z, int phase) 
   if (h->backprojector == 0) {
     if (int rc = ensure_count(h)) return rc;
     const int S = mode == kBpOutSino ? h->geo.S : 1;
-    const int head = mode == kBpOutSino && h->tile_default ? head_slices(h, h->tile.sb, 256) : S;
+    const int head = mode == kBpOutSino && h->back_rest ? head_slices(h, h->tile.sb, 256) : S;
     for (int s0 = 0; s0 < S; s0 += head) {
       TileShape tile = h->tile;
       const int n = s0 == 0 ? head : S - head;
@@ -722,6 +727,10 @@ int trace_set_option(trace_handle_t *h, int option, int value) {
       if (value != 0 && value != 1) return fail(TRACE_E_INVALID, "value must be 0 or 1");
       h->fwd_staged = value;
       return TRACE_OK;
+    case TRACE_OPT_BACK_REST:
+      if (value != 0 && value != 1) return fail(TRACE_E_INVALID, "value must be 0 or 1");
+      h->back_rest = value != 0;
+      return TRACE_OK;
     default:
       return fail(TRACE_E_UNSUPPORTED, "unknown option");
   }
@@ -739,6 +748,8 @@ int trace_get_option(trace_handle_t *h, int option, int *value) {
     case TRACE_OPT_ORDERED_SUMS: *value = h->ordered; return TRACE_OK;
     case TRACE_OPT_ORDERED_TILE: *value = h->ord_tile != 0 ? 1 : 0; return TRACE_OK;
     case TRACE_OPT_FWD_STAGED: *value = h->fwd_staged != 0 ? 1 : 0; return TRACE_OK;
+    case TRACE_OPT_FWD_FORM: *value = forward_form(h); return TRACE_OK;
+    case TRACE_OPT_BACK_REST: *value = h->back_rest ? 1 : 0; return TRACE_OK;
     default: return fail(TRACE_E_UNSUPPORTED, "unknown option");
   }
 }
@@ -757,7 +768,7 @@ int trace_set_launch_shape(trace_handle_t *h, int fwd_batch, int tile_w, int til
   h->fwd_sb = fwd_batch;
   if (!fwd_shape_supported(fwd_batch, h->fwd_lanes)) h->fwd_lanes = 1;
   h->tile = TileShape{tile_w, tile_h, tile_batch};
-  h->tile_default = false;
+  h->back_rest = false;
   return TRACE_OK;
 }
 

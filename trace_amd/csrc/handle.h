@@ -112,7 +112,7 @@ struct trace_handle {
   int fwd_staged = -1;    // TRACE_OPT_FWD_STAGED: 0 or 1 as set, -1 chosen by staged_faster
   trace_hip::StagedPlan staged;  // slab plan of the staged forward projector
   trace_hip::TileShape tile{16, 16, 16};
-  bool tile_default = true;  // not set by the caller
+  bool back_rest = true;  // TRACE_OPT_BACK_REST
   trace_hip::RayInfo *rays = nullptr;     // [P][C]
   bool rays_ready = false;
   int *count = nullptr;        // [P] columns-per-tile bound for count_shape
@@ -161,6 +161,8 @@ int nbatch(int S, int sb);
 int forward_batch(trace_handle *h);
 // Whether the forward projector runs its slab-staged form.
 bool forward_staged(trace_handle *h);
+// The form it runs (TRACE_FORM_*).
+int forward_form(trace_handle *h);
 
 // Ray table and segment statistics (count, longest segment); one
 // synchronous read-back per handle.

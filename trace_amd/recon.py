@@ -191,10 +191,22 @@ class Projector:
         check(lib().trace_set_option(self._h, _capi.TRACE_OPT_ORDERED_TILE, 1 if on else 0))
 
     def set_fwd_staged(self, on: bool):
-        """Slab-staged (LDS, the default) or whole-ray form of the forward
-        projector at 32-slice batches (TRACE_OPT_FWD_STAGED; same bits either
-        way)."""
+        """Slab-staged (LDS) form of the forward projector at batches of 4, 8,
+        16 and 32 slices, or the others (TRACE_OPT_FWD_STAGED; same bits
+        either way).  Until it is set, the faster one for the geometry."""
         check(lib().trace_set_option(self._h, _capi.TRACE_OPT_FWD_STAGED, 1 if on else 0))
+
+    def set_back_rest(self, on: bool):
+        """Whether the slices past a stack's last full batch of 32 are
+        backprojected in a launch of their own where they are few
+        (TRACE_OPT_BACK_REST; same bits either way).  On until a launch shape
+        is set."""
+        check(lib().trace_set_option(self._h, _capi.TRACE_OPT_BACK_REST, 1 if on else 0))
+
+    def fwd_form(self) -> int:
+        """The form the next projection takes at the present launch shape
+        (_capi.TRACE_FORM_*)."""
+        return self.get_option(_capi.TRACE_OPT_FWD_FORM)
 
     def get_option(self, option: int) -> int:
         v = ct.c_int()
