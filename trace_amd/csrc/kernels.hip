@@ -1639,17 +1639,20 @@ int tile_splits(const Geometry &g, const TileShape &ts, int n_slices) {
   const int64_t items = (int64_t)((g.N + 15) / 16) * ((g.N + 15) / 16) * ((n_slices + ts.sb - 1) / ts.sb);
   const int64_t pairs = (int64_t)g.P * 22;  // (angle, column) pairs of a tile
   // one workgroup has two pairs a lane from 2048 on (1024 lanes; 512 at 32
-  // slices), which more than pays for adding the parts, unless these are many
-  // words (8 and 16 slices) or wait for busy CUs (past 64 items).  One workgroup /
-  // several (us) at 94, 110, 125 and 145 angles:
+  // slices), which pays for adding the parts, later where these are many words
+  // (8 and 16 slices) or wait for each other on busy CUs (many items).  One
+  // workgroup / several (us) at 94, 110, 125 and 145 angles:
   //   1 slice    90^2   24 / 22   26 / 23   31 / 23   33 / 24
   //             176^2   25 / 26   27 / 28   31 / 29   34 / 29
   //   4 slices  176^2   36 / 39   41 / 39   42 / 40   50 / 42
   //   8 slices   90^2   38 / 41   43 / 42   45 / 45   53 / 50
   //             176^2   39 / 46   44 / 47   46 / 48   54 / 49
-  //  16 slices  176^2   53 / 62   60 / 63   63 / 66   74 / 68
+  //  16 slices   90^2   52 / 55   59 / 56   62 / 56   73 / 57
+  //             176^2   53 / 62   60 / 63   63 / 66   74 / 68
   //  32 slices  176^2   78 / 76   87 / 85   93 / 88  105 / 100
-  const int64_t least = ts.sb == 8 || ts.sb == 16 ? 3072 : (ts.sb <= 4 && items > 64 ? 2560 : 2048);
+  const int64_t least = ts.sb == 8 || ts.sb == 16 ? 2100 + 8 * items
+                        : ts.sb <= 4 && items > 74 ? 1600 + 6 * items
+                                                   : 2048;
   if (items > 128 || pairs < least) return 1;
   // up to four workgroups of 256 lanes a CU, a pair for every lane, and at most
   // 32768 words for the last one to add up
