@@ -477,23 +477,39 @@ StagedLayout staged_layout(const Geometry &g, const AngleInfo *ang, int sb) {
 // A staged launch sweeps every bundle through the image however few its rays
 // are, which takes 0.5 to 1 us a pixel of the side; the other forms take their
 // segments' gathers, which cost the more the further the image outgrows the
-// caches and the fewer the angles whose rays could share lines.  Over 185
-// geometries, N from 128 to 2048 and 30 to 1500 uniform angles, the side to the
-// power 1.5 times the angles told the faster form, or one within 1% on average
-// (between 1 and 2 the power matters little).  Staged against the better of the
-// others (us):
-//               4 slices      8 slices     16 slices      32 slices
-//   256^2, 1500    237 / 258     270 / 241     392 / 444     539 / 564
-//   600^2,  250    427 / 258     469 / 345     589 / 572    1020 / 684
-//   600^2, 1000    765 / 719     848 / 797    1363 / 1532   1922 / 2186
-//   900^2,  250    634 / 700     889 / 879     905 / 1319   1559 / 1833
-//  1300^2,   60   1012 / 385     906 / 612    1241 / 957    2136 / 1988
-//  1300^2,  250   1137 / 1493   1193 / 1982   2203 / 2892   3441 / 5599
-//  2048^2,  130   1753 / 2709   2136 / 3059   3996 / 4937   7017 / 11913
-//  2048^2, 1000   6299 / 9849   7084 / 15412
+// caches and the fewer the angles whose rays could share lines.  The side to the
+// power 1.75 times the angles tells the faster form, with a least number of
+// angles (bundles of few angles sweep for few rays) and, at 4 and 8 slices, a
+// least side (smaller images stay in the L2s).  Over 277 geometries a batch, N
+// from 128 to 2048 and 30 to 1500 uniform angles, the choice lies above the
+// better form by 0.3, 0.7, 1.0 and 0.9% on average at 4, 8, 16 and 32 slices, and
+// by more than 10% in 4, 6, 11 and 10 of them (by 43% at most; what remains is the
+// grouping's steps, as between 1300^2 and 1600^2 below).  Staged / the better of
+// the others (us):
+//                4 slices      8 slices     16 slices      32 slices
+//   256^2, 1500    228 / 251     257 / 236     379 / 437     518 / 535
+//   512^2,  500    359 / 347     396 / 431     498 / 683     977 / 838
+//   600^2, 1000    736 / 708     826 / 777    1343 / 1487   1880 / 2131
+//   725^2,  720    826 / 600     904 / 975    1461 / 1726   1987 / 2462
+//   900^2,  130    604 / 362     520 / 506     682 / 764    1152 / 1434
+//   900^2,  250    617 / 683     880 / 857     867 / 1303   1513 / 1747
+//  1100^2,   90    662 / 377     883 / 623    1119 / 933    1212 / 1763
+//  1300^2,   60    998 / 368     875 / 592    1197 / 900    2038 / 1896
+//  1300^2,  250   1116 / 1474   1171 / 1953   2170 / 2839   3317 / 5445
+//  1600^2,   60   1224 / 535    1439 / 923    1350 / 1509   2296 / 2962
+//  2048^2,   60   1565 / 810    1665 / 1408   3396 / 2292   5244 / 5010
+//  2048^2,  130   1707 / 2691   2076 / 3001   3910 / 4851   6832 / 11707
 bool staged_faster(const Geometry &g, int sb) {
-  const double side = std::min(g.N, g.C);
-  return side * std::sqrt(side) * g.P >= (sb <= 8 ? 8e6 : (sb == 16 ? 2.8e6 : 4.2e6));
+  struct Limit {
+    int side, angles;
+    double work;
+  };
+  const Limit l = sb == 4    ? Limit{950, 100, 4.5e7}
+                  : sb == 8  ? Limit{512, 90, 3.75e7}
+                  : sb == 16 ? Limit{0, 70, 1.6e7}
+                             : Limit{0, 60, 1.84e7};
+  const double side = std::min(g.N, g.C), root = std::sqrt(side);
+  return side >= l.side && g.P >= l.angles && side * root * std::sqrt(root) * g.P >= l.work;
 }
 
 hipError_t launch_staged_plan(const Geometry &g, const RayInfo *rays, StagedPlan &pl,
