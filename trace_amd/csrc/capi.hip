@@ -269,10 +269,14 @@ int ensure_den(trace_handle *h) {
   float m = 0.f;
   std::memcpy(&m, &b, sizeof(m));
   // The fixed-point den is exact to far below 2^-20 relative.  The float
-  // sum in order is within (n - 1) * 2^-24 of the exact one for n terms,
-  // and a pixel takes at most 6 segments per projection (3 candidate
-  // columns, 2 segments each), so the margin covers 6 P terms.
-  const double margin = 1.0 + 0x1p-16 + (ord ? 6.0 * h->geo.P * 0x1p-24 : 0.0);
+  // sum in order is within (n - 1) * 2^-24 of the exact one for n terms.  The
+  // plain tile form files at most 6 segments of a projection in a pixel (3
+  // candidate columns, 2 segments each), the one for rays on grid lines 12 (3
+  // each, and 3 wrapped ones of another column).  A geometry that neither has
+  // the slots for is summed per pixel, with no such count; the scale leaves half
+  // of the words' range, so it would take a margin short by a factor of two.
+  const int terms = h->wraps || h->ord_tile == 2 ? 12 : 6;
+  const double margin = 1.0 + 0x1p-16 + (ord ? (double)terms * h->geo.P * 0x1p-24 : 0.0);
   h->den_max = std::isfinite(m) && m > 0.f ? (float)(m * margin) : 1.0f;
   h->den_ready = true;
   h->den_exact = h->exact;
