@@ -15,6 +15,7 @@
 #include <cstdio>
 #include <cstring>
 #include <mutex>
+#include <new>
 #include <string>
 #include <utility>
 #include <vector>
@@ -126,7 +127,12 @@ int ensure_staged(trace_handle *h) {
   if (pl.sb == sb) return TRACE_OK;
   if (int rc = ensure_rays(h)) return rc;
   const Geometry &g = h->geo;
-  const StagedLayout lay = staged_layout(g, h->ang.data(), sb);
+  StagedLayout lay;
+  try {
+    lay = staged_layout(g, h->ang.data(), sb);
+  } catch (const std::bad_alloc &) {
+    return fail(TRACE_E_NOMEM, "host memory for the staged projector's plan");
+  }
   free_staged(h);
   pl.H = lay.H;
   pl.ngroups = (int)lay.group.size();
