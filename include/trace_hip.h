@@ -334,6 +334,11 @@ void trace_batch_destroy(trace_batch_t *b);
  * allocations of the library currently live, process-wide. */
 void trace_debug_fail_alloc(int after);
 int64_t trace_debug_live_allocations(void);
+/* Compares the exact mode's square root with the correctly rounded one for
+ * the `count` floats whose bits follow `first` (none past the largest finite
+ * float) on `device`, and writes the number that differ.  Synchronous, on the
+ * null stream. */
+int trace_debug_sqrt_mismatches(int device, unsigned first, unsigned count, int64_t *differ);
 
 /* Thread-local text of the last error ("" if none). */
 const char *trace_last_error(void);

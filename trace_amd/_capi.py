@@ -145,6 +145,8 @@ _SIGS = {
     "trace_batch_destroy": (None, [_vp]),
     "trace_debug_fail_alloc": (None, [ct.c_int]),
     "trace_debug_live_allocations": (ct.c_int64, []),
+    "trace_debug_sqrt_mismatches": (ct.c_int, [ct.c_int, ct.c_uint, ct.c_uint,
+                                               ct.POINTER(ct.c_int64)]),
     "trace_last_error": (ct.c_char_p, []),
     "trace_version": (ct.c_char_p, []),
 }

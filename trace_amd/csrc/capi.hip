@@ -23,6 +23,7 @@
 #include "../../include/trace_hip.h"
 #include "handle.h"
 #include "internal.h"
+#include "traverse.h"
 
 using namespace trace_hip;
 
@@ -422,6 +423,20 @@ int scratch_address(int device, void **out) {
 
 namespace {
 
+// Floats of bits [first, first + count) whose exact-mode square root is not the
+// correctly rounded one.
+__global__ void __launch_bounds__(256)
+k_sqrt_mismatches(unsigned first, unsigned count, unsigned long long *__restrict__ differ) {
+  unsigned bad = 0;
+  const unsigned stride = gridDim.x * 256;
+  for (uint64_t i = blockIdx.x * 256 + threadIdx.x; i < count; i += stride) {
+    const float v = __uint_as_float(first + (unsigned)i);
+    bad += __float_as_uint(seg_sqrt<true>(v)) != __float_as_uint(__builtin_sqrtf(v)) ? 1u : 0u;
+  }
+  for (int off = 32; off > 0; off >>= 1) bad += __shfl_down(bad, off, 64);
+  if ((threadIdx.x & 63) == 0 && bad) atomicAdd(differ, (unsigned long long)bad);
+}
+
 constexpr float kPI = 3.14159265358979f;  // trace_utils.h:8
 
 // trace_utils.cc:41-46
@@ -540,6 +555,26 @@ const char *trace_version(void) { return "trace-hip 0.3 (gfx950)"; }
 void trace_debug_fail_alloc(int after) { g_fail_after.store(after < 0 ? -1 : after); }
 
 int64_t trace_debug_live_allocations(void) { return (int64_t)g_live_allocs.load(); }
+
+int trace_debug_sqrt_mismatches(int device, unsigned first, unsigned count, int64_t *differ) {
+  g_err.clear();
+  if (!differ) return fail(TRACE_E_INVALID, "null argument");
+  if (count == 0 || first > 0x7f7fffffu || count - 1 > 0x7f7fffffu - first)
+    return fail(TRACE_E_INVALID, "floats past the largest finite one");
+  HIP_TRY(hipSetDevice(device));
+  unsigned long long *d = nullptr, n = 0;
+  HIP_TRY(dev_alloc(&d, 1));
+  hipError_t e = launch_fill(reinterpret_cast<float *>(d), 2, 0.f, nullptr);
+  if (e == hipSuccess) {
+    hipLaunchKernelGGL(k_sqrt_mismatches, dim3(2048), dim3(256), 0, nullptr, first, count, d);
+    e = hipGetLastError();
+  }
+  if (e == hipSuccess) e = hipMemcpy(&n, d, sizeof(n), hipMemcpyDeviceToHost);
+  dev_free(d);
+  if (e != hipSuccess) return fail(TRACE_E_HIP, std::string("comparison: ") + hipGetErrorString(e));
+  *differ = (int64_t)n;
+  return TRACE_OK;
+}
 
 void trace_deg2rad(const float *deg, float *rad, int n) {
   // trace_utils.cc:22: float product, double division, float result

@@ -78,15 +78,15 @@ __device__ __forceinline__ float grid_line(int N, int n) {
 
 // Segment length from its square.  The exact form is the correctly rounded
 // square root: v_rsq_f32, one product and one residual correction, equal to
-// the IEEE square root for every float >= 2^-96 (compared over all of them on
-// the GPU) and for 0 (the clamp keeps the reciprocal root finite).  It issues
-// 6 instructions where the general expansion, with its scaling of tiny
-// arguments, issues 18.  A squared length between 0 and 2^-96 would need a
-// crossing within 2^-48 of a grid line without lying on it, which floats
-// allow at the line 0 only, and there only for a ray whose source point has a
-// coordinate below 2^-24 (an angle between 0 and 6e-14 rad and a column
-// through the axis); such a length is off in its last places, or 0 below
-// 2^-60.
+// the IEEE square root for every float from 2^-96 on and for 0, where the clamp
+// keeps the reciprocal root finite (trace_debug_sqrt_mismatches compares them
+// all on the GPU; tests/test_gpu_sqrt.py).  It issues 6 instructions where the
+// general expansion, with its scaling of tiny arguments, issues 18.  Below 2^-96
+// the result is too small, by 31% at 2^-98 and 63% at 2^-100, and tends to 1.5 v
+// 2^48 (less than 2^-48 off in all).  Such a square would need a crossing within
+// 2^-48 of a grid line without lying on it, which floats allow at the line 0
+// only, and there only for a ray whose source point has a coordinate below 2^-24
+// (an angle between 0 and 6e-14 rad and a column through the axis).
 template <bool kExactSqrt>
 __device__ __forceinline__ float seg_sqrt(float v) {
   if constexpr (kExactSqrt) {
