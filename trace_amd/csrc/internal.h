@@ -101,9 +101,9 @@ struct RegParams {
 int tile_count_bound(float sinq, float cosq, int TW, int TH);
 
 // Launchers (kernels.hip).  All are asynchronous on `st`.
-// Ray table; `flags` adds the window flags (kRayWhole, kRayWraps, kRay1D)
-// from one walk per ray, which the tile kernels need and whole-ray walks
-// do not.
+// Ray table; with `counts` ([4], zeroed) also the rays' flags (kRayWhole,
+// kRayWraps, kRay1D, kRayHits) and the geometry's segment statistics, from one
+// walk per ray.  The walks of trace_forward_noalloc need neither.
 hipError_t launch_ray_info(const Geometry &g, RayInfo *rays, unsigned long long *counts,
                            hipStream_t st);
 hipError_t launch_forward(const Geometry &g, const RayInfo *rays, int sb, int bundle_angles,
@@ -204,8 +204,8 @@ struct TileSplit {
 int tile_splits(const Geometry &g, const TileShape &ts, int n_slices);
 size_t tile_split_words(const Geometry &g, const TileShape &ts, int n_slices, int splits);
 
-// Slices [s0, s0 + n) of the stack (s0 = 0, n = 1 for column sums and counts).
-
+// Slices [s0, s0 + n) of the stack (s0 = 0, n = 1 for column sums and counts);
+// split: tiles of these slices shared among workgroups (ensure_split).
 hipError_t launch_backproject(const Geometry &g, const RayInfo *rays, const int *count,
                               const TileShape &ts, int mode, bool exact, const float *w,
                               const unsigned *maxw, float maxlen, float denmax, float *z,

@@ -104,23 +104,6 @@ struct Vec {
 };
 
 template <int SB>
-__device__ __forceinline__ void load_slices(const float *__restrict__ p, float (&o)[SB]) {
-  static_assert(SB == 1 || SB == 2 || SB % 4 == 0, "slice batch: 1, 2 or a multiple of 4");
-  if constexpr (SB == 1) {
-    o[0] = p[0];
-  } else if constexpr (SB == 2) {
-    const float2 q = *reinterpret_cast<const float2 *>(p);
-    o[0] = q.x; o[1] = q.y;
-  } else {
-#pragma unroll
-    for (int k = 0; k < SB; k += 4) {
-      const float4 q = *reinterpret_cast<const float4 *>(p + k);
-      o[k] = q.x; o[k + 1] = q.y; o[k + 2] = q.z; o[k + 3] = q.w;
-    }
-  }
-}
-
-template <int SB>
 __device__ __forceinline__ void store_slices(float *__restrict__ p, const float (&v)[SB]) {
   if constexpr (SB == 1) {
     p[0] = v[0];
