@@ -1,0 +1,40 @@
+"""Ordered sums with rays on grid lines where the tile form serves only some of
+the sums: column sums pixel by pixel and num in tiles (checked for slots when it
+first runs), the reverse, and both either way.  The same bits as with every sum
+pixel by pixel, on the first call and after it."""
+import numpy as np
+import pytest
+
+from trace_amd.phantom import angles_rad
+
+pytestmark = pytest.mark.gpu
+
+CASES = [  # N, P (two of them along the axes), slices
+    (140, 2, 1), (140, 2, 2), (140, 2, 13),  # column sums per pixel, num in tiles
+    (150, 2, 20), (150, 2, 40),
+    (490, 120, 3),                           # column sums in tiles, num per pixel
+    (200, 2, 4), (300, 30, 7)]
+
+
+@pytest.mark.parametrize("alg", ["pml", "apmlr", "mlem"])
+@pytest.mark.parametrize("N,P,S", CASES)
+def test_grid_rays_mixed_forms(gpu, alg, N, P, S):
+    import torch
+    from trace_amd import Projector
+    th = angles_rad(P)
+    rng = np.random.default_rng(N + S)
+    sino = torch.from_numpy(rng.uniform(0.5, 2.0, (P, S, N)).astype(np.float32)).to("cuda:0")
+    out = []
+    for tile in (True, False):
+        with Projector(th, S, N, N / 2.0 + 0.5, device=0) as pj:
+            pj.set_ordered_tile(tile)
+            if alg == "mlem":
+                pj.set_ordered_sums(2)
+            got = []
+            for _ in range(2):
+                x = torch.ones((S, N, N), device="cuda:0")
+                pj.reconstruct(alg, 2, sino, x)
+                got += [x.cpu().numpy(), pj.column_sums().cpu().numpy()]
+        out.append(got)
+    for a, b in zip(*out):
+        assert np.array_equal(a.view(np.int32), b.view(np.int32))

@@ -282,7 +282,7 @@ int ensure_den(trace_handle *h) {
   // each, and 3 wrapped ones of another column).  A geometry that neither has
   // the slots for is summed per pixel, with no such count; the scale leaves half
   // of the words' range, so it would take a margin short by a factor of two.
-  const int terms = h->wraps || h->ord_tile == 2 ? 12 : 6;
+  const int terms = h->wraps || h->ord_tile >= 2 ? 12 : 6;
   const double margin = 1.0 + 0x1p-16 + (ord ? (double)terms * h->geo.P * 0x1p-24 : 0.0);
   h->den_max = std::isfinite(m) && m > 0.f ? (float)(m * margin) : 1.0f;
   h->den_ready = true;
@@ -302,6 +302,19 @@ static int ordered_batch(int mode, int S, int xsb, bool tile) {
   return sb;
 }
 
+// Clears the tile forms' overflow flag, or reads it back.
+static int clear_overflow(trace_handle *h) {
+  HIP_TRY(hipMemsetAsync(h->flag, 0, sizeof(int), h->stream));
+  return TRACE_OK;
+}
+static int read_overflow(trace_handle *h, bool &overflow) {
+  int f = 0;
+  HIP_TRY(hipMemcpyAsync(&f, h->flag, sizeof(f), hipMemcpyDeviceToHost, h->stream));
+  HIP_TRY(hipStreamSynchronize(h->stream));
+  overflow = f != 0;
+  return TRACE_OK;
+}
+
 int ordered_den(trace_handle *h, float *out) {
   if (int rc = ensure_rays(h)) return rc;
   unsigned *ovf = reinterpret_cast<unsigned *>(h->flag);
@@ -309,28 +322,28 @@ int ordered_den(trace_handle *h, float *out) {
     return launch_bp_ordered(h->geo, h->rays, kOrdDen, h->exact, nullptr, nullptr, 1, 1, out,
                              h->wraps, form > 0 ? ovf : nullptr, form == 2, 0, 1, h->stream);
   };
-  // decided before; or undecided where nothing can be read back: the form that
-  // always serves
-  if (h->ord_tile >= 0 || capturing(h)) {
-    TIMED(TRACE_PHASE_SETUP, launch(h->ord_tile < 0 ? 0 : h->ord_tile));
-    return TRACE_OK;
-  }
-  // the plain tile form, the one for rays on grid lines, the per-pixel form: the
-  // first that has the slots
-  for (int form = h->wraps ? 2 : 1; form <= 2; ++form) {
-    if (form == 2 && !ordered_grid_rays_fit(h->geo.N)) break;
-    HIP_TRY(hipMemsetAsync(ovf, 0, sizeof(unsigned), h->stream));
-    TIMED(TRACE_PHASE_SETUP, launch(form));
-    unsigned f = 0;
-    HIP_TRY(hipMemcpyAsync(&f, ovf, sizeof(f), hipMemcpyDeviceToHost, h->stream));
-    HIP_TRY(hipStreamSynchronize(h->stream));
-    if (!f) {
-      h->ord_tile = form;
-      return TRACE_OK;
+  const bool grid = ordered_grid_pays(h->geo.N, h->geo.P, kOrdDen, 1);
+  // The plain tile form, the one for rays on grid lines (where it pays), the
+  // per-pixel form: the first that has the slots.  Where nothing can be read
+  // back, an undecided geometry takes the form that always serves.
+  if ((h->ord_tile < 0 || h->ord_tile == 3) && !capturing(h)) {
+    int left = 3;  // what stays to be tried, 0 nothing
+    for (int form = h->wraps || h->ord_tile == 3 ? 2 : 1; form <= 2; ++form) {
+      if (form == 2 && !grid) break;
+      bool overflow = false;
+      if (int rc = clear_overflow(h)) return rc;
+      TIMED(TRACE_PHASE_SETUP, launch(form));
+      if (int rc = read_overflow(h, overflow)) return rc;
+      if (!overflow) {
+        h->ord_tile = form;
+        return TRACE_OK;
+      }
+      if (form == 2) left = 0;
     }
+    h->ord_tile = left;
   }
-  h->ord_tile = 0;
-  TIMED(TRACE_PHASE_SETUP, launch(0));
+  const bool tile = h->ord_tile == 1 || (h->ord_tile == 2 && grid);
+  TIMED(TRACE_PHASE_SETUP, launch(tile ? h->ord_tile : 0));
   return TRACE_OK;
 }
 
@@ -339,16 +352,28 @@ int backproject_ordered(trace_handle *h, int mode, const float *w, float *z, int
   if (h->ord_tile < 0)  // decided by the den pass (same walks, same slots)
     if (int rc = ordered_den(h, h->z)) return rc;
   if (mode == kOrdNum && !h->xb) return fail(TRACE_E_INVALID, "no slice-batched image copy");
-  const bool tile = h->ord_tile >= 1;
-  const int sb = ordered_batch(mode, h->geo.S, h->xb_sb, tile);
-  // the tile form's overflow flag was checked on this geometry by the den pass
+  int sb = ordered_batch(mode, h->geo.S, h->xb_sb, true);
+  bool tile = h->ord_tile == 1;
+  if (h->ord_tile >= 2) tile = ordered_grid_pays(h->geo.N, h->geo.P, mode, sb);
+  // untried by the den pass, which the per-pixel form served: checked here
+  const bool check = tile && h->ord_tile == 3;
+  if (h->ord_tile < 0 || (check && capturing(h))) tile = false;
+  if (!tile) sb = ordered_batch(mode, h->geo.S, h->xb_sb, false);
   unsigned *ovf = tile ? reinterpret_cast<unsigned *>(h->flag) : nullptr;
+  if (tile && check)
+    if (int rc = clear_overflow(h)) return rc;
   const int S = h->geo.S, head = head_slices(h, sb, 400);
   for (int s0 = 0; s0 < S; s0 += head) {
     const int n = s0 == 0 ? head : S - head;
     TIMED(phase, launch_bp_ordered(h->geo, h->rays, mode, h->exact, w, h->xb, h->xb_sb,
                                    head < S ? batch_for(n) : sb, z, h->wraps, ovf,
-                                   h->ord_tile == 2, s0, n, h->stream));
+                                   tile && h->ord_tile >= 2, s0, n, h->stream));
+  }
+  if (tile && check) {
+    bool overflow = false;
+    if (int rc = read_overflow(h, overflow)) return rc;
+    h->ord_tile = overflow ? 0 : 2;
+    if (overflow) return backproject_ordered(h, mode, w, z, phase);
   }
   return TRACE_OK;
 }

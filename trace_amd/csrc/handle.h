@@ -123,7 +123,8 @@ struct trace_handle {
   bool den_ordered = false;    // den summed in the reference's order
   int ordered = 1;             // TRACE_OPT_ORDERED_SUMS
   int ord_tile = -1;           // tile form of the ordered sums: -1 untried, 0 not
-                               // usable, 1 usable, 2 usable for rays on grid lines
+                               // usable, 1 usable, 2 usable for rays on grid lines,
+                               // 3 only that one can be and is untried
   float *xb = nullptr;         // [ceil(S/fwd_sb)][N][N][fwd_sb]
   int xb_sb = 0;
   float *w = nullptr;          // [P][C][S] per-ray weights

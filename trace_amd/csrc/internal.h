@@ -177,8 +177,9 @@ hipError_t launch_bp_ordered(const Geometry &g, const RayInfo *rays, int mode, b
                              bool wraps, unsigned *tile_overflow, bool grid_rays,
                              int s0, int n, hipStream_t st);
 bool ordered_sb_supported(int mode, int sb, int xsb);
-// Whether an image's side allows the tile form for rays on grid lines.
-bool ordered_grid_rays_fit(int N);
+// Whether the tile form for rays on grid lines serves a launch (sb slices a
+// workgroup), and faster than the per-pixel form.
+bool ordered_grid_pays(int N, int P, int mode, int sb);
 
 // Forward projection with `lanes` lanes per ray (split.hip): sb slices to a
 // slot of xb.  split_lanes: how many a launch should take, 0 for the whole-ray

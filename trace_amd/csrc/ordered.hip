@@ -831,11 +831,30 @@ int ordered_waves(int N, int S, int sb, bool grid_rays) {
   return tiles <= 128 ? 8 : (tiles <= (sb == 32 ? 3000 : 1536) ? 4 : 1);
 }
 
-// A launch holds fewer than 2^32 lanes: four wavefronts a tile reach that from
-// 32761^2 on, where geometries with rays on grid lines keep the per-pixel form.
-bool ordered_grid_rays_fit(int N) {
+// Whether rays on grid lines are served faster by the tile form than pixel by
+// pixel.  Such a ray is walked whole in every tile it touches, which grows with
+// the cube of the side and not with the angles; the per-pixel form walks it once
+// a strip.  Tile / per-pixel form (ms), axis on a grid line, angles 120, 360, 900:
+//              column sums                    num of 1 or 2 slices
+//    512^2   1.1 / 2.3  2.2 / 6.4  4.5 / 15   1.1 / 1.6  2.2 / 4.2  4.7 / 10
+//    640^2   1.9 / 1.5  3.5 / 4.0  7.3 / 9.5  1.9 / 1.8  3.6 / 4.7  7.5 / 11
+//    900^2   4.4 / 2.7  7.7 / 6.8   15 / 16   4.5 / 3.3  7.8 / 8.4   15 / 19
+//   1200^2   9.2 / 3.0   15 / 7.3   28 / 17   9.3 / 5.6   15 / 13    28 / 31
+//   2048^2    39 / 9.8   55 / 19              39 / 20     56 / 42
+//              num of 4 or 8                  num of 32
+//    384^2   1.1 / 1.5  2.2 / 4.1  4.9 / 10   1.2 / 3.2  2.7 / 9.6  6.0 / 23
+//    512^2   2.1 / 1.7  4.2 / 4.4  8.9 / 11   2.4 / 5.1  5.0 / 15    11 / 36
+//    640^2   3.5 / 1.8  6.8 / 4.7   14 / 11   4.1 / 6.5  8.2 / 19    17 / 47
+//   2048^2    73 / 19   106 / 42              81 / 80    122 / 190
+// (16 slices as 1.)  A launch also holds fewer than 2^32 lanes, which four
+// wavefronts a tile reach at 32761^2.
+bool ordered_grid_pays(int N, int P, int mode, int sb) {
   const int64_t side = (N + kOT - 1) / kOT;
-  return side * side * kOWave * ordered_waves(N, 1, 1, true) < (int64_t(1) << 32);
+  if (side * side * kOWave * ordered_waves(N, 1, 1, true) >= (int64_t(1) << 32)) return false;
+  const double cube = (double)N * N * N / P;
+  if (mode == kOrdDen) return cube <= 1.3e6;
+  if (sb == 4 || sb == 8) return N <= 560 && cube <= 9e5;
+  return cube <= (sb == 32 ? 6.5e7 : 3e6);
 }
 
 bool ordered_sb_supported(int mode, int sb, int xsb) {
