@@ -10,10 +10,10 @@ from trace_amd.phantom import angles_rad
 pytestmark = pytest.mark.gpu
 
 CASES = [  # N, P (two of them along the axes), slices
-    (140, 2, 1), (140, 2, 2), (140, 2, 13),  # column sums per pixel, num in tiles
-    (150, 2, 20), (150, 2, 40),
-    (490, 120, 3),                           # column sums in tiles, num per pixel
-    (200, 2, 4), (300, 30, 7)]
+    (140, 2, 1), (140, 2, 2), (140, 2, 13), (150, 2, 20), (150, 2, 40), (490, 120, 3),
+    (200, 2, 4), (300, 30, 7),
+    (700, 60, 20), (700, 60, 40), (1000, 400, 1),  # column sums per pixel, num in tiles
+    (560, 60, 3)]                                  # column sums in tiles, num per pixel
 
 
 @pytest.mark.parametrize("alg", ["pml", "apmlr", "mlem"])

@@ -54,6 +54,8 @@
 // trips a segment, the column sums of 2048^2 / 1500 took 45.3 ms instead of 37.1.
 #include <hip/hip_runtime.h>
 
+#include <cmath>
+
 #include "internal.h"
 
 #pragma clang fp contract(off)
@@ -832,9 +834,13 @@ int ordered_waves(int N, int S, int sb, bool grid_rays) {
 }
 
 // Whether rays on grid lines are served faster by the tile form than pixel by
-// pixel.  Such a ray is walked whole in every tile it touches, which grows with
-// the cube of the side and not with the angles; the per-pixel form walks it once
-// a strip.  Tile / per-pixel form (ms), axis on a grid line, angles 120, 360, 900:
+// pixel.  Such a ray is walked whole in every tile it touches, which costs some
+// N^3 however many the angles (`fixed`, what the per-pixel form spends on it taken
+// off); an angle costs `tile` N^2 in tiles, and in the per-pixel form `pixel` N^2
+// or, where its strips do not fill the GPU, the walks of one (`least`).  In us,
+// fitted to ten sides at 120, 360 and 900 angles: where the two forms differ by
+// more than 5% the faster is chosen in all but one of 196 cases.  Tile /
+// per-pixel form (ms), axis on a grid line, angles 120, 360, 900:
 //              column sums                    num of 1 or 2 slices
 //    512^2   1.1 / 2.3  2.2 / 6.4  4.5 / 15   1.1 / 1.6  2.2 / 4.2  4.7 / 10
 //    640^2   1.9 / 1.5  3.5 / 4.0  7.3 / 9.5  1.9 / 1.8  3.6 / 4.7  7.5 / 11
@@ -846,15 +852,21 @@ int ordered_waves(int N, int S, int sb, bool grid_rays) {
 //    512^2   2.1 / 1.7  4.2 / 4.4  8.9 / 11   2.4 / 5.1  5.0 / 15    11 / 36
 //    640^2   3.5 / 1.8  6.8 / 4.7   14 / 11   4.1 / 6.5  8.2 / 19    17 / 47
 //   2048^2    73 / 19   106 / 42              81 / 80    122 / 190
-// (16 slices as 1.)  A launch also holds fewer than 2^32 lanes, which four
-// wavefronts a tile reach at 32761^2.
+// A launch also holds fewer than 2^32 lanes, which four wavefronts a tile reach
+// at 32761^2.
 bool ordered_grid_pays(int N, int P, int mode, int sb) {
   const int64_t side = (N + kOT - 1) / kOT;
   if (side * side * kOWave * ordered_waves(N, 1, 1, true) >= (int64_t(1) << 32)) return false;
-  const double cube = (double)N * N * N / P;
-  if (mode == kOrdDen) return cube <= 1.3e6;
-  if (sb == 4 || sb == 8) return N <= 560 && cube <= 9e5;
-  return cube <= (sb == 32 ? 6.5e7 : 3e6);
+  struct Cost {
+    double fixed, least, pixel, tile;
+  };
+  const Cost c = mode == kOrdDen ? Cost{3.7e-6, 18, 1.9e-5, 1.65e-5}
+                 : sb <= 2       ? Cost{3.0e-6, 8, 2.7e-5, 1.73e-5}
+                 : sb <= 8       ? Cost{5.9e-6, 12, 2.86e-5, 3.33e-5}
+                 : sb == 16      ? Cost{6.0e-6, 18, 5.4e-5, 3.48e-5}
+                                 : Cost{4.2e-6, 30, 1.095e-4, 4.08e-5};
+  const double n2 = (double)N * N;
+  return c.fixed * n2 * N <= P * (std::fmax(c.least, c.pixel * n2) - c.tile * n2);
 }
 
 bool ordered_sb_supported(int mode, int sb, int xsb) {
