@@ -641,7 +641,8 @@ int trace_create(trace_handle_t **out, const trace_geom_t *g, int device,
   // 1500 angles; trace_amd.autotune refines it for a given geometry)
   const int S = g->num_slices;
   const int n = g->num_grids;
-  // backprojector: the stack in one batch up to 32 slices.  A 32x32 tile's
+  // backprojector: the stack in one batch up to 32 slices, but for a few angles'
+  // small stacks.  A 32x32 tile's
   // pairs serve more segments for their set-up than a 16x16 tile's, but it
   // pays only where the tiles fill the 256 CUs once, nearly, or a few times;
   // the deeper the batch (LDS and registers then hold fewer workgroups) the
@@ -655,7 +656,12 @@ int trace_create(trace_handle_t **out, const trace_geom_t *g, int device,
   //   64 slices  2048^2, in batches of 32 82.9 ms, of 16 in 32x32 95.9 ms
   const double fill = (double)((n + 31) / 32) * ((n + 31) / 32) / 256;
   const bool once = fill >= 0.75 && fill <= 1.0;
-  if (S > 16) {
+  if (S > 8 && S <= 32 && g->num_projs <= 12 && n <= 400) {
+    // a pair a lane, and few tiles: a shallower batch adds less after each walk
+    // (9 / 31 slices at 8 angles, 8 slices a tile and 16 or 32 (us): 64^2 17 / 23,
+    // 17 / 29; 400^2 34 / 43, 43 / 68)
+    h->tile = TileShape{16, 16, 8};
+  } else if (S > 16) {
     h->tile = TileShape{16, 16, 32};
   } else if (S > 8) {
     const int side = once ? 32 : 16;
