@@ -12,7 +12,8 @@ pytestmark = pytest.mark.gpu
 CASES = [  # N, P (two of them along the axes), slices
     (140, 2, 1), (140, 2, 2), (140, 2, 13), (150, 2, 20), (150, 2, 40), (490, 120, 3),
     (200, 2, 4), (300, 30, 7),
-    (700, 60, 20), (700, 60, 40), (1000, 400, 1),  # column sums per pixel, num in tiles
+    (700, 60, 20), (700, 60, 40),
+    (700, 60, 30), (1000, 400, 1),           # column sums per pixel, num in tiles
     (560, 60, 3)]                                  # column sums in tiles, num per pixel
 
 

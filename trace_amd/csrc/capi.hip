@@ -107,14 +107,15 @@ static void free_staged(trace_handle *h) {
 int ensure_rays(trace_handle *h) {
   if (h->rays_ready) return TRACE_OK;
   if (!h->rays) HIP_TRY(dev_alloc(&h->rays, (size_t)h->geo.rays_per_slice()));
-  HIP_TRY(hipMemsetAsync(h->counters, 0, 4 * sizeof(unsigned long long), h->stream));
+  HIP_TRY(hipMemsetAsync(h->counters, 0, 5 * sizeof(unsigned long long), h->stream));
   TIMED(TRACE_PHASE_SETUP, launch_ray_info(h->geo, h->rays, h->counters, h->stream));
-  unsigned long long c[4] = {0, 0, 0, 0};
+  unsigned long long c[5] = {};
   HIP_TRY(hipMemcpyAsync(c, h->counters, sizeof(c), hipMemcpyDeviceToHost, h->stream));
   HIP_TRY(hipStreamSynchronize(h->stream));
   h->nnz = (int64_t)c[0];
   h->nnz_oor = (int64_t)c[1];
   h->wraps = c[3] > 0;
+  h->whole_rays = (int64_t)c[4];
   const unsigned bits = (unsigned)c[2];
   std::memcpy(&h->maxlen, &bits, sizeof(float));
   h->rays_ready = true;
@@ -322,7 +323,7 @@ int ordered_den(trace_handle *h, float *out) {
     return launch_bp_ordered(h->geo, h->rays, kOrdDen, h->exact, nullptr, nullptr, 1, 1, out,
                              h->wraps, form > 0 ? ovf : nullptr, form == 2, 0, 1, h->stream);
   };
-  const bool grid = ordered_grid_pays(h->geo.N, h->geo.P, kOrdDen, 1);
+  const bool grid = ordered_grid_pays(h->geo.N, h->geo.P, h->whole_rays, 1, kOrdDen, 1);
   // The plain tile form, the one for rays on grid lines (where it pays), the
   // per-pixel form: the first that has the slots.  Where nothing can be read
   // back, an undecided geometry takes the form that always serves.
@@ -354,7 +355,8 @@ int backproject_ordered(trace_handle *h, int mode, const float *w, float *z, int
   if (mode == kOrdNum && !h->xb) return fail(TRACE_E_INVALID, "no slice-batched image copy");
   int sb = ordered_batch(mode, h->geo.S, h->xb_sb, true);
   bool tile = h->ord_tile == 1;
-  if (h->ord_tile >= 2) tile = ordered_grid_pays(h->geo.N, h->geo.P, mode, sb);
+  if (h->ord_tile >= 2) 
+    tile = ordered_grid_pays(h->geo.N, h->geo.P, h->whole_rays, h->geo.S, mode, sb);
   // untried by the den pass, which the per-pixel form served: checked here
   const bool check = tile && h->ord_tile == 3;
   if (h->ord_tile < 0 || (check && capturing(h))) tile = false;
@@ -733,7 +735,7 @@ int trace_create(trace_handle_t **out, const trace_geom_t *g, int device,
       (e = dev_alloc(&geo.d_yi, (size_t)geo.C)) != hipSuccess ||
       (e = dev_alloc(&h->den, (size_t)geo.NN())) != hipSuccess ||
       (e = dev_alloc(&h->flag, 1)) != hipSuccess ||
-      (e = dev_alloc(&h->counters, 4)) != hipSuccess)
+      (e = dev_alloc(&h->counters, 5)) != hipSuccess)
     return cleanup_fail(fail(e == hipErrorOutOfMemory ? TRACE_E_NOMEM : TRACE_E_HIP,
                              std::string("allocation: ") + hipGetErrorString(e)));
   if ((e = hipMemcpy(geo.d_ang, h->ang.data(), h->ang.size() * sizeof(AngleInfo),

@@ -132,14 +132,15 @@ struct trace_handle {
   float *xa = nullptr;         // [S+2][N][N] work image (PML/APMLR)
   float *xc = nullptr;         // [S+2][N][N]
   int *flag = nullptr;
-  unsigned long long *counters = nullptr;  // [4]: segments, outside image, max length bits,
-                                           // rays with a segment at ix == N
+  unsigned long long *counters = nullptr;  // [5]: segments, outside image, max length bits,
+                                           // rays with a segment at ix == N, rays walked whole
   unsigned *maxw = nullptr;    // [S] bits of max |w| per slice
   unsigned *split = nullptr;   // tickets and partial tiles (ensure_split)
   size_t split_words = 0;
   float maxlen = 0.f;          // longest segment of the geometry
   float den_max = 0.f;         // bound on the sum of segment lengths per pixel
   int64_t nnz = 0, nnz_oor = 0;
+  int64_t whole_rays = 0;  // rays that the tile kernels walk whole
   bool wraps = false;  // some ray has a segment with ix == N (the tile pass for it runs)
   trace_hip::PhaseTimer timer;
 };

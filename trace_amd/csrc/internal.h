@@ -101,7 +101,7 @@ struct RegParams {
 int tile_count_bound(float sinq, float cosq, int TW, int TH);
 
 // Launchers (kernels.hip).  All are asynchronous on `st`.
-// Ray table; with `counts` ([4], zeroed) also the rays' flags (kRayWhole,
+// Ray table; with `counts` ([5], zeroed) also the rays' flags (kRayWhole,
 // kRayWraps, kRay1D, kRayHits) and the geometry's segment statistics, from one
 // walk per ray.  The walks of trace_forward_noalloc need neither.
 hipError_t launch_ray_info(const Geometry &g, RayInfo *rays, unsigned long long *counts,
@@ -177,9 +177,10 @@ hipError_t launch_bp_ordered(const Geometry &g, const RayInfo *rays, int mode, b
                              bool wraps, unsigned *tile_overflow, bool grid_rays,
                              int s0, int n, hipStream_t st);
 bool ordered_sb_supported(int mode, int sb, int xsb);
-// Whether the tile form for rays on grid lines serves a launch (sb slices a
-// workgroup), and faster than the per-pixel form.
-bool ordered_grid_pays(int N, int P, int mode, int sb);
+// Whether the tile form for rays on grid lines serves the sums of S slices (sb a
+// workgroup), and faster than the per-pixel form, when `whole` rays are walked
+// whole.
+bool ordered_grid_pays(int N, int P, int64_t whole, int S, int mode, int sb);
 
 // Forward projection with `lanes` lanes per ray (split.hip): sb slices to a
 // slot of xb.  split_lanes: how many a launch should take, 0 for the whole-ray

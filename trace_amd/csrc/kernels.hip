@@ -49,7 +49,8 @@ __device__ __forceinline__ void atomic_add_f32(float *p, float v) {
 
 // Ray table.  With `counts` also the rays' flags and the geometry's segment
 // statistics, from one walk of each ray: all segments, those outside the image,
-// the bits of the longest, and the rays with a wrapped one (zeroed beforehand).
+// the bits of the longest, the rays with a wrapped one and those walked whole
+// by the tile kernels (zeroed beforehand).
 // Whole-ray walks (the forward projector) read neither.
 __global__ void __launch_bounds__(kRayBlock)
 k_ray_info(GridInfo g, const AngleInfo *__restrict__ ang, const float *__restrict__ yi,
@@ -57,32 +58,35 @@ k_ray_info(GridInfo g, const AngleInfo *__restrict__ ang, const float *__restric
   const int64_t t = (int64_t)blockIdx.x * kRayBlock + threadIdx.x;
   const bool valid = t < (int64_t)P * g.C;
   RayStats st;
-  unsigned wraps = 0;
+  unsigned wraps = 0, whole = 0;
   if (valid) {
     const int c = (int)(t % g.C), p = (int)(t / g.C);
     RayInfo r = make_ray(g, yi[c], ang[p].sinq, ang[p].cosq);
     if (counts) {
       r.alo |= ray_flags(g, r, ang[p].quadrant, st);
       wraps = (r.alo & kRayWraps) ? 1u : 0u;
+      whole = st.whole ? 1u : 0u;
     }
     rays[t] = r;
   }
   if (!counts) return;
-  __shared__ unsigned s_sum[3], s_longest;
-  if (threadIdx.x < 3) s_sum[threadIdx.x] = 0;
-  if (threadIdx.x == 3) s_longest = 0;
+  __shared__ unsigned s_sum[4], s_longest;
+  if (threadIdx.x < 4) s_sum[threadIdx.x] = 0;
+  if (threadIdx.x == 4) s_longest = 0;
   __syncthreads();
   unsigned lb = __float_as_uint(st.longest);
   for (int off = 32; off > 0; off >>= 1) {
     st.segments += __shfl_down(st.segments, off, 64);
     st.outside += __shfl_down(st.outside, off, 64);
     wraps += __shfl_down(wraps, off, 64);
+    whole += __shfl_down(whole, off, 64);
     lb = max(lb, (unsigned)__shfl_down((int)lb, off, 64));
   }
   if ((threadIdx.x & 63) == 0) {
     atomicAdd(s_sum + 0, st.segments);
     atomicAdd(s_sum + 1, st.outside);
     atomicAdd(s_sum + 2, wraps);
+    atomicAdd(s_sum + 3, whole);
     atomicMax(&s_longest, lb);
   }
   __syncthreads();
@@ -91,6 +95,7 @@ k_ray_info(GridInfo g, const AngleInfo *__restrict__ ang, const float *__restric
     if (s_sum[1]) atomicAdd(counts + 1, (unsigned long long)s_sum[1]);
     raise_max(reinterpret_cast<unsigned *>(counts + 2), s_longest);
     if (s_sum[2]) atomicAdd(counts + 3, (unsigned long long)s_sum[2]);
+    if (s_sum[3]) atomicAdd(counts + 4, (unsigned long long)s_sum[3]);
   }
 }
 

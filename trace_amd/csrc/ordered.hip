@@ -834,13 +834,14 @@ int ordered_waves(int N, int S, int sb, bool grid_rays) {
 }
 
 // Whether rays on grid lines are served faster by the tile form than pixel by
-// pixel.  Such a ray is walked whole in every tile it touches, which costs some
-// N^3 however many the angles (`fixed`, what the per-pixel form spends on it taken
-// off); an angle costs `tile` N^2 in tiles, and in the per-pixel form `pixel` N^2
-// or, where its strips do not fill the GPU, the walks of one (`least`).  In us,
+// pixel.  Such a ray is walked whole in every tile it touches, which costs N^2 a
+// ray (a tenth to a fifth of it in the per-pixel form, whose threads walk it side
+// by side), and so do rays whose lists are not sorted; an angle costs N^2 in tiles,
+// and in the per-pixel form N^2 or, where its strips do not fill the GPU, the walks
+// of one (`least`).  Costs in us of a batch: sb slices in tiles, up to 8 per pixel,
 // fitted to ten sides at 120, 360 and 900 angles: where the two forms differ by
 // more than 5% the faster is chosen in all but one of 196 cases.  Tile /
-// per-pixel form (ms), axis on a grid line, angles 120, 360, 900:
+// per-pixel form (ms), one angle's rays on grid lines, angles 120, 360, 900:
 //              column sums                    num of 1 or 2 slices
 //    512^2   1.1 / 2.3  2.2 / 6.4  4.5 / 15   1.1 / 1.6  2.2 / 4.2  4.7 / 10
 //    640^2   1.9 / 1.5  3.5 / 4.0  7.3 / 9.5  1.9 / 1.8  3.6 / 4.7  7.5 / 11
@@ -854,19 +855,21 @@ int ordered_waves(int N, int S, int sb, bool grid_rays) {
 //   2048^2    73 / 19   106 / 42              81 / 80    122 / 190
 // A launch also holds fewer than 2^32 lanes, which four wavefronts a tile reach
 // at 32761^2.
-bool ordered_grid_pays(int N, int P, int mode, int sb) {
+bool ordered_grid_pays(int N, int P, int64_t whole, int S, int mode, int sb) {
   const int64_t side = (N + kOT - 1) / kOT;
   if (side * side * kOWave * ordered_waves(N, 1, 1, true) >= (int64_t(1) << 32)) return false;
   struct Cost {
-    double fixed, least, pixel, tile;
+    double tile_ray, tile, pixel_ray, pixel, least;
   };
-  const Cost c = mode == kOrdDen ? Cost{3.7e-6, 18, 1.9e-5, 1.65e-5}
-                 : sb <= 2       ? Cost{3.0e-6, 8, 2.7e-5, 1.73e-5}
-                 : sb <= 8       ? Cost{5.9e-6, 12, 2.86e-5, 3.33e-5}
-                 : sb == 16      ? Cost{6.0e-6, 18, 5.4e-5, 3.48e-5}
-                                 : Cost{4.2e-6, 30, 1.095e-4, 4.08e-5};
-  const double n2 = (double)N * N;
-  return c.fixed * n2 * N <= P * (std::fmax(c.least, c.pixel * n2) - c.tile * n2);
+  const Cost c = mode == kOrdDen ? Cost{4.4e-6, 1.65e-5, 0.7e-6, 1.9e-5, 18}
+                 : sb <= 2       ? Cost{3.7e-6, 1.73e-5, 0.7e-6, 2.7e-5, 8}
+                 : sb <= 8       ? Cost{6.6e-6, 3.33e-5, 0.7e-6, 2.86e-5, 12}
+                 : sb == 16      ? Cost{7.4e-6, 3.48e-5, 0.7e-6, 2.7e-5, 9}
+                                 : Cost{7.0e-6, 4.08e-5, 0.7e-6, 2.74e-5, 7.5};
+  const double n2 = (double)N * N, rays = n2 * (double)whole;
+  const int tiles = mode == kOrdDen ? 1 : (S + sb - 1) / sb, pixels = mode == kOrdDen ? 1 : (S + 7) / 8;
+  return tiles * (c.tile_ray * rays + c.tile * n2 * P) <=
+         pixels * (c.pixel_ray * rays + std::fmax(c.least, c.pixel * n2) * P);
 }
 
 bool ordered_sb_supported(int mode, int sb, int xsb) {

@@ -407,6 +407,7 @@ struct AxisCheck {
 struct RayStats {
   unsigned segments = 0, outside = 0;  // all of them, and those not in the image
   float longest = 0.f;                 // under either rounding of the lengths
+  bool whole = false;                  // every window of the ray is the whole of it
 };
 __device__ __forceinline__ int ray_flags(const GridInfo &g, const RayInfo &r, int quadrant,
                                          RayStats &stats) {
@@ -441,6 +442,7 @@ __device__ __forceinline__ int ray_flags(const GridInfo &g, const RayInfo &r, in
   const bool hits = stats.outside < stats.segments;
   const bool whole = sorted && !prim.done(n);
   const bool one_axis = !sec.done(n);
+  stats.whole = stats.segments > 0 && (whole || !sorted);
   return (whole ? kRayWhole : 0) | (wraps ? kRayWraps : 0) | (one_axis ? kRay1D : 0) |
          (hits ? kRayHits : 0);
 }
