@@ -72,7 +72,7 @@ static bool capturing(trace_handle *h) {
 // A capture that finds no plan takes another form (the same sums).
 bool forward_staged(trace_handle *h) {
   if (h->fwd_staged == 0 || !staged_batch(h->fwd_sb)) return false;
-  if (h->fwd_staged != 1 && !staged_faster(h->geo, h->fwd_sb)) return false;
+  if (h->fwd_staged != 1 && !staged_faster(h->geo, h->fwd_sb, h->scattered)) return false;
   return h->staged.sb == h->fwd_sb || !capturing(h);
 }
 
@@ -722,6 +722,7 @@ int trace_create(trace_handle_t **out, const trace_geom_t *g, int device,
     h->ang[p].quadrant = quadrant_of(q);
     h->ang[p].pad = 0;
   }
+  h->scattered = scattered_angles(h->ang.data(), geo.P);
   std::vector<float> yi(geo.C);
   for (int c = 0; c < geo.C; ++c)  // sirt.cc:129
     yi[c] = (float)((double)(1 - geo.C) / 2. + (double)c + (double)geo.mov);

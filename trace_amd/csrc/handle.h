@@ -110,6 +110,7 @@ struct trace_handle {
   int fwd_bundle = 8;     // adjacent angles per forward wavefront
   int fwd_lanes = 1;      // lanes per ray of the forward projector
   int fwd_staged = -1;    // TRACE_OPT_FWD_STAGED: 0 or 1 as set, -1 chosen by staged_faster
+  bool scattered = false; // scattered_angles
   trace_hip::StagedPlan staged;  // slab plan of the staged forward projector
   trace_hip::TileShape tile{16, 16, 16};
   bool back_rest = true;  // TRACE_OPT_BACK_REST

@@ -41,8 +41,10 @@ struct StagedLayout {
   std::vector<int4> group;
 };
 StagedLayout staged_layout(const Geometry &g, const AngleInfo *ang, int sb);
-// Whether the staged form is the fastest one for a geometry at slice batch sb.
-bool staged_faster(const Geometry &g, int sb);
+// Whether the staged form is the fastest one for a geometry at slice batch sb;
+// `scattered`: successive projections point anywhere (scattered_angles).
+bool staged_faster(const Geometry &g, int sb, bool scattered);
+bool scattered_angles(const AngleInfo *ang, int P);
 
 hipError_t launch_staged_plan(const Geometry &g, const RayInfo *rays, StagedPlan &pl,
                               hipStream_t st);

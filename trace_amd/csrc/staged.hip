@@ -499,17 +499,39 @@ StagedLayout staged_layout(const Geometry &g, const AngleInfo *ang, int sb) {
 //  1600^2,   60   1224 / 535    1439 / 923    1350 / 1509   2296 / 2962
 //  2048^2,   60   1565 / 810    1665 / 1408   3396 / 2292   5244 / 5010
 //  2048^2,  130   1707 / 2691   2076 / 3001   3910 / 4851   6832 / 11707
-bool staged_faster(const Geometry &g, int sb) {
+// Projections in no order of direction (random or shuffled angles) leave the other
+// forms' bundles of adjacent projections nothing to share, and the staged form,
+// which sorts them, wins from fewer rays on: 100 geometries a batch, 0 to 0.8%
+// above the better form on average.  Staged / others (us) at random angles:
+// 4 slices 822^2, 908 angles 1219 / 2335; 8 slices 600^2, 400 631 / 732; 32 slices
+// 300^2, 400 443 / 394.
+bool staged_faster(const Geometry &g, int sb, bool scattered) {
+  const double side = std::min(g.N, g.C), root = std::sqrt(side);
   struct Limit {
     int side, angles;
     double work;
   };
+  if (scattered) {
+    const Limit l = sb == 4    ? Limit{450, 0, 1.97e5}
+                    : sb == 8  ? Limit{330, 0, 1.52e5}
+                    : sb == 16 ? Limit{256, 0, 1.02e5}
+                               : Limit{256, 0, 8.9e4};
+    return side >= l.side && side * g.P >= l.work;
+  }
   const Limit l = sb == 4    ? Limit{950, 100, 4.5e7}
                   : sb == 8  ? Limit{512, 90, 3.75e7}
                   : sb == 16 ? Limit{0, 70, 1.6e7}
                              : Limit{0, 60, 1.84e7};
-  const double side = std::min(g.N, g.C), root = std::sqrt(side);
   return side >= l.side && g.P >= l.angles && side * root * std::sqrt(root) * g.P >= l.work;
+}
+
+// Successive projections turned against each other by more than a quarter radian
+// on average (two directions at random: 2/pi in the sine; P over a half turn: pi/P).
+bool scattered_angles(const AngleInfo *ang, int P) {
+  double turn = 0;
+  for (int p = 1; p < P; ++p)
+    turn += std::fabs((double)ang[p].sinq * ang[p - 1].cosq - (double)ang[p].cosq * ang[p - 1].sinq);
+  return P > 1 && turn > 0.25 * (P - 1);
 }
 
 hipError_t launch_staged_plan(const Geometry &g, const RayInfo *rays, StagedPlan &pl,
