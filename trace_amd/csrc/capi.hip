@@ -204,7 +204,7 @@ static int head_slices(const trace_handle *h, int sb, int least_side) {
 // (256 tickets: no more items are split).  In a capture that would need more of
 // them than there are, one workgroup takes a tile (the same sums).
 static int ensure_split(trace_handle *h, const TileShape &tile, int n, TileSplit &split) {
-  split.n = tile_splits(h->geo, tile, n);
+  split.n = tile_splits(h->geo, tile, n, h->whole_rays);
   if (split.n <= 1) return TRACE_OK;
   constexpr size_t kTickets = 256;
   const size_t words = kTickets + tile_split_words(h->geo, tile, n, split.n);

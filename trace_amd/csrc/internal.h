@@ -203,7 +203,7 @@ struct TileSplit {
   unsigned *part = nullptr;    // [slice batch][tile][n][accumulator words]
   unsigned *ticket = nullptr;  // [slice batch][tile], zero between launches
 };
-int tile_splits(const Geometry &g, const TileShape &ts, int n_slices);
+int tile_splits(const Geometry &g, const TileShape &ts, int n_slices, int64_t whole_rays);
 size_t tile_split_words(const Geometry &g, const TileShape &ts, int n_slices, int splits);
 
 // Slices [s0, s0 + n) of the stack (s0 = 0, n = 1 for column sums and counts);

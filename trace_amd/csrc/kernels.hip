@@ -1622,7 +1622,7 @@ hipError_t launch_forward(const Geometry &g, const RayInfo *rays, int sb, int bu
   return hipErrorInvalidValue;
 }
 
-int tile_splits(const Geometry &g, const TileShape &ts, int n_slices) {
+int tile_splits(const Geometry &g, const TileShape &ts, int n_slices, int64_t whole_rays) {
   if (ts.tw != 16 || ts.th != 16) return 1;
   const int64_t items = (int64_t)((g.N + 15) / 16) * ((g.N + 15) / 16) * ((n_slices + ts.sb - 1) / ts.sb);
   const int64_t pairs = (int64_t)g.P * 22;  // (angle, column) pairs of a tile
@@ -1638,9 +1638,13 @@ int tile_splits(const Geometry &g, const TileShape &ts, int n_slices) {
   //  16 slices   90^2   52 / 55   59 / 56   62 / 56   73 / 57
   //             176^2   53 / 62   60 / 63   63 / 66   74 / 68
   //  32 slices  176^2   78 / 76   87 / 85   93 / 88  105 / 100
-  const int64_t least = ts.sb == 8 || ts.sb == 16 ? 2100 + 8 * items
-                        : ts.sb <= 4 && items > 74 ? 1600 + 6 * items
-                                                   : 2048;
+  // Where many rays are walked whole (angles past a half turn), a pair is worth
+  // the more: 8 slices 125^2 at 108 angles over a full turn 73 / 62.
+  const bool long_walks = whole_rays * 8 > g.rays_per_slice();
+  const int64_t least = long_walks                  ? 2048
+                        : ts.sb == 8 || ts.sb == 16 ? 2100 + 8 * items
+                        : ts.sb <= 4 && items > 74  ? 1600 + 6 * items
+                                                    : 2048;
   if (items > 128 || pairs < least) return 1;
   // up to four workgroups of 256 lanes a CU, a pair for every lane, and at most
   // 32768 words for the last one to add up
