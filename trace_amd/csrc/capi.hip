@@ -194,10 +194,14 @@ static int batch_for(int n) {
 // 297 / 258; 1024^2, 240 3678 / 2479, 3669 / 2651, 3717 / 3122; PML num 1024^2,
 // 240 7733 / 5675, 6346, 6692; 512^2, 360 3002 / 2411, 2777, 2935; 320^2, 60
 // 274 / 277, 295, 303.  17 slices in 16 and 1 gain 6% at most and lose where they
-// are ordered.
+// are ordered.  Few angles leave both launches short (42 slices, adjoint 400^2 at 4
+// and 24 angles 57 / 107, 105 / 141; 600^2 at 24 199 / 194).
 static int head_slices(const trace_handle *h, int sb, int least_side) {
-  const int S = h->geo.S, rest = S % 32;
-  return sb == 32 && S > 32 && rest >= 1 && rest <= 16 && h->geo.N >= least_side ? S - rest : S;
+  const Geometry &g = h->geo;
+  const int rest = g.S % 32;
+  const bool enough =
+      g.N >= least_side && (g.N >= 600 || (double)g.N * g.N * g.P >= 4e6);
+  return sb == 32 && g.S > 32 && rest >= 1 && rest <= 16 && enough ? g.S - rest : g.S;
 }
 
 // Partial accumulators and tickets for tiles that several workgroups share
@@ -658,10 +662,10 @@ int trace_create(trace_handle_t **out, const trace_geom_t *g, int device,
   //   64 slices  2048^2, in batches of 32 82.9 ms, of 16 in 32x32 95.9 ms
   const double fill = (double)((n + 31) / 32) * ((n + 31) / 32) / 256;
   const bool once = fill >= 0.75 && fill <= 1.0;
-  if (S > 8 && S <= 32 && g->num_projs <= 12 && n <= 400) {
+  if (S > 8 && g->num_projs <= 12 && n <= 400) {
     // a pair a lane, and few tiles: a shallower batch adds less after each walk
-    // (9 / 31 slices at 8 angles, 8 slices a tile and 16 or 32 (us): 64^2 17 / 23,
-    // 17 / 29; 400^2 34 / 43, 43 / 68)
+    // (9, 31 and 69 slices at 8 angles, 8 slices a tile and 16 or 32 (us): 64^2
+    // 17 / 23, 17 / 29, 17 / 29; 400^2 34 / 43, 43 / 68, 81 / 86)
     h->tile = TileShape{16, 16, 8};
   } else if (S > 16) {
     h->tile = TileShape{16, 16, 32};
@@ -677,8 +681,13 @@ int trace_create(trace_handle_t **out, const trace_geom_t *g, int device,
   }
   // forward: the stack in one batch up to 32 slices (a deeper batch walks
   // each ray once for all: 2048^2, 1500 angles, 4 / 8 / 16 / 32 slices in one
-  // staged batch 9.0 / 10.1 / 17.4 / 24.5 ms)
-  if (S > 16) {
+  // staged batch 9.0 / 10.1 / 17.4 / 24.5 ms); a few angles' rays do not fill the
+  // GPU in one batch (25 slices in batches of 16 / 32 (us), 300^2 at 8 angles
+  // 45 / 55, 20 angles 78 / 89, 40 angles 84 / 87; 1000^2 257 / 354, 466 / 559,
+  // 796 / 775)
+  if (S > 16 && S < 32 && g->num_projs <= 24) {
+    h->fwd_sb = 16, h->fwd_lanes = 2;
+  } else if (S > 16) {
     h->fwd_sb = 32, h->fwd_lanes = 4;
   } else if (S > 8) {
     h->fwd_sb = 16, h->fwd_lanes = 2;
