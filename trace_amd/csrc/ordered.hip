@@ -840,7 +840,8 @@ int ordered_waves(int N, int S, int sb, bool grid_rays) {
 // and in the per-pixel form N^2 or, where its strips do not fill the GPU, the walks
 // of one (`least`).  Costs in us of a batch: sb slices in tiles, up to 8 per pixel,
 // fitted to ten sides at 120, 360 and 900 angles: where the two forms differ by
-// more than 5% the faster is chosen in all but one of 196 cases.  Tile /
+// more than 5% the faster is chosen in all but one of 196 cases (the costs are
+// within 4 and 16% of the measured times on average).  Tile /
 // per-pixel form (ms), one angle's rays on grid lines, angles 120, 360, 900:
 //              column sums                    num of 1 or 2 slices
 //    512^2   1.1 / 2.3  2.2 / 6.4  4.5 / 15   1.1 / 1.6  2.2 / 4.2  4.7 / 10
@@ -861,11 +862,11 @@ bool ordered_grid_pays(int N, int P, int64_t whole, int S, int mode, int sb) {
   struct Cost {
     double tile_ray, tile, pixel_ray, pixel, least;
   };
-  const Cost c = mode == kOrdDen ? Cost{4.4e-6, 1.65e-5, 0.7e-6, 1.9e-5, 18}
-                 : sb <= 2       ? Cost{3.7e-6, 1.73e-5, 0.7e-6, 2.7e-5, 8}
-                 : sb <= 8       ? Cost{6.6e-6, 3.33e-5, 0.7e-6, 2.86e-5, 12}
-                 : sb == 16      ? Cost{7.4e-6, 3.48e-5, 0.7e-6, 2.7e-5, 9}
-                                 : Cost{7.0e-6, 4.08e-5, 0.7e-6, 2.74e-5, 7.5};
+  const Cost c = mode == kOrdDen ? Cost{3.7e-6, 1.63e-5, 0.57e-6, 0.98e-5, 17.5}
+                 : sb <= 2       ? Cost{3.7e-6, 1.72e-5, 1.0e-6, 2.45e-5, 9}
+                 : sb <= 8       ? Cost{6.7e-6, 3.3e-5, 0.95e-6, 2.4e-5, 11.5}
+                 : sb == 16      ? Cost{7.0e-6, 3.46e-5, 0.9e-6, 2.5e-5, 9.3}
+                                 : Cost{7.03e-6, 4.09e-5, 0.71e-6, 2.74e-5, 10};
   const double n2 = (double)N * N, rays = n2 * (double)whole;
   const int tiles = mode == kOrdDen ? 1 : (S + sb - 1) / sb, pixels = mode == kOrdDen ? 1 : (S + 7) / 8;
   return tiles * (c.tile_ray * rays + c.tile * n2 * P) <=
