@@ -84,6 +84,14 @@ def test_last_slices(gpu, S):
     assert torch.equal(z[0], z[1]) and torch.equal(z[0], z[2])
 
 
+@pytest.mark.parametrize("S,batches", [(1, {1}), (2, {1, 2}), (3, {1, 2, 4}), (5, {1, 2, 4, 8})])
+def test_forward_batches_fill_the_stack(gpu, S, batches):
+    import torch
+    pj, res, _ = _tune(torch, 48, 20, S, bundles=(8,), tiles=((16, 16, 4),))
+    with pj:
+        assert {int(k.split("x")[0]) for k in res["forward_ms"]} == batches
+
+
 def test_form_is_read_only(gpu):
     from trace_amd import Projector, _capi
     with Projector(angles_rad(8), 4, 16, 8.0) as pj:

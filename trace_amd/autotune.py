@@ -43,6 +43,15 @@ def batch_candidates(batches, S: int):
     c = [b for b in batches if b <= hi and 8 * b >= S]
     return c or [max(batches)]
 
+
+def forward_batches(batches, S: int):
+    """Those of batch_candidates that the stack fills: a deeper one gathers
+    padding, and with one slice to a batch the image needs no copy, which the
+    forward projector's time does not show."""
+    c = batch_candidates(batches, S)
+    return [b for b in c if b <= _pow2_ceil(S)] or c[:1]
+
+
 _CACHE: dict = {}
 
 
@@ -116,7 +125,7 @@ def autotune(pj, sino, recon, alg: str = "mlem", params=None,
     base_tile = next(t for t in tiles if t[2] in tile_batches)
     pj.set_phase_timing(True)
     try:
-        for fb in batch_candidates(fwd_batches, pj.S):
+        for fb in forward_batches(fwd_batches, pj.S):
             apply_shape(pj, {"shape": (fb, *base_tile), "bundle": 1, "lanes": 1})
             for lanes, ba in forward_pairs(pj, fb, lanes_per_ray, bundles):
                 apply_shape(pj, {"shape": (fb, *base_tile), "bundle": ba, "lanes": lanes})
