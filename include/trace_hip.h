@@ -124,11 +124,11 @@ typedef struct trace_handle trace_handle_t;
                                        too (sirt.cc:61, mlem.cc:56) */
 #define TRACE_OPT_ORDERED_TILE 7 /* form of the ordered sums (same bits either
                                     way): 1 (default) LDS-slotted 8x8 tiles
-                                    where the geometry allows (no segment
-                                    wrapping to the next row, at most two
-                                    segments per ray and pixel; checked once
-                                    per geometry), else per pixel; 0 always
-                                    per pixel */
+                                    where the geometry's segments have the
+                                    slots (checked once per geometry) and, with
+                                    rays on grid lines, where tiles are the
+                                    faster, else per pixel; 0 always per
+                                    pixel */
 #define TRACE_OPT_FWD_STAGED 8 /* form of the forward projector at batches of
                                   4, 8, 16 and 32 slices (same bits either
                                   way): 1: bundles of up to 16 angles of
@@ -300,7 +300,7 @@ int trace_batch_create(trace_batch_t **b, const trace_batch_slice_t *slices, int
 
 /* Ray-bundle width (adjacent angles per forward wavefront: 1, 2, 4, 8, 16)
  * and backprojector tile (16x16, 32x32 or 64x64); trace_amd.autotune picks
- * them.  Default 8 and 32x32. */
+ * them.  Default 8 and 64x64. */
 int trace_batch_set_launch_shape(trace_batch_t *b, int bundle_angles, int tile_w, int tile_h);
 int trace_batch_get_launch_shape(trace_batch_t *b, int *bundle_angles, int *tile_w,
                                  int *tile_h);

@@ -43,8 +43,9 @@
 // in one pixel, one after the other, on the geometries measured (two where
 // it grazes a corner); a geometry that would need more sets a flag when den
 // is computed.  Geometries with rays on grid lines need more, and have
-// wrapped segments: a variant of the shared form below serves them, and what
-// overflows there too keeps the per-pixel form.
+// wrapped segments: a variant of the shared form below serves them where it is
+// the faster (ordered_grid_pays), and the per-pixel form elsewhere and what
+// overflows there too.
 //
 // The walks bound the one-slice form, the sums the deeper ones.  Filing a
 // segment waits for nothing: its slot is the lane's own (the ray's column
@@ -824,8 +825,9 @@ hipError_t ord_tile_launch(const OrdArgs &a, bool exact, unsigned *overflow, hip
 //   300^2,  300                  471 / 345 /  589              686 /  610 /  802
 //   400^2,  300                  547 / 622 /  997             1220 / 1005 / 1358
 //   511^2,  200                  498 / 639 / 1110              916 / 1102 / 1487
-// Geometries with rays on grid lines always share (129^2, 110 angles, 11 slices:
-// 175 us, 745 in the per-pixel form; den of 125^2, 122 angles 94, per pixel 2131).
+// Tiles of geometries with rays on grid lines always share (129^2, 110 angles, 11
+// slices: 175 us, 745 in the per-pixel form; den of 125^2, 122 angles 94, per pixel
+// 2131).
 int ordered_waves(int N, int S, int sb, bool grid_rays) {
   const int64_t tiles =
       (int64_t)((N + kOT - 1) / kOT) * ((N + kOT - 1) / kOT) * ((S + sb - 1) / sb);
@@ -835,7 +837,7 @@ int ordered_waves(int N, int S, int sb, bool grid_rays) {
 
 // Whether rays on grid lines are served faster by the tile form than pixel by
 // pixel.  Such a ray is walked whole in every tile it touches, which costs N^2 a
-// ray (a tenth to a fifth of it in the per-pixel form, whose threads walk it side
+// ray (a tenth to a quarter of it in the per-pixel form, whose threads walk it side
 // by side), and so do rays whose lists are not sorted; an angle costs N^2 in tiles,
 // and in the per-pixel form N^2 or, where its strips do not fill the GPU, the walks
 // of one (`least`).  Costs in us of a batch: sb slices in tiles, up to 8 per pixel,

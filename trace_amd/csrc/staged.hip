@@ -32,7 +32,7 @@
 // Bound by vector issue (0.9 of the rate) with the LDS reads close behind: 45
 // instructions of walk and window test a segment, a multiply and an add per
 // slice.  64 slices of 2048^2 at 1500 angles take 49 ms; 64 with the bundles
-// in projection order and the walk before it lost its integer lines, 108 in
+// in projection order and the walk before it lost its integer lines, 100 in
 // the whole-ray form.
 #include <hip/hip_runtime.h>
 
